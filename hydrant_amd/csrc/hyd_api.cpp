@@ -55,6 +55,25 @@ template <class T> int32_t upload_reuse(T *&dst, size_t &cap, const void *src, s
   return HYD_OK;
 }
 
+// Over page mappings {k, b}: least and greatest k, least b, greatest k + b.  NaN anywhere
+// gives a NaN, which every later test of the range refuses.
+void page_range(const float4 *pg, int32_t n, float &k_min, float &k_max, float &lo, float &hi) {
+  k_min = lo = INFINITY;
+  k_max = hi = -INFINITY;
+  float sum = 0.f;
+  for (int32_t i = 0; i < n; ++i) {
+    k_min = std::min(k_min, pg[i].x);
+    k_max = std::max(k_max, pg[i].x);
+    lo = std::min(lo, std::min(pg[i].y, std::min(pg[i].z, pg[i].w)));
+    hi = std::max(hi, pg[i].x + std::max(pg[i].y, std::max(pg[i].z, pg[i].w)));
+    sum += 0.f * (pg[i].x + pg[i].y + pg[i].z + pg[i].w);   // NaN for a NaN or an infinity
+  }
+  k_min += sum;
+  k_max += sum;
+  lo += sum;
+  hi += sum;
+}
+
 // One code per brick from the host copies of the page table and chebyshev grid
 // (when both are set with equal dims): the marches then read one entry per
 // brick instead of two dependent ones.
@@ -74,6 +93,15 @@ int32_t rebuild_codes(Ctx *c) {
   c->codes_valid = true;
   return HYD_OK;
 }
+
+// Whether no tap of a brick position wraps or clamps in any page: coordinates pad
+// (x k + b) - 0.5 for x in [0, 1] stay in [0, pad - 1], with 1e-3 to spare for
+// their rounding.
+int32_t inner_mapping(float k_min, float lo, float hi, int32_t pad) {
+  const bool all = k_min >= 0.f && float(pad) * lo - 0.5f >= 1e-3f && float(pad) * hi - 0.5f <= float(pad) - 1.001f;
+  return all ? kInnerAlways : kInnerTest;
+}
+int32_t pages_inner(const Ctx *c) { return inner_mapping(c->page_k_min, c->page_lo, c->page_hi, c->pool.pad); }
 
 int32_t check_volume_state(const Ctx *c) {
   HYD_REQUIRE(c->pool.data, HYD_ERR_STATE, "no brick pool: call hyd_upload_pool first");
@@ -113,7 +141,10 @@ int32_t fill_volume_args(const Ctx *c, const hyd_volume_params *p, VolumeArgs &a
   a.pool = c->pool.data;
   a.pool_elems = (uint64_t)c->pool.n_pages * c->pool.pad * c->pool.pad * c->pool.pad;
   a.pad = c->pool.pad;
-  a.u8_lut = c->u8_lut;
+  // the inner marches' table lookup reads the next entry at weight 0, which
+  // must be finite
+  a.inner = c->tf_finite ? pages_inner(c) : (int32_t)kInnerNever;
+  a.monotone = c->tf_finite && c->tf_alpha_min >= 0.f && p->density >= 0.f && c->tf_alpha_max * p->density <= 1.f;
   return HYD_OK;
 }
 
@@ -214,18 +245,13 @@ int32_t hyd_create(int32_t device, hyd_ctx **out) {
     return HYD_ERR_HIP;
   }
   c->stream = c->own_stream;
-  // float(v) / 255.f for every u8 value: the normalisation Texture3D<u8>
-  // applies on upload (texture_3d.hpp:78-86, glm_math.hpp:83-89).
-  // Then the sRGB byte thresholds of the composite.
-  float lut[512];
-  for (int i = 0; i < 256; ++i) lut[i] = float(i) / 255.f;
-  srgb8_thresholds(lut + 256);
-  int32_t st = upload(c->own_lut, lut, sizeof(lut), c->stream);
+  // the sRGB byte thresholds of the composite
+  float srgb[256];
+  srgb8_thresholds(srgb);
+  int32_t st = upload(c->srgb8_t, srgb, sizeof(srgb), c->stream);
   if (st != HYD_OK) { (void)hipStreamDestroy(c->own_stream); delete c; return st; }
-  c->u8_lut = c->own_lut;
-  c->srgb8_t = c->own_lut + 256;
   if ((st = resolve_scratch(device)) != HYD_OK) {
-    (void)hipFree(c->own_lut);
+    (void)hipFree(c->srgb8_t);
     (void)hipStreamDestroy(c->own_stream);
     delete c;
     return st;
@@ -246,7 +272,7 @@ int32_t hyd_destroy(hyd_ctx *c) {
   free_dev(c->own_cheb);
   free_dev(c->own_mean);
   free_dev(c->own_tf);
-  free_dev(c->own_lut);
+  free_dev(c->srgb8_t);
   free_dev(c->own_vols);
   free_dev(c->own_cells);
   free_dev(c->own_diff_views);
@@ -334,6 +360,7 @@ int32_t hyd_set_page_table(hyd_ctx *c, const int32_t dims[3], const int32_t *vad
   c->paging.page = c->own_page;
   c->paging.n_pages = n_pages;
   c->paging.lowest_blkcnt = lowest_blkcnt;
+  page_range(pages.data(), n_pages, c->page_k_min, c->page_k_max, c->page_lo, c->page_hi);
   c->host_vaddr.assign(vaddr, vaddr + cells);
   return rebuild_codes(c);
 }
@@ -374,6 +401,15 @@ int32_t hyd_set_tf(hyd_ctx *c, int32_t n, const float *rgba) {
   if (st) return st;
   c->tf = c->own_tf;
   c->tf_n = n;
+  c->tf_finite = true;
+  c->tf_alpha_min = c->tf_alpha_max = rgba[3];
+  for (int32_t i = 0; i < 4 * n; ++i) {
+    c->tf_finite = c->tf_finite && std::isfinite(rgba[i]);
+    if (i % 4 == 3) {
+      c->tf_alpha_min = std::min(c->tf_alpha_min, rgba[i]);
+      c->tf_alpha_max = std::max(c->tf_alpha_max, rgba[i]);
+    }
+  }
   ++c->batch_state_gen;
   return HYD_OK;
 }
@@ -562,6 +598,7 @@ struct hyd_segment_set {
   const void *pool[hyd::kMaxSegBatches] = {};
   int32_t *codes = nullptr;   // [n][cells]
   float4 *pages = nullptr;    // [n][max_pages]
+  float k_min = 0.f, k_max = 0.f, lo = 0.f, hi = 0.f;   // page_range over every batch
 };
 
 extern "C" {
@@ -788,7 +825,7 @@ int32_t hyd_render_iso(hyd_ctx *c, const hyd_iso_params *p, const hyd_view *view
   a.pool = c->pool.data;
   a.pool_elems = (uint64_t)c->pool.n_pages * c->pool.pad * c->pool.pad * c->pool.pad;
   a.pad = c->pool.pad;
-  a.u8_lut = c->u8_lut;
+  a.inner = pages_inner(c);
   a.out = out_dev;
   a.samples = samples_dev;
   HYD_CHECK_HIP(launch_iso(a, c->pool.fmt, c->stream));

@@ -94,9 +94,11 @@ struct Ctx {
   int32_t *own_cheb = nullptr;
   float *own_mean = nullptr;
   float *own_tf = nullptr;
-  const float *u8_lut = nullptr;  // 256-entry float(v)/255 table
-  const float *srgb8_t = nullptr; // 256 sRGB byte thresholds (srgb8_thresholds)
-  float *own_lut = nullptr;       // both tables, 512 floats
+  float page_lo = 0.f, page_hi = 0.f;   // over the page mappings: least b, greatest k + b (NaN: none)
+  float page_k_min = 0.f, page_k_max = 0.f;
+  bool tf_finite = false;         // every transfer-function entry is finite
+  float tf_alpha_min = 0.f, tf_alpha_max = 0.f;
+  float *srgb8_t = nullptr;       // 256 sRGB byte thresholds (srgb8_thresholds)
   // multi-volume set of the batched renderer
   void *own_vols = nullptr;       // BatchVolDev[n_vols]
   int32_t *own_cells = nullptr;   // concatenated cell codes
@@ -128,6 +130,11 @@ __device__ __forceinline__ int rotated_tile_x() {
   return (int)((blockIdx.x + (unsigned)HYD_TILE_ROTATE * blockIdx.y) % gridDim.x);
 }
 
+// Samplers of a march (hyd_sampler.hpp): the clamping one for every sample;
+// the inner one for groups of samples whose taps are found inside their page;
+// or the inner one throughout (every page maps a brick inside its tap centres).
+enum { kInnerNever = 0, kInnerTest = 1, kInnerAlways = 2 };
+
 struct VolumeArgs {
   // shader
   f3 bmin, bmax;
@@ -158,7 +165,8 @@ struct VolumeArgs {
   const void *pool;
   uint64_t pool_elems;    // voxels in the pool (n_pages * pad^3)
   int32_t pad;
-  const float *u8_lut;
+  int32_t inner;          // kInner*: which samples take the sampler without wraps and clamps
+  int32_t monotone;       // opacities in [0, 1]: a ray's alpha never falls
   // outputs
   hyd_volume_pixel *film;
   float4 *rgba;
@@ -239,7 +247,7 @@ struct IsoArgs {
   const void *pool;
   uint64_t pool_elems;    // voxels in the pool (n_pages * pad^3)
   int32_t pad;
-  const float *u8_lut;
+  int32_t inner;          // as VolumeArgs::inner
   hyd_iso_pixel *out;
   unsigned long long *samples;
 };

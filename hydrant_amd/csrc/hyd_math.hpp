@@ -36,6 +36,8 @@ HD f3 add(f3 a, f3 b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }
 HD f3 sub(f3 a, f3 b) { return {a.x - b.x, a.y - b.y, a.z - b.z}; }
 HD f3 mul(f3 a, f3 b) { return {a.x * b.x, a.y * b.y, a.z * b.z}; }
 HD f3 muls(f3 a, float s) { return {a.x * s, a.y * s, a.z * s}; }
+// Componentwise, so that the values and not their addresses are selected.
+HD f3 pick(bool c, f3 a, f3 b) { return {c ? a.x : b.x, c ? a.y : b.y, c ? a.z : b.z}; }
 HD f3 floor3(f3 a) { return {floorf(a.x), floorf(a.y), floorf(a.z)}; }
 HD f3 abs3(f3 a) { return {fabsf(a.x), fabsf(a.y), fabsf(a.z)}; }
 HD float comp_max(f3 v) { float r = v.x; r = gmax(r, v.y); r = gmax(r, v.z); return r; }

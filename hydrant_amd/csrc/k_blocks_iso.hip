@@ -100,20 +100,20 @@ __global__ __launch_bounds__(64) void blocks_kernel(BlocksArgs a) {
   a.rgba[(size_t)y * a.W + x] = v;
 }
 
-template <int FMT> __device__ __forceinline__ float vox(const void *pool, size_t i, const float *lut);
-template <> __device__ __forceinline__ float vox<HYD_FMT_F32>(const void *pool, size_t i, const float *) {
+template <int FMT> __device__ __forceinline__ float vox(const void *pool, size_t i);
+template <> __device__ __forceinline__ float vox<HYD_FMT_F32>(const void *pool, size_t i) {
   return static_cast<const float *>(pool)[i];
 }
-template <> __device__ __forceinline__ float vox<HYD_FMT_F16>(const void *pool, size_t i, const float *) {
+template <> __device__ __forceinline__ float vox<HYD_FMT_F16>(const void *pool, size_t i) {
   return __half2float(static_cast<const __half *>(pool)[i]);
 }
-template <> __device__ __forceinline__ float vox<HYD_FMT_U8>(const void *pool, size_t i, const float *lut) {
-  return lut[static_cast<const uint8_t *>(pool)[i]];
+template <> __device__ __forceinline__ float vox<HYD_FMT_U8>(const void *pool, size_t i) {
+  return u8_norm(static_cast<const uint8_t *>(pool)[i]);
 }
 
 // BlockSampler::sample_3d (mapping + CpuSampler Wrap/Linear), as in the volume kernel.
 template <int FMT>
-__device__ float iso_sample(const IsoArgs &a, const float *lut, int pgid, f3 x) {
+__device__ float iso_sample(const IsoArgs &a, int pgid, f3 x) {
   const float4 pg = a.page[pgid];
   const int pad = a.pad;
   const float fd = float(pad);
@@ -131,7 +131,7 @@ __device__ float iso_sample(const IsoArgs &a, const float *lut, int pgid, f3 x) 
     j[c] = iclamp((int)ceilf(fx), 0, pad - 1);
   }
   const size_t base = (size_t)pgid * pad * pad * pad;
-  auto at = [&](int xx, int yy, int zz) { return vox<FMT>(a.pool, base + ((size_t)zz * pad + yy) * pad + xx, lut); };
+  auto at = [&](int xx, int yy, int zz) { return vox<FMT>(a.pool, base + ((size_t)zz * pad + yy) * pad + xx); };
   const float bx = 1.f - w[0], by = 1.f - w[1], bz = 1.f - w[2];
   float x00 = at(i[0], i[1], i[2]) * bx + at(j[0], i[1], i[2]) * w[0];
   float x10 = at(i[0], j[1], i[2]) * bx + at(j[0], j[1], i[2]) * w[0];
@@ -169,7 +169,7 @@ constexpr int32_t kIsoPending = -1;
 // the first crossing; values, positions, counts and the pending pixel are those
 // of the one-step march.
 template <int FMT, int U, class OFF>
-__device__ bool iso_march_grouped(const IsoArgs &a, const float *lut, f3 &o, f3 d, int nsteps, float cdu,
+__device__ bool iso_march_grouped(const IsoArgs &a, f3 &o, f3 d, int nsteps, float cdu,
                                   hyd_iso_pixel &px, unsigned &count) {
   const f3 invr = recip3(d);
   const OFF pad3 = (OFF)a.pad * (OFF)a.pad * (OFF)a.pad;
@@ -237,8 +237,8 @@ __device__ bool iso_march_grouped(const IsoArgs &a, const float *lut, f3 &o, f3 
 #pragma unroll
     for (int j = 0; j < U; ++j) {
       if (ok[j] && live) {
-        if (fresh[j]) ref_values<FMT, OFF>(raw[j], t[j], a.pad, lut, cur);
-        const float value = ref_interp<OFF>(cur, t[j]);
+        if (fresh[j]) ref_values<FMT, OFF>(raw[j], t[j], a.pad, cur);
+        const float value = ref_interp(cur, t[j]);
         c0 = t[j].r00 + (OFF)t[j].ix;
         c7 = t[j].r11 + (OFF)t[j].jx;
         ++count;
@@ -269,10 +269,6 @@ __device__ bool iso_march_grouped(const IsoArgs &a, const float *lut, f3 &o, f3 
 
 template <int FMT, bool BIG>
 __global__ __launch_bounds__(64) void iso_march_grouped_kernel(IsoArgs a) {
-  __shared__ float s_lut[FMT == HYD_FMT_U8 ? 256 : 1];
-  if (FMT == HYD_FMT_U8)
-    for (int i = threadIdx.x; i < 256; i += blockDim.x) s_lut[i] = a.u8_lut[i];
-  __syncthreads();
   const int x = rotated_tile_x() * kTile + (threadIdx.x % kTile);
   const int y = blockIdx.y * kTile + (threadIdx.x / kTile);
   if (x >= a.W || y >= a.H) return;
@@ -291,7 +287,7 @@ __global__ __launch_bounds__(64) void iso_march_grouped_kernel(IsoArgs a) {
     const int n = (int)((tfar - tnear) / a.step);
     const int nsteps = a.max_steps < n ? a.max_steps : n;
     const float cdu = 1.f / comp_max(abs3(d));
-    iso_march_grouped<FMT, HYD_ISO_GROUP, std::conditional_t<BIG, uint64_t, uint32_t>>(a, s_lut, o, d, nsteps, cdu,
+    iso_march_grouped<FMT, HYD_ISO_GROUP, std::conditional_t<BIG, uint64_t, uint32_t>>(a, o, d, nsteps, cdu,
                                                                                         px, count);
   }
   a.out[(size_t)y * a.W + x] = px;
@@ -303,10 +299,6 @@ __global__ __launch_bounds__(64) void iso_march_grouped_kernel(IsoArgs a) {
 // the march had them), the previous and the crossing value.
 template <int FMT>
 __global__ __launch_bounds__(64) void iso_hit_kernel(IsoArgs a) {
-  __shared__ float s_lut[FMT == HYD_FMT_U8 ? 256 : 1];
-  if (FMT == HYD_FMT_U8)
-    for (int i = threadIdx.x; i < 256; i += blockDim.x) s_lut[i] = a.u8_lut[i];
-  __syncthreads();
   const int x = blockIdx.x * kTile + (threadIdx.x % kTile);
   const int y = blockIdx.y * kTile + (threadIdx.x / kTile);
   if (x >= a.W || y >= a.H) return;
@@ -330,12 +322,12 @@ __global__ __launch_bounds__(64) void iso_hit_kernel(IsoArgs a) {
                  bl * (p.z - dt * d.z) + al * p.z};
     const f3 q = sub(inter_p, ip);
     const float h = a.du * 2.f;
-    nn = f3{iso_sample<FMT>(a, s_lut, pgid, f3{q.x - h, q.y - 0.f, q.z - 0.f}) -
-                iso_sample<FMT>(a, s_lut, pgid, f3{q.x + h, q.y + 0.f, q.z + 0.f}),
-            iso_sample<FMT>(a, s_lut, pgid, f3{q.x - 0.f, q.y - h, q.z - 0.f}) -
-                iso_sample<FMT>(a, s_lut, pgid, f3{q.x + 0.f, q.y + h, q.z + 0.f}),
-            iso_sample<FMT>(a, s_lut, pgid, f3{q.x - 0.f, q.y - 0.f, q.z - h}) -
-                iso_sample<FMT>(a, s_lut, pgid, f3{q.x + 0.f, q.y + 0.f, q.z + h})};
+    nn = f3{iso_sample<FMT>(a, pgid, f3{q.x - h, q.y - 0.f, q.z - 0.f}) -
+                iso_sample<FMT>(a, pgid, f3{q.x + h, q.y + 0.f, q.z + 0.f}),
+            iso_sample<FMT>(a, pgid, f3{q.x - 0.f, q.y - h, q.z - 0.f}) -
+                iso_sample<FMT>(a, pgid, f3{q.x + 0.f, q.y + h, q.z + 0.f}),
+            iso_sample<FMT>(a, pgid, f3{q.x - 0.f, q.y - 0.f, q.z - h}) -
+                iso_sample<FMT>(a, pgid, f3{q.x + 0.f, q.y + 0.f, q.z + h})};
   } else {
     f3 plo = p;
     f3 phi = f3{p.x - dt * d.x, p.y - dt * d.y, p.z - dt * d.z};
@@ -344,7 +336,7 @@ __global__ __launch_bounds__(64) void iso_hit_kernel(IsoArgs a) {
       const f3 mid = {(plo.x + phi.x) * 0.5f, (plo.y + phi.y) * 0.5f, (plo.z + phi.z) * 0.5f};
       const f3 mip = floor3(mid);
       const int mpg = a.vaddr[grid_index(mip, a.vdim)];
-      const float mv = mpg == -1 ? value : iso_sample<FMT>(a, s_lut, mpg, sub(mid, mip));
+      const float mv = mpg == -1 ? value : iso_sample<FMT>(a, mpg, sub(mid, mip));
       if (gsign(mv - a.isovalue) == sprev) phi = mid; else plo = mid;
     }
     inter_p = f3{(plo.x + phi.x) * 0.5f, (plo.y + phi.y) * 0.5f, (plo.z + phi.z) * 0.5f};
@@ -353,12 +345,12 @@ __global__ __launch_bounds__(64) void iso_hit_kernel(IsoArgs a) {
     if (gpg == -1) { gpg = pgid; gip = ip; }
     const f3 q = sub(inter_p, gip);
     const float h = a.du;
-    const f3 g = {iso_sample<FMT>(a, s_lut, gpg, f3{q.x + h, q.y + 0.f, q.z + 0.f}) -
-                      iso_sample<FMT>(a, s_lut, gpg, f3{q.x - h, q.y - 0.f, q.z - 0.f}),
-                  iso_sample<FMT>(a, s_lut, gpg, f3{q.x + 0.f, q.y + h, q.z + 0.f}) -
-                      iso_sample<FMT>(a, s_lut, gpg, f3{q.x - 0.f, q.y - h, q.z - 0.f}),
-                  iso_sample<FMT>(a, s_lut, gpg, f3{q.x + 0.f, q.y + 0.f, q.z + h}) -
-                      iso_sample<FMT>(a, s_lut, gpg, f3{q.x - 0.f, q.y - 0.f, q.z - h})};
+    const f3 g = {iso_sample<FMT>(a, gpg, f3{q.x + h, q.y + 0.f, q.z + 0.f}) -
+                      iso_sample<FMT>(a, gpg, f3{q.x - h, q.y - 0.f, q.z - 0.f}),
+                  iso_sample<FMT>(a, gpg, f3{q.x + 0.f, q.y + h, q.z + 0.f}) -
+                      iso_sample<FMT>(a, gpg, f3{q.x - 0.f, q.y - h, q.z - 0.f}),
+                  iso_sample<FMT>(a, gpg, f3{q.x + 0.f, q.y + 0.f, q.z + h}) -
+                      iso_sample<FMT>(a, gpg, f3{q.x - 0.f, q.y - 0.f, q.z - h})};
     nn = muls(g, sprev);
   }
   float wp4[4], n4[4];

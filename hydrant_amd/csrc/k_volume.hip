@@ -8,8 +8,8 @@
 //
 // Sampling is done in software with the reference CPU backend's exact
 // arithmetic (CpuSampler, include/hydrant/bridge/cpu_sampler.hpp:88-166):
-// hardware texture filtering would not reproduce it.  The transfer function
-// and the u8 normalisation table are staged in LDS per workgroup.
+// hardware texture filtering would not reproduce it.  The transfer function is
+// staged in LDS per workgroup.
 #include <hip/hip_fp16.h>
 
 #include <cstdlib>
@@ -27,19 +27,18 @@ constexpr int kMaxTf = 256;        // LDS capacity of the TF table (entries)
 
 template <int FMT> struct Voxel;
 template <> struct Voxel<HYD_FMT_F32> {
-  static __device__ __forceinline__ float at(const void *base, size_t i, const float *) {
+  static __device__ __forceinline__ float at(const void *base, size_t i) {
     return static_cast<const float *>(base)[i];
   }
 };
 template <> struct Voxel<HYD_FMT_F16> {
-  static __device__ __forceinline__ float at(const void *base, size_t i, const float *) {
+  static __device__ __forceinline__ float at(const void *base, size_t i) {
     return __half2float(static_cast<const __half *>(base)[i]);
   }
 };
 template <> struct Voxel<HYD_FMT_U8> {
-  // float(v) / 255.f, correctly rounded, from the LDS table
-  static __device__ __forceinline__ float at(const void *base, size_t i, const float *lut) {
-    return lut[static_cast<const uint8_t *>(base)[i]];
+  static __device__ __forceinline__ float at(const void *base, size_t i) {
+    return u8_norm(static_cast<const uint8_t *>(base)[i]);
   }
 };
 
@@ -72,7 +71,7 @@ struct VolTaps {
 // on whether they were reloaded.
 template <int FMT>
 __device__ __forceinline__ float brick_sample_reuse(const void *pool, int pad, int pgid, float4 pg, f3 x,
-                                                    const float *lut, TapIdx *taps, VolTaps &c) {
+                                                    TapIdx *taps, VolTaps &c) {
   const float fd = float(pad);
   float u[3] = {x.x * pg.x + pg.y, x.y * pg.x + pg.z, x.z * pg.x + pg.w};
   float a[3];
@@ -94,10 +93,10 @@ __device__ __forceinline__ float brick_sample_reuse(const void *pool, int pad, i
   if (row_ii + i[0] != c.id0 || row_jj + j[0] != c.id7) {
     const size_t row_ji = base + ((size_t)i[2] * pad + j[1]) * pad;
     const size_t row_ij = base + ((size_t)j[2] * pad + i[1]) * pad;
-    c.v[0] = Voxel<FMT>::at(pool, row_ii + i[0], lut); c.v[1] = Voxel<FMT>::at(pool, row_ii + j[0], lut);
-    c.v[2] = Voxel<FMT>::at(pool, row_ji + i[0], lut); c.v[3] = Voxel<FMT>::at(pool, row_ji + j[0], lut);
-    c.v[4] = Voxel<FMT>::at(pool, row_ij + i[0], lut); c.v[5] = Voxel<FMT>::at(pool, row_ij + j[0], lut);
-    c.v[6] = Voxel<FMT>::at(pool, row_jj + i[0], lut); c.v[7] = Voxel<FMT>::at(pool, row_jj + j[0], lut);
+    c.v[0] = Voxel<FMT>::at(pool, row_ii + i[0]); c.v[1] = Voxel<FMT>::at(pool, row_ii + j[0]);
+    c.v[2] = Voxel<FMT>::at(pool, row_ji + i[0]); c.v[3] = Voxel<FMT>::at(pool, row_ji + j[0]);
+    c.v[4] = Voxel<FMT>::at(pool, row_ij + i[0]); c.v[5] = Voxel<FMT>::at(pool, row_ij + j[0]);
+    c.v[6] = Voxel<FMT>::at(pool, row_jj + i[0]); c.v[7] = Voxel<FMT>::at(pool, row_jj + j[0]);
     c.id0 = row_ii + i[0];
     c.id7 = row_jj + j[0];
   }
@@ -113,20 +112,32 @@ __device__ __forceinline__ float brick_sample_reuse(const void *pool, int pad, i
   return y0 * bz + y1 * az;
 }
 
+// The transfer function in LDS, edge entries repeated: entry i + 1 holds tf[i],
+// entry 0 tf[0] and entry n + 1 tf[n - 1], so the lookup needs no clamps; entries n + 2
+// and n + 3 are zero, where a value outside [0, 1] looks (the Border).
+constexpr int kTfLds = kMaxTf + 4;
+__device__ __forceinline__ void stage_tf(float4 *ext, const float *tf, int n) {
+  for (int i = threadIdx.x; i < n + 4; i += blockDim.x)
+    ext[i] = i < n + 2 ? reinterpret_cast<const float4 *>(tf)[iclamp(i - 1, 0, n - 1)] : make_float4(0.f, 0.f, 0.f, 0.f);
+}
+
 // Transfer function: Border + Linear + normalised 1-D lookup
-// (transfer_fn.hpp:14-28, cpu_sampler.hpp:117-124,142-166).
-__device__ __forceinline__ float4 tf_sample(const float *tf, int n, float s) {
+// (transfer_fn.hpp:14-28, cpu_sampler.hpp:117-124,142-166).  fx - 0.5 lies in
+// [-0.5, n - 0.5], so floor + 1 indexes the staged table.  The upper entry is the next one
+// wherever the weight is not zero; at weight zero the reference reads the lower
+// entry twice, the same sum as with the next one while the table is finite
+// (FINITE), which saves the select.
+template <bool FINITE = false>
+__device__ __forceinline__ float4 tf_sample(const float4 *ext, int n, float s) {
   const float fd = float(n);
   float fx = fd * s;
-  if (!(0.f <= fx && fx <= fd)) return make_float4(0.f, 0.f, 0.f, 0.f);
+  fx = __builtin_amdgcn_fmed3f(fx, 0.f, fd) == fx ? fx : fd + 1.5f;   // outside, or NaN: the zero entries
   fx = fx - 0.5f;
-  float flr = floorf(fx);
-  float a = fx - flr;
-  int ix = iclamp((int)flr, 0, n - 1);
-  int jx = iclamp((int)ceilf(fx), 0, n - 1);
-  const float w = 1.f - a;
-  const float *p = tf + 4 * ix, *q = tf + 4 * jx;
-  return make_float4(p[0] * w + q[0] * a, p[1] * w + q[1] * a, p[2] * w + q[2] * a, p[3] * w + q[3] * a);
+  const float flr = floorf(fx);
+  const float a = fx - flr, w = 1.f - a;
+  const float4 *e = ext + ((int)flr + 1);
+  const float4 p = e[0], q = e[FINITE || a != 0.f ? 1 : 0];
+  return make_float4(p.x * w + q.x * a, p.y * w + q.y * a, p.z * w + q.z * a, p.w * w + q.w * a);
 }
 
 struct MarchState {
@@ -143,17 +154,19 @@ struct MarchState {
 // they are never observed and THETA = false leaves them out.
 // shade_sample gives the premultiplied colour of a sample (it does not depend
 // on the ray's state), composite_ub adds it behind what the ray holds.
-template <bool WEIGHTED = false>
-__device__ __forceinline__ float4 shade_sample(const VolumeArgs &a, const float *tf, float s, int pgid, float w) {
-  float4 ub = tf_sample(tf, a.tf_n, s);
+template <bool WEIGHTED = false, bool FINITE = false>
+__device__ __forceinline__ float4 shade_sample(const VolumeArgs &a, const float4 *tf, float s, int pgid, float w) {
+  float4 ub = tf_sample<FINITE>(tf, a.tf_n, s);
   ub.w = ub.w * a.density;
   if (WEIGHTED) ub.w = ub.w * w;
-  if (a.mode == HYD_MODE_PARTITION) {
-    float l = length3(f3{ub.x, ub.y, ub.z});
-    float r = a.rank, q = 1.f - r;
-    ub = make_float4((1.f * q + 0.f * r) * l, (0.f * q + 0.f * r) * l, (0.f * q + 1.f * r) * l, ub.w);
-  } else if (a.mode == HYD_MODE_PAGING) {
-    ub = pgid >= a.lowest_blkcnt ? make_float4(0.f, 1.f, 0.f, ub.w) : make_float4(1.f, 0.f, 0.f, ub.w);
+  if (__builtin_expect(a.mode != HYD_MODE_DEFAULT, 0)) {   // one uniform branch a sample
+    if (a.mode == HYD_MODE_PARTITION) {
+      float l = length3(f3{ub.x, ub.y, ub.z});
+      float r = a.rank, q = 1.f - r;
+      ub = make_float4((1.f * q + 0.f * r) * l, (0.f * q + 0.f * r) * l, (0.f * q + 1.f * r) * l, ub.w);
+    } else {
+      ub = pgid >= a.lowest_blkcnt ? make_float4(0.f, 1.f, 0.f, ub.w) : make_float4(1.f, 0.f, 0.f, ub.w);
+    }
   }
   const float aw = ub.w;
   ub.x = ub.x * aw; ub.y = ub.y * aw; ub.z = ub.z * aw;
@@ -176,16 +189,16 @@ __device__ __forceinline__ void composite_ub(float4 ub, MarchState &st) {
 }
 
 template <bool WEIGHTED = false, bool THETA = true>
-__device__ __forceinline__ void shade_composite_impl(const VolumeArgs &a, const float *tf, float s, int pgid,
+__device__ __forceinline__ void shade_composite_impl(const VolumeArgs &a, const float4 *tf, float s, int pgid,
                                                      MarchState &st, float w) {
   composite_ub<THETA>(shade_sample<WEIGHTED>(a, tf, s, pgid, w), st);
 }
 
-__device__ __forceinline__ void shade_composite(const VolumeArgs &a, const float *tf, float s, int pgid,
+__device__ __forceinline__ void shade_composite(const VolumeArgs &a, const float4 *tf, float s, int pgid,
                                                 MarchState &st) {
   shade_composite_impl<false>(a, tf, s, pgid, st, 1.f);
 }
-__device__ __forceinline__ void shade_composite(const VolumeArgs &a, const float *tf, float s, int pgid,
+__device__ __forceinline__ void shade_composite(const VolumeArgs &a, const float4 *tf, float s, int pgid,
                                                 MarchState &st, float w) {
   shade_composite_impl<true>(a, tf, s, pgid, st, w);
 }
@@ -227,7 +240,7 @@ __device__ __forceinline__ int cell_code(const VolumeArgs &a, f3 ip) {
 // 0.85; for binary32 inputs `x > 0.93` equals `x >= 0.93f` (0.93f rounds up),
 // likewise for 0.85.
 template <int FMT, bool COUNT, bool TRACE>
-__device__ void march_reference(const VolumeArgs &a, const float *tf, const float *lut, MarchState &st,
+__device__ void march_reference(const VolumeArgs &a, const float4 *tf, MarchState &st,
                                 unsigned &count, hyd_trace_rec *trace, int max_trace, int &ntrace) {
   const float cdu = 1.f / comp_max(abs3(st.d));
   const f3 d = st.d;
@@ -259,7 +272,7 @@ __device__ void march_reference(const VolumeArgs &a, const float *tf, const floa
         cpg = pgid;
       }
       TapIdx taps;
-      const float s = brick_sample_reuse<FMT>(a.pool, a.pad, pgid, pgd, sub(o, ip), lut, TRACE ? &taps : nullptr,
+      const float s = brick_sample_reuse<FMT>(a.pool, a.pad, pgid, pgd, sub(o, ip), TRACE ? &taps : nullptr,
                                               tc);
       if (TRACE && ntrace < max_trace) {
         const int gx = gi % a.vdim[0], gy = (gi / a.vdim[0]) % a.vdim[1], gz = gi / (a.vdim[0] * a.vdim[1]);
@@ -289,16 +302,15 @@ __device__ void march_reference(const VolumeArgs &a, const float *tf, const floa
 // latency exposed on every sample.  Inside one brick the next sample positions
 // follow from the current step size alone (o += (d * step) * step_size, the
 // same binary32 operations one at a time), so a group of U samples resolves
-// its positions, tap offsets and weights first, issues the loads of every
-// sample, and then composites the samples in order.  (Skipping the loads of a
+// its positions, values and colours first (they do not depend on the ray's
+// state) and then composites the samples in order.  (Skipping the loads of a
 // sample whose cell repeats its predecessor's saved memory work, but its
-// branches and register copies cost more instructions than the loads: the
-// 512^2 FP32 frame took 0.534 ms with that reuse and groups of 2, 0.509 /
-// 0.499 / 0.607 ms without it and groups of 3 / 4 / 5.)  Escalation changes the step size; a group stops at the
-// sample that escalates (the ones after it were placed with the old step and
-// are dropped), so positions, taps, values and step budget are those of the
-// one-sample-at-a-time march, bit for bit.  Samples are also cut at the
-// brick's boundary and at the end of the step budget.
+// branches and register copies cost more instructions than the loads.)
+// Escalation changes the step size; a group stops at the sample that escalates
+// (the ones after it were placed with the old step and are dropped), so
+// positions, taps, values and step budget are those of the one-sample-at-a-time
+// march, bit for bit.  Samples are also cut at the brick's boundary and at the
+// end of the step budget.
 //
 // Voxels are addressed by element offsets from the pool base: 32-bit when the
 // pool is below 4 GiB (OFF = uint32_t, so the base stays in scalar registers),
@@ -317,8 +329,46 @@ __device__ void march_reference(const VolumeArgs &a, const float *tf, const floa
 constexpr int kCoopLanes = HYD_COOP_LANES;
 constexpr int kCoopRays = 64 / kCoopLanes;
 
+// Colours ub[j] of a group's samples x[j] (brick coordinates) where ok[j].
+template <int FMT, class OFF, int N>
+__device__ __forceinline__ void group_colours(const VolumeArgs &a, const float4 *tf, bool inner, const f3 (&x)[N],
+                                              const bool (&ok)[N], float4 pgd, OFF page_base, int pgid,
+                                              float4 (&ub)[N]) {
+  float s[N];
+  group_values<FMT, OFF, N>(a.pool, a.pad, inner, x, ok, pgd, page_base, s);
+  if (a.inner != kInnerNever) {   // the table is finite
+#pragma unroll
+    for (int j = 0; j < N; ++j) ub[j] = shade_sample<false, true>(a, tf, s[j], pgid, 1.f);
+  } else {
+#pragma unroll
+    for (int j = 0; j < N; ++j) ub[j] = shade_sample<false, false>(a, tf, s[j], pgid, 1.f);
+  }
+}
+
+// Alpha at which a sample changes the step (volume_shader.cu:71-76: v.w > 0.93
+// gives 16, else v.w > 0.85 gives 4; see march_reference for the literals).  At 16
+// only a falling alpha does, which opacities in [0, 1] rule out.
+__device__ __forceinline__ float escalation_alpha(const VolumeArgs &a, int step_size) {
+  return step_size == 4 ? 0.93f : step_size == 16 && a.monotone ? INFINITY : 0.85f;
+}
+__device__ __forceinline__ int escalated_step(float alpha, int step_size) {
+  return alpha >= 0.93f ? 16 : alpha >= 0.85f ? 4 : step_size;
+}
+
+// Composites samples J .. N-1 of a group while they are valid and the step does
+// not change; n_done counts them.
+template <int J, int N, bool THETA, class UB>
+__device__ __forceinline__ void composite_group(const UB &ub, const bool (&ok)[N], float esc, MarchState &st,
+                                                int &n_done) {
+  composite_ub<THETA>(ub(std::integral_constant<int, J>{}), st);
+  n_done = J + 1;
+  if constexpr (J + 1 < N) {
+    if (ok[J + 1] & !(st.v.w >= esc)) composite_group<J + 1, N, THETA>(ub, ok, esc, st, n_done);
+  }
+}
+
 template <int FMT, int U, bool COUNT, bool THETA, class OFF>
-__device__ void march_reference_grouped(const VolumeArgs &a, const float *tf, const float *lut, MarchState &st,
+__device__ void march_reference_grouped(const VolumeArgs &a, const float4 *tf, MarchState &st,
                                         unsigned &count, bool &handed) {
   const float cdu = 1.f / comp_max(abs3(st.d));
   const f3 d = st.d;
@@ -329,6 +379,7 @@ __device__ void march_reference_grouped(const VolumeArgs &a, const float *tf, co
   const OFF pad3 = (OFF)a.pad * (OFF)a.pad * (OFF)a.pad;
   int cpg = -1;
   float4 pgd = make_float4(0.f, 0.f, 0.f, 0.f);
+  OFF page_base = 0;
   BrickLookup bl;
   while (nsteps > 0) {
     // few rays left in this wave: the wave's lanes take them over together
@@ -354,69 +405,44 @@ __device__ void march_reference_grouped(const VolumeArgs &a, const float *tf, co
     if (pgid == -1) break;
     if (pgid != cpg) {
       pgd = a.page[pgid];
+      page_base = (OFF)pgid * pad3;
       cpg = pgid;
     }
-    const OFF page_base = (OFF)pgid * pad3;
     // positions of the group: the same additions the one-sample march makes
     const f3 inc = muls(muls(d, a.step), float(step_size));
-    f3 p[U];
+    f3 p[U], x[U];
     bool ok[U];
     p[0] = o;
+    x[0] = sub(o, ip);
     ok[0] = true;
+    int left = nsteps;
 #pragma unroll
     for (int j = 1; j < U; ++j) {
       p[j] = add(p[j - 1], inc);
-      const f3 q = floor3(p[j]);
-      ok[j] = ok[j - 1] && nsteps - j * step_size > 0 && q.x == ip.x && q.y == ip.y && q.z == ip.z;
+      x[j] = sub(p[j], ip);
+      left -= step_size;
+      ok[j] = ok[j - 1] & (left > 0) & in_unit(x[j]);
     }
-    // taps and loads of every sample of the group
-    RefTap<OFF> t[U];
-    RawTaps<FMT> raw[U];
+    bool inner = a.inner == kInnerAlways;
+    if (a.inner == kInnerTest) inner = __all(ok[U - 1] & inner_span(x[0], x[U - 1], pgd, a.pad));
+    float4 ub[U];
+    group_colours<FMT, OFF, U>(a, tf, inner, x, ok, pgd, page_base, pgid, ub);
+    int n = 0;
+    composite_group<0, U, THETA>([&](auto j) { return ub[decltype(j)::value]; }, ok, escalation_alpha(a, step_size), st,
+                                 n);
+    if (COUNT) count += (unsigned)n;
+    // samples 0 .. n-2 advanced by the group's step, the last by its own
+    const int last_ss = escalated_step(st.v.w, step_size);
+    f3 plast = p[U - 1];
 #pragma unroll
-    for (int j = 0; j < U; ++j) {
-      t[j] = ref_tap<OFF>(sub(p[j], ip), pgd, a.pad, page_base);
-      if (ok[j]) ref_fetch<FMT, OFF>(a.pool, t[j], a.pad, raw[j]);
-    }
-    // composite in order; stop at the sample that escalates
-    int last = 0, last_ss = step_size;
-    f3 plast = p[0];
-    bool live = true;
-#pragma unroll
-    for (int j = 0; j < U; ++j) {
-      if (ok[j] && live) {
-        float cur[8];
-        ref_values<FMT, OFF>(raw[j], t[j], a.pad, lut, cur);
-        const float s = ref_interp<OFF>(cur, t[j]);
-        shade_composite_impl<false, THETA>(a, tf, s, pgid, st, 1.f);
-        if (COUNT) ++count;
-        last = j;
-        plast = p[j];
-        if (st.v.w >= 0.93f) {   // v.w > 0.93 (double), see march_reference
-          last_ss = 16;
-        } else if (st.v.w >= 0.85f) {
-          last_ss = 4;
-        }
-        if (last_ss != step_size) live = false;
-      }
-    }
-    // samples 0 .. last-1 advanced by the group's step, the last by its own
+    for (int j = U - 1; j > 0; --j) plast = pick(n == j, p[j - 1], plast);
     o = add(plast, muls(muls(d, a.step), float(last_ss)));
-    nsteps -= last * step_size + last_ss;
+    nsteps -= (n - 1) * step_size + last_ss;
     step_size = last_ss;
   }
   st.o = o;
   st.nsteps = nsteps;
   st.step_size = step_size;
-}
-
-// Calls f(std::integral_constant<int, j>) for j = 0 .. N-1, so that the body
-// sees j as a constant (DPP controls must be).
-template <int... I, class F>
-__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F &&f) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, class F> __device__ __forceinline__ void static_for(F &&f) {
-  static_for_impl(std::make_integer_sequence<int, N>{}, f);
 }
 
 // Lane J of each group of G lanes, to every lane of the group.  Groups of 4
@@ -440,7 +466,7 @@ template <int G, int J> __device__ __forceinline__ float group_bcast(float v) {
 // for bit.  A lane's instruction stream per group holds UL samples' sampling
 // and shading instead of G * UL, which is what a long ray's time is made of.
 template <int FMT, bool COUNT, bool THETA, class OFF, int G, int UL = 1>
-__device__ void march_reference_coop(const VolumeArgs &a, const float *tf, const float *lut, MarchState &st, int h,
+__device__ void march_reference_coop(const VolumeArgs &a, const float4 *tf, MarchState &st, int h,
                                      unsigned &count) {
   constexpr int N = G * UL;
   const float cdu = 1.f / comp_max(abs3(st.d));
@@ -452,6 +478,7 @@ __device__ void march_reference_coop(const VolumeArgs &a, const float *tf, const
   const OFF pad3 = (OFF)a.pad * (OFF)a.pad * (OFF)a.pad;
   int cpg = -1;
   float4 pgd = make_float4(0.f, 0.f, 0.f, 0.f);
+  OFF page_base = 0;
   BrickLookup bl;
   while (nsteps > 0) {
     const f3 ip = floor3(o);
@@ -472,23 +499,23 @@ __device__ void march_reference_coop(const VolumeArgs &a, const float *tf, const
     if (pgid == -1) break;
     if (pgid != cpg) {
       pgd = a.page[pgid];
+      page_base = (OFF)pgid * pad3;
       cpg = pgid;
     }
-    const OFF page_base = (OFF)pgid * pad3;
     const f3 inc = muls(muls(d, a.step), float(step_size));
     f3 p[N];
     bool ok[N];
     p[0] = o;
     ok[0] = true;
+    int left = nsteps;
 #pragma unroll
     for (int j = 1; j < N; ++j) {
       p[j] = add(p[j - 1], inc);
-      const f3 q = floor3(p[j]);
-      ok[j] = ok[j - 1] && nsteps - j * step_size > 0 && q.x == ip.x && q.y == ip.y && q.z == ip.z;
+      left -= step_size;
+      ok[j] = ok[j - 1] & (left > 0) & in_unit(sub(p[j], ip));
     }
-    // this lane's samples h + G * k: taps and loads first, then values and colours
-    RefTap<OFF> t[UL];
-    RawTaps<FMT> raw[UL];
+    // this lane's samples h + G * k
+    f3 x[UL];
     bool okh[UL];
 #pragma unroll
     for (int k = 0; k < UL; ++k) {
@@ -501,43 +528,32 @@ __device__ void march_reference_coop(const VolumeArgs &a, const float *tf, const
           okh[k] = ok[G * k + q];
         }
       }
-      t[k] = ref_tap<OFF>(sub(ph, ip), pgd, a.pad, page_base);
-      if (okh[k]) ref_fetch<FMT, OFF>(a.pool, t[k], a.pad, raw[k]);
+      x[k] = sub(ph, ip);
     }
+    bool inner = a.inner == kInnerAlways;
+    if (a.inner == kInnerTest) inner = __all(ok[N - 1] & inner_span(sub(o, ip), sub(p[N - 1], ip), pgd, a.pad));
+    // a lane past the group's end repeats its ray's first sample
+    x[0] = pick(okh[0], x[0], sub(o, ip));
+    okh[0] = true;
     float4 ubh[UL];
+    group_colours<FMT, OFF, UL>(a, tf, inner, x, okh, pgd, page_base, pgid, ubh);
+    // composite in order, each sample's colour from its lane
+    int n = 0;
+    composite_group<0, N, THETA>(
+        [&](auto jc) {
+          constexpr int j = decltype(jc)::value;
+          const float4 &uk = ubh[j / G];
+          return make_float4(group_bcast<G, j % G>(uk.x), group_bcast<G, j % G>(uk.y), group_bcast<G, j % G>(uk.z),
+                             group_bcast<G, j % G>(uk.w));
+        },
+        ok, escalation_alpha(a, step_size), st, n);
+    if (COUNT && h == 0) count += (unsigned)n;
+    const int last_ss = escalated_step(st.v.w, step_size);
+    f3 plast = p[N - 1];
 #pragma unroll
-    for (int k = 0; k < UL; ++k) {
-      ubh[k] = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (okh[k]) {
-        float cur[8];
-        ref_values<FMT, OFF>(raw[k], t[k], a.pad, lut, cur);
-        ubh[k] = shade_sample<false>(a, tf, ref_interp<OFF>(cur, t[k]), pgid, 1.f);
-      }
-    }
-    // composite in order; stop at the sample that escalates
-    int last = 0, last_ss = step_size;
-    f3 plast = p[0];
-    bool live = true;
-    static_for<N>([&](auto jc) {
-      constexpr int j = decltype(jc)::value;
-      const float4 &uk = ubh[j / G];
-      const float4 ub = make_float4(group_bcast<G, j % G>(uk.x), group_bcast<G, j % G>(uk.y),
-                                    group_bcast<G, j % G>(uk.z), group_bcast<G, j % G>(uk.w));
-      if (ok[j] && live) {
-        composite_ub<THETA>(ub, st);
-        if (COUNT && h == 0) ++count;
-        last = j;
-        plast = p[j];
-        if (st.v.w >= 0.93f) {   // v.w > 0.93 (double), see march_reference
-          last_ss = 16;
-        } else if (st.v.w >= 0.85f) {
-          last_ss = 4;
-        }
-        if (last_ss != step_size) live = false;
-      }
-    });
+    for (int j = N - 1; j > 0; --j) plast = pick(n == j, p[j - 1], plast);
     o = add(plast, muls(muls(d, a.step), float(last_ss)));
-    nsteps -= last * step_size + last_ss;
+    nsteps -= (n - 1) * step_size + last_ss;
     step_size = last_ss;
   }
   st.o = o;
@@ -552,7 +568,7 @@ __device__ void march_reference_coop(const VolumeArgs &a, const float *tf, const
 // termination once v.w > ert.  Film: o = o0, nsteps slot = bits of L (float),
 // step_size = next lattice index.
 template <int FMT, bool COUNT, bool THETA = true>
-__device__ void march_lattice(const VolumeArgs &a, const float *tf, const float *lut, MarchState &st,
+__device__ void march_lattice(const VolumeArgs &a, const float4 *tf, MarchState &st,
                               unsigned &count) {
   const f3 o0 = st.o, d = st.d;
   const float lf = __int_as_float(st.nsteps);
@@ -584,7 +600,7 @@ __device__ void march_lattice(const VolumeArgs &a, const float *tf, const float 
       pgd = a.page[pgid];
       cpg = pgid;
     }
-    const float s = brick_sample_reuse<FMT>(a.pool, a.pad, pgid, pgd, sub(o, ip), lut, nullptr, tc);
+    const float s = brick_sample_reuse<FMT>(a.pool, a.pad, pgid, pgd, sub(o, ip), nullptr, tc);
     shade_composite_impl<true, THETA>(a, tf, s, pgid, st, w);
     if (COUNT) ++count;
     ++k;
@@ -693,12 +709,9 @@ __global__ __launch_bounds__(64) void volume_kernel(VolumeArgs a) {
   constexpr bool RESUME = MODE == kResume;
   constexpr bool THETA = MODE != kEmitRgba;
   static_assert(LANES == 1 || (kTile % LANES == 0 && ref_group<FMT>() % LANES == 0), "lanes per ray");
-  __shared__ float s_tf[4 * kMaxTf];
-  __shared__ float s_lut[FMT == HYD_FMT_U8 ? 256 : 1];
+  __shared__ float4 s_tf[kTfLds];
   __shared__ unsigned long long s_count;
-  for (int i = threadIdx.x; i < 4 * a.tf_n; i += blockDim.x) s_tf[i] = a.tf[i];
-  if (FMT == HYD_FMT_U8)
-    for (int i = threadIdx.x; i < 256; i += blockDim.x) s_lut[i] = a.u8_lut[i];
+  stage_tf(s_tf, a.tf, a.tf_n);
   if (COUNT && threadIdx.x == 0) s_count = 0;
   __syncthreads();
 
@@ -722,11 +735,11 @@ __global__ __launch_bounds__(64) void volume_kernel(VolumeArgs a) {
     }
     if (live) {
       if (LANES > 1)   // reference schedule only (the launch sees to it)
-        march_reference_coop<FMT, COUNT, THETA, OFF, LANES, ref_group<FMT>() / LANES>(a, s_tf, s_lut, st, h, count);
+        march_reference_coop<FMT, COUNT, THETA, OFF, LANES, ref_group<FMT>() / LANES>(a, s_tf, st, h, count);
       else if (a.schedule == HYD_SCHED_LATTICE)
-        march_lattice<FMT, COUNT, THETA>(a, s_tf, s_lut, st, count);
+        march_lattice<FMT, COUNT, THETA>(a, s_tf, st, count);
       else
-        march_reference_grouped<FMT, ref_group<FMT>(), COUNT, THETA, OFF>(a, s_tf, s_lut, st, count, handed);
+        march_reference_grouped<FMT, ref_group<FMT>(), COUNT, THETA, OFF>(a, s_tf, st, count, handed);
     }
     if (!handed && h == 0) store_pixel(a, idx, st);
   }
@@ -749,7 +762,7 @@ __global__ __launch_bounds__(64) void volume_kernel(VolumeArgs a) {
     const int r = lane / kCoopLanes, h = lane % kCoopLanes;
     if (r < __popcll(hm)) {
       MarchState c = s_st[r];
-      march_reference_coop<FMT, COUNT, THETA, OFF, kCoopLanes>(a, s_tf, s_lut, c, h, count);
+      march_reference_coop<FMT, COUNT, THETA, OFF, kCoopLanes>(a, s_tf, c, h, count);
       if (h == 0) store_pixel(a, s_idx[r], c);
     }
   }
@@ -763,16 +776,14 @@ __global__ __launch_bounds__(64) void volume_kernel(VolumeArgs a) {
 template <int FMT>
 __global__ __launch_bounds__(64) void volume_trace_kernel(VolumeArgs a, int x, int y, hyd_trace_rec *out,
                                                           int max_recs, int *n_out) {
-  __shared__ float s_tf[4 * kMaxTf];
-  __shared__ float s_lut[256];
-  for (int i = threadIdx.x; i < 4 * a.tf_n; i += blockDim.x) s_tf[i] = a.tf[i];
-  for (int i = threadIdx.x; i < 256; i += blockDim.x) s_lut[i] = a.u8_lut ? a.u8_lut[i] : 0.f;
+  __shared__ float4 s_tf[kTfLds];
+  stage_tf(s_tf, a.tf, a.tf_n);
   __syncthreads();
   if (threadIdx.x != 0) return;
   MarchState st;
   unsigned count = 0;
   int nt = 0;
-  if (emit(a, x, y, st)) march_reference<FMT, false, true>(a, s_tf, s_lut, st, count, out, max_recs, nt);
+  if (emit(a, x, y, st)) march_reference<FMT, false, true>(a, s_tf, st, count, out, max_recs, nt);
   *n_out = nt;
 }
 
@@ -854,7 +865,7 @@ __device__ __forceinline__ bool seg_walk_cell(const VolumeArgs &a, f3 o0, f3 d, 
 // Samples [kk, min(kk + U, kc)) of a run in cell ip of page pgid, their tap
 // loads in flight together, composited in order into seg.
 template <int FMT, bool COUNT, int U, typename OFF>
-__device__ __forceinline__ void seg_sample_group(const VolumeArgs &a, const float *s_tf, const float *s_lut, f3 o0,
+__device__ __forceinline__ void seg_sample_group(const VolumeArgs &a, const float4 *s_tf, f3 o0,
                                                  f3 d, float lf, f3 ip, float4 pgd, OFF page_base, int pgid, int kk,
                                                  int kc, MarchState &seg, unsigned &count) {
   RefTap<OFF> tp[U];
@@ -872,8 +883,8 @@ __device__ __forceinline__ void seg_sample_group(const VolumeArgs &a, const floa
   for (int j = 0; j < U; ++j) {
     if (ok[j]) {
       float cur[8];
-      ref_values<FMT, OFF>(raw[j], tp[j], a.pad, s_lut, cur);
-      const float s = ref_interp<OFF>(cur, tp[j]);
+      ref_values<FMT, OFF>(raw[j], tp[j], a.pad, cur);
+      const float s = ref_interp(cur, tp[j]);
       shade_composite_impl<true, false>(a, s_tf, s, pgid, seg, wj[j]);
       if (COUNT) ++count;
     }
@@ -889,12 +900,9 @@ __global__ __launch_bounds__(64) void segment_kernel(VolumeArgs a, SegBatchTable
     a.page = tb.page[blockIdx.z];
   }
   constexpr int U = HYD_SEG_GROUP;
-  __shared__ float s_tf[4 * kMaxTf];
-  __shared__ float s_lut[FMT == HYD_FMT_U8 ? 256 : 1];
+  __shared__ float4 s_tf[kTfLds];
   __shared__ unsigned long long s_count;
-  for (int i = threadIdx.x; i < 4 * a.tf_n; i += blockDim.x) s_tf[i] = a.tf[i];
-  if (FMT == HYD_FMT_U8)
-    for (int i = threadIdx.x; i < 256; i += blockDim.x) s_lut[i] = a.u8_lut[i];
+  stage_tf(s_tf, a.tf, a.tf_n);
   if (COUNT && threadIdx.x == 0) s_count = 0;
   __syncthreads();
   const int x = rotated_tile_x() * kTile + (threadIdx.x % kTile);
@@ -924,7 +932,7 @@ __global__ __launch_bounds__(64) void segment_kernel(VolumeArgs a, SegBatchTable
           const OFF page_base = (OFF)pgid * pad3;
           seg.v = make_float4(0.f, 0.f, 0.f, 0.f);
           for (int kk = k; kk < kc; kk += U)
-            seg_sample_group<FMT, COUNT, U, OFF>(a, s_tf, s_lut, o0, d, lf, ip, pgd, page_base, pgid, kk, kc, seg,
+            seg_sample_group<FMT, COUNT, U, OFF>(a, s_tf, o0, d, lf, ip, pgd, page_base, pgid, kk, kc, seg,
                                                  count);
           a.slots[(size_t)ord * P + ray] = seg.v;
           ++ord;
@@ -959,7 +967,7 @@ __global__ __launch_bounds__(64) void segment_kernel(VolumeArgs a, SegBatchTable
             }
           }
           if (!in_run) continue;
-          seg_sample_group<FMT, COUNT, U, OFF>(a, s_tf, s_lut, o0, d, lf, ip, pgd, page_base, pgid, kk, kc, seg,
+          seg_sample_group<FMT, COUNT, U, OFF>(a, s_tf, o0, d, lf, ip, pgd, page_base, pgid, kk, kc, seg,
                                                count);
           kk += U;
           if (kk >= kc) {   // the run is complete: its slot, then the next cell

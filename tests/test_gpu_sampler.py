@@ -1,0 +1,82 @@
+"""The march's samplers at their edges, bit for bit against the oracle: tap weights of exactly
+zero (rays along an axis through voxel centres), voxels and transfer-function entries that are
+not finite, page faces, and the register form of the u8 normalisation."""
+import numpy as np
+import pytest
+
+from hydrant_amd import _lib as L
+from hydrant_amd import dataset as D
+from hydrant_amd import workloads as W
+from tests.helpers import film_fields, oracle_film_fields, oracle_view, oracle_volume
+
+pytestmark = pytest.mark.gpu
+
+
+def _scene(n, fmt, bs, arm, density=1e-2, tf=None, poke=None):
+    vol = D.gen_blobs(n, 6, 31, sig=(4.0, 10.0), sigma_scale=n / 32.0, amp=(0.4, 1.0))
+    if fmt == L.FMT_F32:
+        vol = vol.astype(np.float32) / np.float32(255)
+    elif fmt == L.FMT_F16:
+        vol = (vol.astype(np.float32) / np.float32(255)).astype(np.float16).view(np.uint16)
+    if poke is not None:
+        flat = vol.reshape(-1)
+        v = flat if fmt == L.FMT_F32 else flat.view(np.float16)
+        at = np.random.default_rng(3).choice(flat.size, flat.size // 50, replace=False)
+        v[at] = np.resize(np.array(poke, v.dtype), at.size)
+    b = D.make_bricked(vol, bs or n, 1 if bs else 0, fmt, None, resident=1.0, seed=5)
+    geom = D.geometry((n, n, n), bs or n, 0.5)
+    return W.Scene("sampler", b, D.README_TF.copy() if tf is None else tf, 37, 29, arm, 60.0, geom, density=density)
+
+
+def _same(a, b):
+    a, b = np.asarray(a, np.float32), np.asarray(b, np.float32)
+    return np.array_equal(a, b, equal_nan=True)
+
+
+def _check(ctx, sc):
+    ctx.load(sc.bricked, sc.tf)
+    out = ctx.render_volume(sc.volume_params(), sc.view(), sc.W, sc.H, film=True, count=True)
+    img = ctx.render_volume(sc.volume_params(), sc.view(), sc.W, sc.H, film=False)["rgba"].cpu().numpy()
+    g = film_fields(out["film"].cpu().numpy())
+    with np.errstate(all="ignore"):
+        r = oracle_volume(sc).render(oracle_view(sc), 32, film=True)
+        o = oracle_film_fields(r["film"])
+    assert int(out["samples"].item()) == r["samples"] > 0
+    assert _same(img, r["rgba"])
+    for k in ("v", "theta", "phi", "o"):
+        assert _same(g[k], o[k]), k
+    assert np.array_equal(g["nsteps"], o["nsteps"]) and np.array_equal(g["step_size"], o["step_size"])
+
+
+AXIS = [(0.0, 0.0, 2.2), (90.0, 0.0, 2.2), (33.0, 21.0, 2.2)]
+
+
+@pytest.mark.parametrize("arm", AXIS)
+@pytest.mark.parametrize("fmt,n,bs", [(L.FMT_F32, 25, 0), (L.FMT_F32, 33, 16), (L.FMT_F16, 25, 0), (L.FMT_F16, 48, 16),
+                                      (L.FMT_U8, 25, 0), (L.FMT_U8, 33, 16), (L.FMT_U8, 5, 0)])
+def test_zero_weights_and_faces(gpu_ctx, fmt, n, bs, arm):
+    _check(gpu_ctx, _scene(n, fmt, bs, arm))
+
+
+@pytest.mark.parametrize("arm", AXIS)
+@pytest.mark.parametrize("fmt,bs", [(L.FMT_F32, 0), (L.FMT_F32, 8), (L.FMT_F16, 0), (L.FMT_F16, 8)])
+def test_voxels_that_are_not_finite(gpu_ctx, fmt, bs, arm):
+    _check(gpu_ctx, _scene(25, fmt, bs, arm, poke=[np.nan, np.inf, -np.inf, -1.0, 3.0]))
+
+
+@pytest.mark.parametrize("fmt,bs", [(L.FMT_F32, 0), (L.FMT_U8, 16)])
+@pytest.mark.parametrize("bad", [(3, 1, np.inf), (4, 2, np.nan), (5, 3, -0.5), (2, 3, 40.0)])
+def test_transfer_functions_outside_the_unit_range(gpu_ctx, fmt, bs, bad):
+    tf = D.README_TF.copy()
+    tf[bad[0], bad[1]] = bad[2]
+    _check(gpu_ctx, _scene(25, fmt, bs, AXIS[2], density=1.0, tf=tf))
+
+
+def test_u8_normalisation_of_every_count(gpu_ctx):
+    """A volume holding every count, read at voxel centres: the alpha of a linear table."""
+    vol = np.arange(256, dtype=np.uint8).repeat(108)[: 30 ** 3 - 30 ** 3 % 27].tolist()
+    vol = np.resize(np.array(vol, np.uint8), (30, 30, 30))
+    b = D.single_brick(vol, L.FMT_U8)
+    tf = np.stack([np.linspace(0, 1, 256)] * 3 + [np.linspace(0, 0.5, 256)], 1).astype(np.float32)
+    sc = W.Scene("u8", b, tf, 33, 31, AXIS[2], 60.0, D.geometry((30, 30, 30), 30, 0.5), density=0.1)
+    _check(gpu_ctx, sc)
