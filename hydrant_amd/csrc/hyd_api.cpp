@@ -145,6 +145,7 @@ int32_t fill_volume_args(const Ctx *c, const hyd_volume_params *p, VolumeArgs &a
   // must be finite
   a.inner = c->tf_finite ? pages_inner(c) : (int32_t)kInnerNever;
   a.monotone = c->tf_finite && c->tf_alpha_min >= 0.f && p->density >= 0.f && c->tf_alpha_max * p->density <= 1.f;
+  macro_fill(c, a);
   return HYD_OK;
 }
 
@@ -277,6 +278,7 @@ int32_t hyd_destroy(hyd_ctx *c) {
   free_dev(c->own_cells);
   free_dev(c->own_diff_views);
   free_dev(c->own_diff_scratch);
+  macro_free(c);
   if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
   delete c;
   return HYD_OK;
@@ -307,7 +309,7 @@ int32_t hyd_upload_pool(hyd_ctx *c, int32_t fmt, int32_t pad_edge, int32_t n_pag
   c->pool = Pool{c->own_pool, fmt, pad_edge, n_pages, true};
   ++c->pool_gen;
   ++c->batch_state_gen;
-  return HYD_OK;
+  return macro_pool_uploaded(c);
 }
 
 int32_t hyd_bind_pool_device(hyd_ctx *c, int32_t fmt, int32_t pad_edge, int32_t n_pages, const void *pool_dev) {
@@ -334,7 +336,8 @@ int32_t hyd_write_pool_pages(hyd_ctx *c, int32_t first_page, int32_t n_pages, co
   HYD_CHECK_HIP(hipMemcpyAsync(dst, host, (size_t)n_pages * page, hipMemcpyHostToDevice, c->stream));
   HYD_CHECK_HIP(hipStreamSynchronize(c->stream));
   // the batched renderer's oriented copies of these pages follow (in place, so
-  // captured graphs stay valid)
+  // captured graphs stay valid), and so do their macrocells
+  if ((st = macro_pages_written(c, first_page, n_pages))) return st;
   return refresh_oriented_pages(c, first_page, n_pages);
 }
 
@@ -403,15 +406,18 @@ int32_t hyd_set_tf(hyd_ctx *c, int32_t n, const float *rgba) {
   c->tf_n = n;
   c->tf_finite = true;
   c->tf_alpha_min = c->tf_alpha_max = rgba[3];
+  c->tf_rgb_max = 0.f;
   for (int32_t i = 0; i < 4 * n; ++i) {
     c->tf_finite = c->tf_finite && std::isfinite(rgba[i]);
     if (i % 4 == 3) {
       c->tf_alpha_min = std::min(c->tf_alpha_min, rgba[i]);
       c->tf_alpha_max = std::max(c->tf_alpha_max, rgba[i]);
+    } else {
+      c->tf_rgb_max = std::max(c->tf_rgb_max, std::fabs(rgba[i]));
     }
   }
   ++c->batch_state_gen;
-  return HYD_OK;
+  return macro_tf_set(c);
 }
 
 int32_t hyd_render_volume(hyd_ctx *c, const hyd_volume_params *p, const hyd_view *view, int32_t width,
@@ -580,6 +586,7 @@ int32_t hyd_segments_pass(hyd_ctx *c, const hyd_volume_params *p, const hyd_view
   fill_view(view, a.trans, a.ctg, a.ray_o);
   a.W = width;
   a.H = height;
+  a.macro.cls = nullptr;
   a.slots = reinterpret_cast<float4 *>(slots_dev);
   a.nslots = nslots_dev;
   a.max_slots = max_slots;
@@ -687,6 +694,7 @@ int32_t hyd_segments_pass_set(hyd_ctx *c, const hyd_segment_set *set, const hyd_
   fill_view(view, a.trans, a.ctg, a.ray_o);
   a.W = width;
   a.H = height;
+  a.macro.cls = nullptr;
   a.slots = reinterpret_cast<float4 *>(slots_dev);
   a.nslots = nslots_dev;
   a.max_slots = max_slots;

@@ -97,7 +97,7 @@ struct Ctx {
   float page_lo = 0.f, page_hi = 0.f;   // over the page mappings: least b, greatest k + b (NaN: none)
   float page_k_min = 0.f, page_k_max = 0.f;
   bool tf_finite = false;         // every transfer-function entry is finite
-  float tf_alpha_min = 0.f, tf_alpha_max = 0.f;
+  float tf_alpha_min = 0.f, tf_alpha_max = 0.f, tf_rgb_max = 0.f;   // tf_rgb_max: of the magnitudes
   float *srgb8_t = nullptr;       // 256 sRGB byte thresholds (srgb8_thresholds)
   // multi-volume set of the batched renderer
   void *own_vols = nullptr;       // BatchVolDev[n_vols]
@@ -106,6 +106,16 @@ struct Ctx {
   int32_t vol_pad = 0;            // padded brick edge shared by every volume
   int32_t vol_max_page = -1;   // largest page a cell of the volume set names (-1: none)
   int32_t n_cus = 0;
+  // macrocells of the pool (hyd_macro.hpp): value ranges, and their classes under
+  // the transfer function for the frame marches (owned pools only: a bound
+  // pool's contents may change without notice)
+  float2 *own_mm = nullptr;
+  uint8_t *own_mflags = nullptr, *own_mcls = nullptr;
+  unsigned long long *own_mcount = nullptr;   // macrocells that may contribute (one word)
+  size_t macro_cap = 0;           // macrocells the arrays hold
+  uint64_t mm_gen = ~0ull;        // pool_gen the ranges were made from
+  bool mcls_valid = false;        // own_mcls belongs to own_mm and the current transfer function
+  double macro_empty = 0.0;       // share of the pool's macrocells that are empty
   // differentiable renderer: device copy of the views
   void *own_diff_views = nullptr;
   int32_t diff_view_cap = 0;
@@ -129,6 +139,15 @@ struct Ctx {
 __device__ __forceinline__ int rotated_tile_x() {
   return (int)((blockIdx.x + (unsigned)HYD_TILE_ROTATE * blockIdx.y) % gridDim.x);
 }
+
+// The pool's macrocells as a march sees them.  Every page has one mapping
+// (tap coordinate = x K + B on each axis), so its constants are scalars.
+struct MacroGrid {
+  const uint8_t *cls;   // classes, page after page (null: none)
+  int32_t nm, cells;    // macrocells per page edge and per page
+  float K, B;           // voxels per brick unit, tap coordinate of x = 0
+  float run_max;        // longest run to skip at once
+};
 
 // Samplers of a march (hyd_sampler.hpp): the clamping one for every sample;
 // the inner one for groups of samples whose taps are found inside their page;
@@ -167,6 +186,7 @@ struct VolumeArgs {
   int32_t pad;
   int32_t inner;          // kInner*: which samples take the sampler without wraps and clamps
   int32_t monotone;       // opacities in [0, 1]: a ray's alpha never falls
+  MacroGrid macro;        // hyd_macro.hpp
   // outputs
   hyd_volume_pixel *film;
   float4 *rgba;
@@ -257,6 +277,15 @@ int32_t activate(Ctx *c);
 // After pool pages [first, first + n) were overwritten in place: updates the
 // batched renderer's oriented copies of those pages if they are current.
 int32_t refresh_oriented_pages(Ctx *c, int32_t first, int32_t n);
+// Macrocells of an owned pool (hyd_macro.cpp), each complete on return: the
+// whole pool's ranges and classes after an upload, those of pages [first, first
+// + n) after a write, the classes after a new transfer function.
+int32_t macro_pool_uploaded(Ctx *c);
+int32_t macro_pages_written(Ctx *c, int32_t first, int32_t n);
+int32_t macro_tf_set(Ctx *c);
+void macro_free(Ctx *c);
+// Points the march at the classes when they apply to it, else leaves it without.
+void macro_fill(const Ctx *c, VolumeArgs &a);
 
 }  // namespace hyd
 

@@ -1,0 +1,118 @@
+// Host side of the macrocells: when they are made and when a march may use them.
+#include <algorithm>
+#include <cmath>
+
+#include "hyd_macro.hpp"
+
+namespace hyd {
+namespace {
+
+// Share of empty macrocells from which a frame looks them up: the lookups cost
+// about 5% of a march (the 1024^3 fBm volume, 16% empty, breaks even: 186 and 187
+// us a paged frame without and with them), and 44% empty saves 27% of it.
+constexpr double kMacroWorth = 0.1;
+
+size_t page_cells(const Ctx *c) {
+  const size_t nm = (size_t)macro_edge(c->pool.pad);
+  return nm * nm * nm;
+}
+
+bool reserve(Ctx *c, size_t cells) {
+  if (c->macro_cap >= cells) return true;
+  macro_free(c);
+  if (hipMalloc((void **)&c->own_mm, cells * sizeof(float2)) != hipSuccess ||
+      hipMalloc((void **)&c->own_mflags, cells) != hipSuccess ||
+      hipMalloc((void **)&c->own_mcls, cells) != hipSuccess ||
+      hipMalloc((void **)&c->own_mcount, sizeof(*c->own_mcount)) != hipSuccess) {
+    (void)hipGetLastError();   // no memory for them: the marches sample everything
+    macro_free(c);
+    return false;
+  }
+  c->macro_cap = cells;
+  return true;
+}
+
+int32_t classes(Ctx *c, int32_t first, int32_t n) {
+  const float scale = c->pool.fmt == HYD_FMT_U8 ? 1.f / 255.f : 1.f;
+  HYD_CHECK_HIP(launch_macro_classes(c->own_mm, c->pool.pad, first, n, c->tf, c->tf_n, scale, nullptr,
+                                     c->own_mflags, c->own_mcls, c->own_mcount, c->stream));
+  return HYD_OK;
+}
+
+}  // namespace
+
+void macro_free(Ctx *c) {
+  for (void *p : {(void *)c->own_mm, (void *)c->own_mflags, (void *)c->own_mcls, (void *)c->own_mcount})
+    if (p) (void)hipFree(p);
+  c->own_mm = nullptr;
+  c->own_mflags = c->own_mcls = nullptr;
+  c->own_mcount = nullptr;
+  c->macro_cap = 0;
+  c->mm_gen = ~0ull;
+  c->mcls_valid = false;
+}
+
+int32_t macro_pool_uploaded(Ctx *c) {
+  c->mcls_valid = false;
+  c->mm_gen = ~0ull;
+  if (!reserve(c, (size_t)c->pool.n_pages * page_cells(c))) return HYD_OK;
+  HYD_CHECK_HIP(launch_macro_minmax(c->pool.fmt, c->pool.data, c->pool.pad, 0, c->pool.n_pages, c->own_mm,
+                                    c->stream));
+  c->mm_gen = c->pool_gen;
+  if (c->tf) return macro_tf_set(c);
+  HYD_CHECK_HIP(hipStreamSynchronize(c->stream));
+  return HYD_OK;
+}
+
+int32_t macro_tf_set(Ctx *c) {
+  c->mcls_valid = false;
+  if (c->mm_gen != c->pool_gen) return HYD_OK;
+  unsigned long long n = 0;
+  HYD_CHECK_HIP(hipMemcpyAsync(c->own_mcount, &n, sizeof(n), hipMemcpyHostToDevice, c->stream));
+  int32_t st = classes(c, 0, c->pool.n_pages);
+  if (st) return st;
+  HYD_CHECK_HIP(hipMemcpyAsync(&n, c->own_mcount, sizeof(n), hipMemcpyDeviceToHost, c->stream));
+  HYD_CHECK_HIP(hipStreamSynchronize(c->stream));   // complete before a march on another stream reads them
+  c->macro_empty = 1.0 - (double)n / ((double)c->pool.n_pages * (double)page_cells(c));
+  c->mcls_valid = true;
+  return HYD_OK;
+}
+
+int32_t macro_pages_written(Ctx *c, int32_t first, int32_t n) {
+  if (c->mm_gen != c->pool_gen || n <= 0) return HYD_OK;
+  HYD_CHECK_HIP(launch_macro_minmax(c->pool.fmt, c->pool.data, c->pool.pad, first, n, c->own_mm, c->stream));
+  if (c->mcls_valid) {
+    int32_t st = classes(c, first, n);
+    if (st) return st;
+  }
+  HYD_CHECK_HIP(hipStreamSynchronize(c->stream));
+  return HYD_OK;
+}
+
+void macro_fill(const Ctx *c, VolumeArgs &a) {
+  if (!c->pool.owned || !c->mcls_valid || c->mm_gen != c->pool_gen || c->macro_empty < kMacroWorth) return;
+  // every page has the same mapping, one b on each axis, inside the page
+  const float k = c->page_k_min, lo = c->page_lo;
+  if (!(k > 0.f && c->page_k_max == k && lo >= 0.f && c->page_hi == k + lo && k + lo <= 1.000001f)) return;
+  const size_t cells = page_cells(c);
+  if ((uint64_t)c->pool.n_pages * cells > 0xffffffffull) return;   // 32-bit class offsets
+  // opacities in [0, 1] and colours whose length is finite keep the composite
+  // finite, so that a zero contribution leaves it as it is
+  if (!a.monotone || !(c->tf_rgb_max <= 1e15f)) return;
+  if (a.mode == HYD_MODE_PARTITION && !(std::fabs(a.rank) <= 1e15f)) return;
+  // n position additions at coordinates up to D voxels round by at most n D
+  // 2^-24 voxels, which has to stay below kMacroSlack
+  float ext = 0.f;
+  for (float v : {a.bmin.x, a.bmin.y, a.bmin.z, a.bmax.x, a.bmax.y, a.bmax.z}) ext = std::max(ext, std::fabs(v));
+  const float K = k * float(c->pool.pad);
+  const float run = kMacroSlack * 16777216.f / (ext * K);
+  if (!(run >= 8.f)) return;
+  a.macro.cls = c->own_mcls;
+  a.macro.nm = macro_edge(c->pool.pad);
+  a.macro.cells = (int32_t)cells;
+  a.macro.K = K;
+  a.macro.B = lo * float(c->pool.pad) - 0.5f;
+  a.macro.run_max = std::min(std::floor(run), 4096.f);
+}
+
+}  // namespace hyd

@@ -17,6 +17,7 @@
 #include <utility>
 
 #include "hyd_internal.hpp"
+#include "hyd_macro.hpp"
 #include "hyd_sampler.hpp"
 
 namespace hyd {
@@ -210,21 +211,23 @@ __device__ __forceinline__ void shade_composite(const VolumeArgs &a, const float
 struct BrickLookup {
   f3 ip = {-INFINITY, -INFINITY, -INFINITY};
   int cd = 0, gi = 0, pg = -1;
-  __device__ __forceinline__ void update(const VolumeArgs &a, f3 p) {
-    if (p.x == ip.x && p.y == ip.y && p.z == ip.z) return;
+  // true when p is another brick
+  __device__ __forceinline__ bool update(const VolumeArgs &a, f3 p) {
+    if (p.x == ip.x && p.y == ip.y && p.z == ip.z) return false;
     ip = p;
     if (a.codes) {
       gi = grid_index(p, a.vdim);
       const int code = a.codes[gi];
       cd = code <= -2 ? -1 - code : 0;
       pg = code;
-      return;
+      return true;
     }
     cd = a.cheb[grid_index(p, a.cdim)];
     if (cd == 0) {
       gi = grid_index(p, a.vdim);
       pg = a.vaddr[gi];
     }
+    return true;
   }
 };
 
@@ -329,19 +332,37 @@ __device__ void march_reference(const VolumeArgs &a, const float4 *tf, MarchStat
 constexpr int kCoopLanes = HYD_COOP_LANES;
 constexpr int kCoopRays = 64 / kCoopLanes;
 
-// Colours ub[j] of a group's samples x[j] (brick coordinates) where ok[j].
-template <int FMT, class OFF, int N>
+// Advances o over the samples that lie in empty macrocells of brick ip, where
+// o's macrocell has class c >= 1: the march's own additions, one per sample,
+// and its step budget, without the sampling.  Returns their number (0: the
+// sample at o may contribute).
+__device__ __forceinline__ int skip_empty(const VolumeArgs &a, int c, f3 ip, f3 invr, f3 inc,
+                                          int step_size, f3 &o, int &nsteps) {
+  // 1, 4 or 16; a film from elsewhere may hold anything
+  if (step_size <= 0 || (step_size & (step_size - 1)) != 0) return 0;
+  int n = macro_run(a.macro, c, sub(o, ip), invr, a.step * float(step_size));
+  // samples left in the step budget: ceil(nsteps / step_size)
+  n = min(n, (int)(((unsigned)nsteps + (unsigned)step_size - 1u) >> (31 - __clz(step_size))));
+#pragma unroll 4
+  for (int i = 0; i < n; ++i) o = add(o, inc);
+  nsteps -= n * step_size;
+  return n;
+}
+
+// Colours ub[j] of a group's samples x[j] (brick coordinates) where ok[j];
+// WEIGHTED: their opacities scaled by w[j].
+template <int FMT, class OFF, int N, bool WEIGHTED = false>
 __device__ __forceinline__ void group_colours(const VolumeArgs &a, const float4 *tf, bool inner, const f3 (&x)[N],
                                               const bool (&ok)[N], float4 pgd, OFF page_base, int pgid,
-                                              float4 (&ub)[N]) {
+                                              float4 (&ub)[N], const float *w = nullptr) {
   float s[N];
   group_values<FMT, OFF, N>(a.pool, a.pad, inner, x, ok, pgd, page_base, s);
   if (a.inner != kInnerNever) {   // the table is finite
 #pragma unroll
-    for (int j = 0; j < N; ++j) ub[j] = shade_sample<false, true>(a, tf, s[j], pgid, 1.f);
+    for (int j = 0; j < N; ++j) ub[j] = shade_sample<WEIGHTED, true>(a, tf, s[j], pgid, WEIGHTED ? w[j] : 1.f);
   } else {
 #pragma unroll
-    for (int j = 0; j < N; ++j) ub[j] = shade_sample<false, false>(a, tf, s[j], pgid, 1.f);
+    for (int j = 0; j < N; ++j) ub[j] = shade_sample<WEIGHTED, false>(a, tf, s[j], pgid, WEIGHTED ? w[j] : 1.f);
   }
 }
 
@@ -355,15 +376,14 @@ __device__ __forceinline__ int escalated_step(float alpha, int step_size) {
   return alpha >= 0.93f ? 16 : alpha >= 0.85f ? 4 : step_size;
 }
 
-// Composites samples J .. N-1 of a group while they are valid and the step does
-// not change; n_done counts them.
+// Composites samples J .. N-1 of a group while they are valid and the alpha is
+// below esc; n counts them.
 template <int J, int N, bool THETA, class UB>
-__device__ __forceinline__ void composite_group(const UB &ub, const bool (&ok)[N], float esc, MarchState &st,
-                                                int &n_done) {
+__device__ __forceinline__ void composite_group(const UB &ub, const bool (&ok)[N], float esc, MarchState &st, int &n) {
   composite_ub<THETA>(ub(std::integral_constant<int, J>{}), st);
-  n_done = J + 1;
+  n = J + 1;
   if constexpr (J + 1 < N) {
-    if (ok[J + 1] & !(st.v.w >= esc)) composite_group<J + 1, N, THETA>(ub, ok, esc, st, n_done);
+    if (ok[J + 1] & !(st.v.w >= esc)) composite_group<J + 1, N, THETA>(ub, ok, esc, st, n);
   }
 }
 
@@ -381,6 +401,7 @@ __device__ void march_reference_grouped(const VolumeArgs &a, const float4 *tf, M
   float4 pgd = make_float4(0.f, 0.f, 0.f, 0.f);
   OFF page_base = 0;
   BrickLookup bl;
+  int cls = -1;   // class of o's macrocell (-1: not looked up)
   while (nsteps > 0) {
     // few rays left in this wave: the wave's lanes take them over together
     if (__popcll(__ballot(1)) <= kCoopRays) {
@@ -388,7 +409,7 @@ __device__ void march_reference_grouped(const VolumeArgs &a, const float4 *tf, M
       break;
     }
     const f3 ip = floor3(o);
-    bl.update(a, ip);
+    if (bl.update(a, ip)) cls = -1;
     if (bl.cd) {
       // skip_nblock_steps (volume_shader.cu:5-14) with step * step_size
       const float sstep = a.step * float(step_size);
@@ -410,22 +431,32 @@ __device__ void march_reference_grouped(const VolumeArgs &a, const float4 *tf, M
     }
     // positions of the group: the same additions the one-sample march makes
     const f3 inc = muls(muls(d, a.step), float(step_size));
-    f3 p[U], x[U];
+    if (cls > 0) {   // samples in empty macrocells: their position updates alone
+      const int k = skip_empty(a, cls, ip, invr, inc, step_size, o, nsteps);
+      if (k > 0) {
+        if (COUNT) count += (unsigned)k;
+        cls = macro_class(a.macro, pgid, sub(o, ip));
+        continue;
+      }
+    }
+    f3 q = o, x[U];
     bool ok[U];
-    p[0] = o;
     x[0] = sub(o, ip);
     ok[0] = true;
     int left = nsteps;
 #pragma unroll
     for (int j = 1; j < U; ++j) {
-      p[j] = add(p[j - 1], inc);
-      x[j] = sub(p[j], ip);
+      q = add(q, inc);
+      x[j] = sub(q, ip);
       left -= step_size;
       ok[j] = ok[j - 1] & (left > 0) & in_unit(x[j]);
     }
     bool inner = a.inner == kInnerAlways;
     if (a.inner == kInnerTest) inner = __all(ok[U - 1] & inner_span(x[0], x[U - 1], pgd, a.pad));
+    // the class at the position after the group: loaded behind the taps, waited for after the shading
+    int cnext = -1;
     float4 ub[U];
+    if (a.macro.cls) cnext = macro_class(a.macro, pgid, sub(add(q, inc), ip));
     group_colours<FMT, OFF, U>(a, tf, inner, x, ok, pgd, page_base, pgid, ub);
     int n = 0;
     composite_group<0, U, THETA>([&](auto j) { return ub[decltype(j)::value]; }, ok, escalation_alpha(a, step_size), st,
@@ -433,10 +464,13 @@ __device__ void march_reference_grouped(const VolumeArgs &a, const float4 *tf, M
     if (COUNT) count += (unsigned)n;
     // samples 0 .. n-2 advanced by the group's step, the last by its own
     const int last_ss = escalated_step(st.v.w, step_size);
-    f3 plast = p[U - 1];
-#pragma unroll
-    for (int j = U - 1; j > 0; --j) plast = pick(n == j, p[j - 1], plast);
-    o = add(plast, muls(muls(d, a.step), float(last_ss)));
+    cls = n == U && last_ss == step_size ? cnext : -1;
+    if (n == U) {
+      o = q;
+    } else {   // the last sample's position, by the same additions
+      for (int j = 1; j < n; ++j) o = add(o, inc);
+    }
+    o = add(o, muls(muls(d, a.step), float(last_ss)));
     nsteps -= (n - 1) * step_size + last_ss;
     step_size = last_ss;
   }
@@ -480,9 +514,10 @@ __device__ void march_reference_coop(const VolumeArgs &a, const float4 *tf, Marc
   float4 pgd = make_float4(0.f, 0.f, 0.f, 0.f);
   OFF page_base = 0;
   BrickLookup bl;
+  int cls = -1;   // class of o's macrocell (-1: not looked up)
   while (nsteps > 0) {
     const f3 ip = floor3(o);
-    bl.update(a, ip);
+    if (bl.update(a, ip)) cls = -1;
     if (bl.cd) {
       // skip_nblock_steps (volume_shader.cu:5-14) with step * step_size
       const float sstep = a.step * float(step_size);
@@ -503,6 +538,14 @@ __device__ void march_reference_coop(const VolumeArgs &a, const float4 *tf, Marc
       cpg = pgid;
     }
     const f3 inc = muls(muls(d, a.step), float(step_size));
+    if (cls > 0) {   // samples in empty macrocells: their position updates alone
+      const int k = skip_empty(a, cls, ip, invr, inc, step_size, o, nsteps);
+      if (k > 0) {
+        if (COUNT && h == 0) count += (unsigned)k;
+        cls = macro_class(a.macro, pgid, sub(o, ip));
+        continue;
+      }
+    }
     f3 p[N];
     bool ok[N];
     p[0] = o;
@@ -535,6 +578,8 @@ __device__ void march_reference_coop(const VolumeArgs &a, const float4 *tf, Marc
     // a lane past the group's end repeats its ray's first sample
     x[0] = pick(okh[0], x[0], sub(o, ip));
     okh[0] = true;
+    int cnext = -1;   // the class at the position after the group
+    if (a.macro.cls) cnext = macro_class(a.macro, pgid, sub(add(p[N - 1], inc), ip));
     float4 ubh[UL];
     group_colours<FMT, OFF, UL>(a, tf, inner, x, okh, pgd, page_base, pgid, ubh);
     // composite in order, each sample's colour from its lane
@@ -549,10 +594,13 @@ __device__ void march_reference_coop(const VolumeArgs &a, const float4 *tf, Marc
         ok, escalation_alpha(a, step_size), st, n);
     if (COUNT && h == 0) count += (unsigned)n;
     const int last_ss = escalated_step(st.v.w, step_size);
-    f3 plast = p[N - 1];
-#pragma unroll
-    for (int j = N - 1; j > 0; --j) plast = pick(n == j, p[j - 1], plast);
-    o = add(plast, muls(muls(d, a.step), float(last_ss)));
+    cls = n == N && last_ss == step_size ? cnext : -1;
+    if (n == N) {
+      o = p[N - 1];
+    } else {   // the last sample's position, by the same additions
+      for (int j = 1; j < n; ++j) o = add(o, inc);
+    }
+    o = add(o, muls(muls(d, a.step), float(last_ss)));
     nsteps -= (n - 1) * step_size + last_ss;
     step_size = last_ss;
   }
@@ -561,35 +609,49 @@ __device__ void march_reference_coop(const VolumeArgs &a, const float4 *tf, Marc
   st.step_size = step_size;
 }
 
+// Sample k of the lattice walk: position o0 + d * ((k + w/2) * step), w = min(1, L - k).
+__device__ __forceinline__ f3 lattice_pos(f3 o0, f3 d, float lf, float step, int k, float &w) {
+  w = gmin(1.f, lf - float(k));
+  const float t = (float(k) + 0.5f * w) * step;
+  return add(o0, muls(d, t));
+}
+
 // Lattice schedule: sample k covers w = min(1, L - k) steps (L the ray extent
 // in steps, k < ceil(L)), sits at the covered segment's midpoint
 // o0 + d * ((k + w/2) * step) and its opacity is scaled by w; empty regions are
 // skipped to the next lattice point; early
 // termination once v.w > ert.  Film: o = o0, nsteps slot = bits of L (float),
-// step_size = next lattice index.
-template <int FMT, bool COUNT, bool THETA = true>
-__device__ void march_lattice(const VolumeArgs &a, const float4 *tf, MarchState &st,
-                              unsigned &count) {
+// step_size = next lattice index.  Samples go in groups of U of one brick, as
+// in the reference march (one at a time the march waited out each sample's
+// loads); runs in empty macrocells move k alone.
+template <int FMT, int U, bool COUNT, bool THETA, class OFF>
+__device__ void march_lattice(const VolumeArgs &a, const float4 *tf, MarchState &st, unsigned &count) {
   const f3 o0 = st.o, d = st.d;
+  const f3 invr = recip3(d);
   const float lf = __int_as_float(st.nsteps);
   int k = st.step_size;
   const int kend = (int)ceilf(lf);
   const float cdu = 1.f / comp_max(abs3(d));
-  VolTaps tc;                 // taps of the last sample
+  // v.w > ert as v.w >= the next float
+  const float stop = a.ert > 0.f ? __uint_as_float(__float_as_uint(a.ert) + 1u) : INFINITY;
+  const OFF pad3 = (OFF)a.pad * (OFF)a.pad * (OFF)a.pad;
   int cpg = -1;               // page of the cached descriptor
   float4 pgd = make_float4(0.f, 0.f, 0.f, 0.f);
+  OFF page_base = 0;
   BrickLookup bl;
+  int cls = -1;               // class of sample k's macrocell (-1: not looked up)
   while (k < kend) {
-    const float w = gmin(1.f, lf - float(k));       // coverage of sample k
-    const float t = (float(k) + 0.5f * w) * a.step;  // midpoint of the covered segment
-    const f3 o = add(o0, muls(d, t));
+    f3 x[U];
+    float w[U];
+    bool ok[U];
+    const f3 o = lattice_pos(o0, d, lf, a.step, k, w[0]);
     const f3 ip = floor3(o);
-    bl.update(a, ip);
-    const int cd = bl.cd;
-    if (cd) {
+    if (bl.update(a, ip)) cls = -1;
+    if (bl.cd) {
+      const float t = (float(k) + 0.5f * w[0]) * a.step;
       float tn, tfar;
-      intersect_box(o, d, ip, f3{ip.x + 1.f, ip.y + 1.f, ip.z + 1.f}, tn, tfar);
-      const float t_exit = t + tfar + float(cd - 1) * cdu;
+      intersect_box_inv(o, invr, ip, f3{ip.x + 1.f, ip.y + 1.f, ip.z + 1.f}, tn, tfar);
+      const float t_exit = t + tfar + float(bl.cd - 1) * cdu;
       const int kn = (int)ceilf(t_exit / a.step - 0.5f);
       k = kn > k + 1 ? kn : k + 1;
       continue;
@@ -598,13 +660,41 @@ __device__ void march_lattice(const VolumeArgs &a, const float4 *tf, MarchState 
     if (pgid == -1) break;
     if (pgid != cpg) {
       pgd = a.page[pgid];
+      page_base = (OFF)pgid * pad3;
       cpg = pgid;
     }
-    const float s = brick_sample_reuse<FMT>(a.pool, a.pad, pgid, pgd, sub(o, ip), nullptr, tc);
-    shade_composite_impl<true, THETA>(a, tf, s, pgid, st, w);
-    if (COUNT) ++count;
-    ++k;
-    if (a.ert > 0.f && st.v.w > a.ert) { k = kend; break; }
+    x[0] = sub(o, ip);
+    ok[0] = true;
+    if (cls > 0) {
+      const int n = min(macro_run(a.macro, cls, x[0], invr, a.step), kend - k);
+      if (n > 0) {
+        k += n;
+        if (COUNT) count += (unsigned)n;
+        float wk;
+        cls = macro_class(a.macro, pgid, sub(lattice_pos(o0, d, lf, a.step, k, wk), ip));
+        continue;
+      }
+    }
+#pragma unroll
+    for (int j = 1; j < U; ++j) {
+      x[j] = sub(lattice_pos(o0, d, lf, a.step, k + j, w[j]), ip);
+      ok[j] = ok[j - 1] & (k + j < kend) & in_unit(x[j]);
+    }
+    bool inner = a.inner == kInnerAlways;
+    if (a.inner == kInnerTest) inner = __all(ok[U - 1] & inner_span(x[0], x[U - 1], pgd, a.pad));
+    int cnext = -1;           // the class at the sample after the group
+    if (a.macro.cls) {
+      float wk;
+      cnext = macro_class(a.macro, pgid, sub(lattice_pos(o0, d, lf, a.step, k + U, wk), ip));
+    }
+    float4 ub[U];
+    group_colours<FMT, OFF, U, true>(a, tf, inner, x, ok, pgd, page_base, pgid, ub, w);
+    int n = 0;
+    composite_group<0, U, THETA>([&](auto j) { return ub[decltype(j)::value]; }, ok, stop, st, n);
+    if (COUNT) count += (unsigned)n;
+    cls = n == U ? cnext : -1;
+    k += n;
+    if (st.v.w >= stop) k = kend;
   }
   st.step_size = k;
 }
@@ -734,10 +824,8 @@ __global__ __launch_bounds__(64) void volume_kernel(VolumeArgs a) {
       live = emit(a, x, y, st);
     }
     if (live) {
-      if (LANES > 1)   // reference schedule only (the launch sees to it)
+      if constexpr (LANES > 1)
         march_reference_coop<FMT, COUNT, THETA, OFF, LANES, ref_group<FMT>() / LANES>(a, s_tf, st, h, count);
-      else if (a.schedule == HYD_SCHED_LATTICE)
-        march_lattice<FMT, COUNT, THETA>(a, s_tf, st, count);
       else
         march_reference_grouped<FMT, ref_group<FMT>(), COUNT, THETA, OFF>(a, s_tf, st, count, handed);
     }
@@ -765,6 +853,37 @@ __global__ __launch_bounds__(64) void volume_kernel(VolumeArgs a) {
       march_reference_coop<FMT, COUNT, THETA, OFF, kCoopLanes>(a, s_tf, c, h, count);
       if (h == 0) store_pixel(a, s_idx[r], c);
     }
+  }
+  if (COUNT) {
+    if (count) atomicAdd(&s_count, (unsigned long long)count);
+    __syncthreads();
+    if (threadIdx.x == 0 && s_count) atomicAdd(a.samples, s_count);
+  }
+}
+
+// Lattice-schedule frame, one lane per ray (a kernel of its own: in
+// volume_kernel it cost the reference march 11 registers).
+template <int FMT, bool COUNT, int MODE, bool BIG>
+__global__ __launch_bounds__(64) void lattice_kernel(VolumeArgs a) {
+  __shared__ float4 s_tf[kTfLds];
+  __shared__ unsigned long long s_count;
+  stage_tf(s_tf, a.tf, a.tf_n);
+  if (COUNT && threadIdx.x == 0) s_count = 0;
+  __syncthreads();
+  const int x = rotated_tile_x() * kTile + (threadIdx.x % kTile);
+  const int y = blockIdx.y * kTile + (threadIdx.x / kTile);
+  unsigned count = 0;
+  if (x < a.W && y < a.H) {
+    const size_t idx = (size_t)y * a.W + x;
+    MarchState st;
+    bool live = true;
+    if (MODE == kResume) load_pixel(a, idx, st);
+    else live = emit(a, x, y, st);
+    if (MODE == kResume) live = st.nsteps > 0;
+    if (live)
+      march_lattice<FMT, ref_group<FMT>(), COUNT, MODE != kEmitRgba, std::conditional_t<BIG, uint64_t, uint32_t>>(
+          a, s_tf, st, count);
+    store_pixel(a, idx, st);
   }
   if (COUNT) {
     if (count) atomicAdd(&s_count, (unsigned long long)count);
@@ -810,13 +929,6 @@ __global__ __launch_bounds__(64) void volume_trace_kernel(VolumeArgs a, int x, i
 #ifndef HYD_SEG_GROUP
 #define HYD_SEG_GROUP 4
 #endif
-
-// Sample k of the lattice walk: position o0 + d * ((k + w/2) * step), w = min(1, L - k).
-__device__ __forceinline__ f3 lattice_pos(f3 o0, f3 d, float lf, float step, int k, float &w) {
-  w = gmin(1.f, lf - float(k));
-  const float t = (float(k) + 0.5f * w) * step;
-  return add(o0, muls(d, t));
-}
 
 __device__ __forceinline__ bool same_cell(f3 p, f3 ip) {
   const f3 q = floor3(p);
@@ -1013,16 +1125,16 @@ hipError_t launch_segments_fmt(const VolumeArgs &a, hipStream_t s);
 
 template <int FMT, int MODE, bool BIG>
 void launch_mode(const VolumeArgs &a, hipStream_t s) {
-  dim3 block(kTile * kTile);
   constexpr int L = ref_lanes<FMT>();
-  if (L > 1 && a.schedule == HYD_SCHED_REFERENCE) {
-    dim3 grid((a.W + kTile - 1) / kTile, (a.H + kTile / L - 1) / (kTile / L));
+  const bool lattice = a.schedule == HYD_SCHED_LATTICE;
+  const int rows = lattice ? kTile : kTile / L;
+  const dim3 block(kTile * kTile), grid((a.W + kTile - 1) / kTile, (a.H + rows - 1) / rows);
+  if (lattice) {
+    if (a.samples) hipLaunchKernelGGL((lattice_kernel<FMT, true, MODE, BIG>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((lattice_kernel<FMT, false, MODE, BIG>), grid, block, 0, s, a);
+  } else {
     if (a.samples) hipLaunchKernelGGL((volume_kernel<FMT, true, MODE, BIG, L>), grid, block, 0, s, a);
     else hipLaunchKernelGGL((volume_kernel<FMT, false, MODE, BIG, L>), grid, block, 0, s, a);
-  } else {
-    dim3 grid((a.W + kTile - 1) / kTile, (a.H + kTile - 1) / kTile);
-    if (a.samples) hipLaunchKernelGGL((volume_kernel<FMT, true, MODE, BIG, 1>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((volume_kernel<FMT, false, MODE, BIG, 1>), grid, block, 0, s, a);
   }
 }
 
