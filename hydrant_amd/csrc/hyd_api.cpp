@@ -834,6 +834,7 @@ int32_t hyd_render_iso(hyd_ctx *c, const hyd_iso_params *p, const hyd_view *view
   a.pool_elems = (uint64_t)c->pool.n_pages * c->pool.pad * c->pool.pad * c->pool.pad;
   a.pad = c->pool.pad;
   a.inner = pages_inner(c);
+  macro_fill_iso(c, a);
   a.out = out_dev;
   a.samples = samples_dev;
   HYD_CHECK_HIP(launch_iso(a, c->pool.fmt, c->stream));

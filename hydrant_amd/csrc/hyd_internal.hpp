@@ -268,6 +268,11 @@ struct IsoArgs {
   uint64_t pool_elems;    // voxels in the pool (n_pages * pad^3)
   int32_t pad;
   int32_t inner;          // as VolumeArgs::inner
+  // value ranges of the pool's macrocells as stored (null: none) and the factor
+  // to their values (hyd_macro.hpp); macro.cls is not used
+  const float2 *mm;
+  float mm_scale;
+  MacroGrid macro;
   hyd_iso_pixel *out;
   unsigned long long *samples;
 };
@@ -286,6 +291,8 @@ int32_t macro_tf_set(Ctx *c);
 void macro_free(Ctx *c);
 // Points the march at the classes when they apply to it, else leaves it without.
 void macro_fill(const Ctx *c, VolumeArgs &a);
+struct IsoArgs;
+void macro_fill_iso(const Ctx *c, IsoArgs &a);
 
 }  // namespace hyd
 

@@ -89,30 +89,44 @@ int32_t macro_pages_written(Ctx *c, int32_t first, int32_t n) {
   return HYD_OK;
 }
 
-void macro_fill(const Ctx *c, VolumeArgs &a) {
-  if (!c->pool.owned || !c->mcls_valid || c->mm_gen != c->pool_gen || c->macro_empty < kMacroWorth) return;
+namespace {
+// The grid for marches within [bmin, bmax]; false when it does not apply.
+bool grid_of(const Ctx *c, f3 bmin, f3 bmax, MacroGrid &g) {
+  if (!c->pool.owned || c->mm_gen != c->pool_gen) return false;
   // every page has the same mapping, one b on each axis, inside the page
   const float k = c->page_k_min, lo = c->page_lo;
-  if (!(k > 0.f && c->page_k_max == k && lo >= 0.f && c->page_hi == k + lo && k + lo <= 1.000001f)) return;
+  if (!(k > 0.f && c->page_k_max == k && lo >= 0.f && c->page_hi == k + lo && k + lo <= 1.000001f)) return false;
   const size_t cells = page_cells(c);
-  if ((uint64_t)c->pool.n_pages * cells > 0xffffffffull) return;   // 32-bit class offsets
+  if ((uint64_t)c->pool.n_pages * cells > 0xffffffffull) return false;   // 32-bit class offsets
+  // n position additions at coordinates up to D voxels round by at most n D
+  // 2^-24 voxels, which has to stay below kMacroSlack
+  float ext = 0.f;
+  for (float v : {bmin.x, bmin.y, bmin.z, bmax.x, bmax.y, bmax.z}) ext = std::max(ext, std::fabs(v));
+  const float K = k * float(c->pool.pad);
+  const float run = kMacroSlack * 16777216.f / (ext * K);
+  if (!(run >= 8.f)) return false;
+  g.nm = macro_edge(c->pool.pad);
+  g.cells = (int32_t)cells;
+  g.K = K;
+  g.B = lo * float(c->pool.pad) - 0.5f;
+  g.run_max = std::min(std::floor(run), 4096.f);
+  return true;
+}
+}  // namespace
+
+void macro_fill(const Ctx *c, VolumeArgs &a) {
+  if (!c->mcls_valid || c->macro_empty < kMacroWorth || !grid_of(c, a.bmin, a.bmax, a.macro)) return;
   // opacities in [0, 1] and colours whose length is finite keep the composite
   // finite, so that a zero contribution leaves it as it is
   if (!a.monotone || !(c->tf_rgb_max <= 1e15f)) return;
   if (a.mode == HYD_MODE_PARTITION && !(std::fabs(a.rank) <= 1e15f)) return;
-  // n position additions at coordinates up to D voxels round by at most n D
-  // 2^-24 voxels, which has to stay below kMacroSlack
-  float ext = 0.f;
-  for (float v : {a.bmin.x, a.bmin.y, a.bmin.z, a.bmax.x, a.bmax.y, a.bmax.z}) ext = std::max(ext, std::fabs(v));
-  const float K = k * float(c->pool.pad);
-  const float run = kMacroSlack * 16777216.f / (ext * K);
-  if (!(run >= 8.f)) return;
   a.macro.cls = c->own_mcls;
-  a.macro.nm = macro_edge(c->pool.pad);
-  a.macro.cells = (int32_t)cells;
-  a.macro.K = K;
-  a.macro.B = lo * float(c->pool.pad) - 0.5f;
-  a.macro.run_max = std::min(std::floor(run), 4096.f);
+}
+
+void macro_fill_iso(const Ctx *c, IsoArgs &a) {
+  if (!grid_of(c, a.bmin, a.bmax, a.macro)) return;
+  a.mm = c->own_mm;
+  a.mm_scale = c->pool.fmt == HYD_FMT_U8 ? 1.f / 255.f : 1.f;
 }
 
 }  // namespace hyd

@@ -38,18 +38,22 @@ __device__ __forceinline__ float macro_floor(float f8, float hi) {
   return __builtin_amdgcn_fmed3f(floorf(f8), 0.f, hi);
 }
 
-// Class of the macrocell at x (brick coordinates, x = o - floor(o)) of page
-// pgid.  A march issues this load with the tap loads of a group for the
-// position that follows the group, so that it never waits for it before
-// sampling.  Float arithmetic good to far below kMacroGuard; page * cells stays
-// below 2^32 (the host sees to it).
-__device__ __forceinline__ int macro_class(const MacroGrid &g, int pgid, f3 x) {
+// Index of x's macrocell among the pool's, the cell clamped to its page (x
+// in brick coordinates, x = o - floor(o)).  Float arithmetic good to far below
+// kMacroGuard; page * cells stays below 2^32 (the host sees to it).
+__device__ __forceinline__ uint32_t macro_index(const MacroGrid &g, int pgid, f3 x) {
   const float inv8 = 1.f / float(kMacro), hi = float(g.nm - 1), k8 = g.K * inv8, b8 = g.B * inv8;
   const float mx = macro_floor(fmaf(x.x, k8, b8), hi), my = macro_floor(fmaf(x.y, k8, b8), hi),
               mz = macro_floor(fmaf(x.z, k8, b8), hi);
   const uint32_t cell = (uint32_t)fmaf(fmaf(mz, float(g.nm), my), float(g.nm), mx);   // nm <= 128: below 2^24
-  return g.cls[(uint32_t)pgid * (uint32_t)g.cells + cell];
+  return (uint32_t)pgid * (uint32_t)g.cells + cell;
 }
+
+// Class of the macrocell at x (brick coordinates, x = o - floor(o)) of page
+// pgid.  A march issues this load with the tap loads of a group for the
+// position that follows the group, so that it never waits for it before
+// sampling.
+__device__ __forceinline__ int macro_class(const MacroGrid &g, int pgid, f3 x) { return g.cls[macro_index(g, pgid, x)]; }
 
 // Number of samples from x in steps of d * sstep that lie in empty macrocells
 // of the page, starting with the one at x, given the class c >= 1 of x's

@@ -3,6 +3,7 @@
 #include <hip/hip_fp16.h>
 
 #include "hyd_internal.hpp"
+#include "hyd_macro.hpp"
 #include "hyd_sampler.hpp"
 
 #include <cstdlib>
@@ -162,28 +163,47 @@ __device__ __forceinline__ float iso_srgb(float linear) {
 // latency of the tap loads.
 constexpr int32_t kIsoPending = -1;
 
+// Side of the isovalue that every sample of a macrocell lies on, from its
+// value range widened by 2^-19 of its magnitude (the interpolation's rounding):
+// +1, -1, or 0 when both sides (or a voxel that is not finite) are possible.
+__device__ __forceinline__ float range_side(float2 r, float scale, float iso) {
+  const float m = fmaxf(fabsf(r.x), fabsf(r.y)) * 1.9073486e-6f;
+  return (r.x - m) * scale > iso ? 1.f : (r.y + m) * scale < iso ? -1.f : 0.f;
+}
+
 // The march of IsosurfaceShaderKernel::main up to the first crossing, with the
 // tap loads of up to U consecutive samples in flight together (the step is
 // fixed, so the next positions inside a brick follow from the same additions
 // the one-step march makes).  The group is evaluated, then scanned in order for
 // the first crossing; values, positions, counts and the pending pixel are those
-// of the one-step march.
+// of the one-step march, but for a skipped sample's value (below).
+//
+// Macrocells on one side of the isovalue, the previous sample's side, cannot
+// hold a crossing: their samples move the position alone, and the previous
+// value becomes the range's end nearest the isovalue (only its side is used).
+// In the 512^3 sphere field 93% of the macrocells are such, and a ray takes 32
+// quarter-voxel samples across one.  The ranges are compared here rather than
+// classified ahead for an isovalue: it is an argument of every frame.  The
+// range at the position that follows a group is loaded behind the group's taps.
+// 1024^2 FP16 frame of that field: 2427 -> 947 us.
 template <int FMT, int U, class OFF>
-__device__ bool iso_march_grouped(const IsoArgs &a, f3 &o, f3 d, int nsteps, float cdu,
-                                  hyd_iso_pixel &px, unsigned &count) {
+__device__ bool iso_march_grouped(const IsoArgs &a, f3 &o, f3 d, int nsteps, float cdu, hyd_iso_pixel &px,
+                                  unsigned &count) {
   const f3 invr = recip3(d);
   const OFF pad3 = (OFF)a.pad * (OFF)a.pad * (OFF)a.pad;
+  const f3 inc = muls(d, a.step);
   float prev_value = 0.f;
   bool have_prev = false;
-  OFF c0 = ~(OFF)0, c7 = ~(OFF)0;   // taps of the last evaluated sample
-  float cur[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   f3 cip = {-INFINITY, -INFINITY, -INFINITY};
   int ccd = 0, cpg = -1, dpg = -1;
   float4 pgd = make_float4(0.f, 0.f, 0.f, 0.f);
+  OFF page_base = 0;
+  float2 range = make_float2(NAN, NAN);   // of o's macrocell (NaN: not looked up)
   while (nsteps > 0) {
     const f3 ip = floor3(o);
     if (ip.x != cip.x || ip.y != cip.y || ip.z != cip.z) {
       cip = ip;
+      range = make_float2(NAN, NAN);
       if (a.codes) {
         const int code = a.codes[grid_index(ip, a.vdim)];
         ccd = code <= -2 ? -1 - code : 0;
@@ -204,61 +224,74 @@ __device__ bool iso_march_grouped(const IsoArgs &a, f3 &o, f3 d, int nsteps, flo
     if (pgid == -1) break;
     if (pgid != dpg) {
       pgd = a.page[pgid];
+      page_base = (OFF)pgid * pad3;
       dpg = pgid;
     }
-    const OFF page_base = (OFF)pgid * pad3;
-    const f3 inc = muls(d, a.step);
-    f3 p[U];
+    f3 x[U];
+    x[0] = sub(o, ip);
+    const float side = range_side(range, a.mm_scale, a.isovalue);
+    const bool same = a.corrected && !have_prev ? true : side == gsign(prev_value - a.isovalue);
+    if (side != 0.f && same) {
+      const int n = min(macro_run(a.macro, 1, x[0], invr, a.step), nsteps);
+      if (n > 0) {
+#pragma unroll 4
+        for (int i = 0; i < n; ++i) o = add(o, inc);
+        nsteps -= n;
+        count += (unsigned)n;
+        if (a.corrected) { prev_value = (side > 0.f ? range.x : range.y) * a.mm_scale; have_prev = true; }
+        range = a.mm[macro_index(a.macro, pgid, sub(o, ip))];
+        continue;
+      }
+    }
     bool ok[U];
-    p[0] = o;
+    f3 q = o;
     ok[0] = true;
 #pragma unroll
     for (int j = 1; j < U; ++j) {
-      p[j] = add(p[j - 1], inc);
-      const f3 q = floor3(p[j]);
-      ok[j] = ok[j - 1] && nsteps - j > 0 && q.x == ip.x && q.y == ip.y && q.z == ip.z;
+      q = add(q, inc);
+      x[j] = sub(q, ip);
+      ok[j] = ok[j - 1] & (nsteps - j > 0) & in_unit(x[j]);
     }
-    RefTap<OFF> t[U];
-    RawTaps<FMT> raw[U];
-    bool fresh[U];
-    OFF p0 = c0, p7 = c7;
-#pragma unroll
-    for (int j = 0; j < U; ++j) {
-      t[j] = ref_tap<OFF>(sub(p[j], ip), pgd, a.pad, page_base);
-      const OFF i0 = t[j].r00 + (OFF)t[j].ix, i7 = t[j].r11 + (OFF)t[j].jx;
-      fresh[j] = i0 != p0 || i7 != p7;
-      p0 = i0;
-      p7 = i7;
-      if (ok[j] && fresh[j]) ref_fetch<FMT, OFF>(a.pool, t[j], a.pad, raw[j]);
-    }
-    int last = 0;
-    f3 plast = p[0];
+    bool inner = a.inner == kInnerAlways;
+    if (a.inner == kInnerTest) inner = __all(ok[U - 1] & inner_span(x[0], x[U - 1], pgd, a.pad));
+    float2 rnext = make_float2(NAN, NAN);
+    if (a.mm) rnext = a.mm[macro_index(a.macro, pgid, sub(add(q, inc), ip))];
+    float value[U];
+    group_values<FMT, OFF, U>(a.pool, a.pad, inner, x, ok, pgd, page_base, value);
+    // n: samples before the crossing; cross: the value there
+    int n = 0;
     bool live = true;
+    float cross = 0.f;
 #pragma unroll
     for (int j = 0; j < U; ++j) {
-      if (ok[j] && live) {
-        if (fresh[j]) ref_values<FMT, OFF>(raw[j], t[j], a.pad, cur);
-        const float value = ref_interp(cur, t[j]);
-        c0 = t[j].r00 + (OFF)t[j].ix;
-        c7 = t[j].r11 + (OFF)t[j].jx;
-        ++count;
-        bool crossing = gsign(value - a.isovalue) != gsign(prev_value - a.isovalue);
-        if (a.corrected) crossing = crossing && have_prev;
-        if (crossing) {
-          px.v[0] = p[j].x; px.v[1] = p[j].y; px.v[2] = p[j].z; px.v[3] = prev_value;
-          px.depth = value;
-          px.hit = kIsoPending;
-          live = false;
-        } else {
-          if (a.corrected) { prev_value = value; have_prev = true; }
-          last = j;
-          plast = p[j];
-        }
+      const float s = gsign(value[j] - a.isovalue);
+      const bool differs = s != gsign(prev_value - a.isovalue) && (have_prev || !a.corrected);
+      const bool on = ok[j] & live;
+      if (on) {
+        cross = value[j];
+        live = !differs;
+      }
+      if (on & !differs) {
+        ++n;
+        if (a.corrected) { prev_value = value[j]; have_prev = true; }
       }
     }
-    if (!live) return true;
-    o = add(plast, inc);
-    nsteps -= last + 1;
+    count += (unsigned)n;
+    if (n == U) {
+      o = add(q, inc);
+    } else {
+      for (int j = 0; j < n; ++j) o = add(o, inc);   // the same additions
+    }
+    if (!live) {
+      ++count;
+      px.v[0] = o.x; px.v[1] = o.y; px.v[2] = o.z; px.v[3] = prev_value;
+      px.depth = cross;
+      px.hit = kIsoPending;
+      return true;
+    }
+    nsteps -= n;
+    range = rnext;
+    if (n < U) range = make_float2(NAN, NAN);
   }
   return false;
 }

@@ -93,3 +93,35 @@ def test_new_transfer_function_and_pages(gpu_ctx):
     ref = _bound(gpu_ctx, sc, tf2)
     gpu_ctx.load(b, tf2)
     _equal(_render(gpu_ctx, sc), ref)
+
+
+@pytest.mark.parametrize("corrected", [0, 1])
+@pytest.mark.parametrize("fmt", [L.FMT_U8, L.FMT_F16, L.FMT_F32])
+@pytest.mark.parametrize("n,bs", [(12, 8), (50, 7), (70, 16), (96, 32)])
+def test_isosurface_owned_equals_bound(gpu_ctx, fmt, n, bs, corrected):
+    import torch
+
+    rng = np.random.default_rng(n + bs)
+    if fmt == L.FMT_U8:
+        vol, iso = D.gen_blobs(n, 3, n, sig=(3.0, 6.0), sigma_scale=n / 32.0, amp=(0.4, 1.0)), 0.3
+    else:
+        vol, iso = D.gen_sdf_spheres(n, 9, (2.0, n / 5.0), 2.0, n), 0.25
+        if fmt == L.FMT_F32:
+            vol = vol.view(np.float16).astype(np.float32)
+            vol.reshape(-1)[rng.choice(vol.size, 20, replace=False)] = np.resize([np.nan, np.inf, -np.inf], 20)
+    b = D.make_bricked(vol, bs, 1, fmt, None, resident=1.0, seed=5)
+    arm = (float(rng.uniform(0, 360)), float(rng.uniform(-80, 80)), 2.2)
+    sc = W.Scene("iso", b, np.zeros((1, 4), np.float32), 61, 43, arm, 60.0, D.geometry((n, n, n), bs, 1.0),
+                 extra={"isovalue": iso, "corrected": corrected, "bisect_steps": 8})
+    p = W.iso_params(sc)
+    t = torch.from_numpy(b.pool.view(np.int16) if b.pool.dtype == np.uint16 else b.pool).cuda()
+    res = []
+    for owned in (False, True):
+        gpu_ctx.load(b)
+        if not owned:
+            gpu_ctx.bind_pool_device(b.fmt, b.pad, b.n_pages, t.data_ptr())
+        r = gpu_ctx.render_iso(p, sc.view(), sc.W, sc.H, count=True)
+        gpu_ctx.synchronize()
+        res.append((r["px"].view(torch.int32).clone(), int(r["samples"].item())))
+    assert res[0][1] == res[1][1] > 0
+    assert torch.equal(res[0][0], res[1][0])
