@@ -155,6 +155,26 @@ void fill_view(const hyd_view *v, float trans[16], float &ctg, f3 &ray_o) {
   ray_o = f3{v->ray_o[0], v->ray_o[1], v->ray_o[2]};
 }
 
+// The work of a frame as a number of rays of its longest chord: an 8 x 8 grid
+// of its pixels' chords through the box.
+float full_rays(const VolumeArgs &a) {
+  const float px = float(a.W) * float(a.H);
+  if (px <= 24576.f || px > 4194304.f) return px;   // decided by the pixels alone
+  double sum = 0.0, longest = 0.0;
+  for (int j = 0; j < 8; ++j)
+    for (int i = 0; i < 8; ++i) {
+      const int x = (int)((2ll * i + 1) * a.W / 16), y = (int)((2ll * j + 1) * a.H / 16);
+      float tn, tf;
+      if (!intersect_box(a.ray_o, pixel_ray_dir(a.trans, a.ctg, a.ray_o, x, y, a.W, a.H), a.bmin, a.bmax, tn, tf))
+        continue;
+      const double c = std::max(0.0, (double)tf) - std::max(0.0, (double)tn);
+      if (!(c > 0.0)) continue;
+      sum += c;
+      longest = std::max(longest, c);
+    }
+  return longest > 0.0 ? (float)(px * sum / (64.0 * longest)) : px;
+}
+
 }  // namespace
 
 namespace {
@@ -435,6 +455,7 @@ int32_t hyd_render_volume(hyd_ctx *c, const hyd_volume_params *p, const hyd_view
   a.film = film_dev;
   a.rgba = reinterpret_cast<float4 *>(rgba_dev);
   a.samples = samples_dev;
+  a.full_rays = full_rays(a);
   HYD_CHECK_HIP(launch_volume(a, c->pool.fmt, false, c->stream));
   return HYD_OK;
 }
@@ -452,6 +473,7 @@ int32_t hyd_resume_volume(hyd_ctx *c, const hyd_volume_params *p, int32_t width,
   a.film = film_dev;
   a.rgba = reinterpret_cast<float4 *>(rgba_dev);
   a.samples = samples_dev;
+  a.full_rays = 0.42f * float(width) * float(height);   // of a square view of a cube: the film holds no view
   HYD_CHECK_HIP(launch_volume(a, c->pool.fmt, true, c->stream));
   return HYD_OK;
 }

@@ -185,6 +185,7 @@ struct VolumeArgs {
   uint64_t pool_elems;    // voxels in the pool (n_pages * pad^3)
   int32_t pad;
   int32_t inner;          // kInner*: which samples take the sampler without wraps and clamps
+  float full_rays;        // the frame's work in rays of its longest chord (host: lanes per ray)
   int32_t monotone;       // opacities in [0, 1]: a ray's alpha never falls
   MacroGrid macro;        // hyd_macro.hpp
   // outputs

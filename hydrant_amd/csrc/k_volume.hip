@@ -12,6 +12,7 @@
 // staged in LDS per workgroup.
 #include <hip/hip_fp16.h>
 
+#include <cmath>
 #include <cstdlib>
 #include <type_traits>
 #include <utility>
@@ -479,12 +480,24 @@ __device__ void march_reference_grouped(const VolumeArgs &a, const float4 *tf, M
   st.step_size = step_size;
 }
 
+// Calls f(std::integral_constant<int, j>) for j = 0 .. N-1, so that the body
+// sees j as a constant (DPP controls must be).
+template <int... I, class F>
+__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F &&f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F> __device__ __forceinline__ void static_for(F &&f) {
+  static_for_impl(std::make_integer_sequence<int, N>{}, f);
+}
+
 // Lane J of each group of G lanes, to every lane of the group.  Groups of 4
 // are the hardware quads: one DPP quad_perm move (a VALU operation) instead
 // of an LDS permute.
 template <int G, int J> __device__ __forceinline__ float group_bcast(float v) {
   if constexpr (G == 4)
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), J * 0x55, 0xF, 0xF, false));
+  else if constexpr (G == 16)   // row_newbcast
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + J, 0xF, 0xF, false));
   else
     return __shfl(v, J, G);
 }
@@ -620,12 +633,14 @@ __device__ __forceinline__ f3 lattice_pos(f3 o0, f3 d, float lf, float step, int
 // in steps, k < ceil(L)), sits at the covered segment's midpoint
 // o0 + d * ((k + w/2) * step) and its opacity is scaled by w; empty regions are
 // skipped to the next lattice point; early
-// termination once v.w > ert.  Film: o = o0, nsteps slot = bits of L (float),
+// termination once v.w > ert.  G lanes hold one ray (as in
+// march_reference_coop), lane h.  Film: o = o0, nsteps slot = bits of L (float),
 // step_size = next lattice index.  Samples go in groups of U of one brick, as
 // in the reference march (one at a time the march waited out each sample's
 // loads); runs in empty macrocells move k alone.
-template <int FMT, int U, bool COUNT, bool THETA, class OFF>
-__device__ void march_lattice(const VolumeArgs &a, const float4 *tf, MarchState &st, unsigned &count) {
+template <int FMT, int G, int U, bool COUNT, bool THETA, class OFF>
+__device__ void march_lattice(const VolumeArgs &a, const float4 *tf, MarchState &st, int h, unsigned &count) {
+  constexpr int N = G * U;
   const f3 o0 = st.o, d = st.d;
   const f3 invr = recip3(d);
   const float lf = __int_as_float(st.nsteps);
@@ -641,14 +656,12 @@ __device__ void march_lattice(const VolumeArgs &a, const float4 *tf, MarchState 
   BrickLookup bl;
   int cls = -1;               // class of sample k's macrocell (-1: not looked up)
   while (k < kend) {
-    f3 x[U];
-    float w[U];
-    bool ok[U];
-    const f3 o = lattice_pos(o0, d, lf, a.step, k, w[0]);
+    float w0;
+    const f3 o = lattice_pos(o0, d, lf, a.step, k, w0);
     const f3 ip = floor3(o);
     if (bl.update(a, ip)) cls = -1;
     if (bl.cd) {
-      const float t = (float(k) + 0.5f * w[0]) * a.step;
+      const float t = (float(k) + 0.5f * w0) * a.step;
       float tn, tfar;
       intersect_box_inv(o, invr, ip, f3{ip.x + 1.f, ip.y + 1.f, ip.z + 1.f}, tn, tfar);
       const float t_exit = t + tfar + float(bl.cd - 1) * cdu;
@@ -663,36 +676,62 @@ __device__ void march_lattice(const VolumeArgs &a, const float4 *tf, MarchState 
       page_base = (OFF)pgid * pad3;
       cpg = pgid;
     }
-    x[0] = sub(o, ip);
-    ok[0] = true;
     if (cls > 0) {
-      const int n = min(macro_run(a.macro, cls, x[0], invr, a.step), kend - k);
+      const int n = min(macro_run(a.macro, cls, sub(o, ip), invr, a.step), kend - k);
       if (n > 0) {
         k += n;
-        if (COUNT) count += (unsigned)n;
+        if (COUNT && h == 0) count += (unsigned)n;
         float wk;
         cls = macro_class(a.macro, pgid, sub(lattice_pos(o0, d, lf, a.step, k, wk), ip));
         continue;
       }
     }
+    // this lane's samples k + h + G u
+    f3 x[U];
+    float w[U];
+    bool ok[U];
 #pragma unroll
-    for (int j = 1; j < U; ++j) {
-      x[j] = sub(lattice_pos(o0, d, lf, a.step, k + j, w[j]), ip);
-      ok[j] = ok[j - 1] & (k + j < kend) & in_unit(x[j]);
+    for (int u = 0; u < U; ++u) {
+      const int kk = k + h + G * u;
+      x[u] = sub(lattice_pos(o0, d, lf, a.step, kk, w[u]), ip);
+      ok[u] = (kk < kend) & in_unit(x[u]);
+      if (u == 0) ok[u] |= h == 0;
     }
+    const bool mine = ok[0];
     bool inner = a.inner == kInnerAlways;
-    if (a.inner == kInnerTest) inner = __all(ok[U - 1] & inner_span(x[0], x[U - 1], pgd, a.pad));
+    if (a.inner == kInnerTest) inner = __all(ok[U - 1] & inner_span(sub(o, ip), x[U - 1], pgd, a.pad));
+    if (G > 1) {   // a lane past the run repeats its ray's first sample
+      x[0] = pick(mine, x[0], sub(o, ip));
+      ok[0] = true;
+    }
     int cnext = -1;           // the class at the sample after the group
     if (a.macro.cls) {
       float wk;
-      cnext = macro_class(a.macro, pgid, sub(lattice_pos(o0, d, lf, a.step, k + U, wk), ip));
+      cnext = macro_class(a.macro, pgid, sub(lattice_pos(o0, d, lf, a.step, k + N, wk), ip));
     }
     float4 ub[U];
     group_colours<FMT, OFF, U, true>(a, tf, inner, x, ok, pgd, page_base, pgid, ub, w);
+    bool okn[N];
+    static_for<N>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      const bool mine_j = j / G == 0 ? mine : ok[j / G];
+      if constexpr (G > 1) okn[j] = group_bcast<G, j % G>(mine_j ? 1.f : 0.f) != 0.f;
+      else okn[j] = mine_j;
+    });
     int n = 0;
-    composite_group<0, U, THETA>([&](auto j) { return ub[decltype(j)::value]; }, ok, stop, st, n);
-    if (COUNT) count += (unsigned)n;
-    cls = n == U ? cnext : -1;
+    composite_group<0, N, THETA>(
+        [&](auto jc) {
+          constexpr int j = decltype(jc)::value;
+          const float4 &uk = ub[j / G];
+          if constexpr (G > 1)
+            return make_float4(group_bcast<G, j % G>(uk.x), group_bcast<G, j % G>(uk.y), group_bcast<G, j % G>(uk.z),
+                               group_bcast<G, j % G>(uk.w));
+          else
+            return uk;
+        },
+        okn, stop, st, n);
+    if (COUNT && h == 0) count += (unsigned)n;
+    cls = n == N ? cnext : -1;
     k += n;
     if (st.v.w >= stop) k = kend;
   }
@@ -750,13 +789,12 @@ __device__ __forceinline__ void load_pixel(const VolumeArgs &a, size_t idx, Marc
   st.phi = f3v.w;
 }
 
-// Samples whose tap loads a reference-schedule group issues together, per
-// brick format.  Measured on the 512^2 frames: FP32 (256^3 single brick) takes
-// 0.499 ms with 4 (128 registers, 4 waves per SIMD hold the whole frame) and
-// 0.509 / 0.607 / 0.603 ms with 3 / 5 / 6; u8 (1024^3 paged, 4 lanes per ray)
-// 0.357, 0.354 and 0.350 ms with 4, 8 and 12.
+// Samples whose tap loads a one-lane reference-schedule or lattice group issues
+// together, per brick format: 4 keeps the marches within 128 registers (8 for u8: 145;
+// 640^2 and 1024^2 frames of a 500^3 volume 713 and 1274 us with 8, 800 and 1181
+// with 4).
 #ifndef HYD_REF_GROUP_U8
-#define HYD_REF_GROUP_U8 8
+#define HYD_REF_GROUP_U8 4
 #endif
 #ifndef HYD_REF_GROUP_F16
 #define HYD_REF_GROUP_F16 4
@@ -768,27 +806,31 @@ template <int FMT> constexpr int ref_group() {
   return FMT == HYD_FMT_U8 ? HYD_REF_GROUP_U8 : FMT == HYD_FMT_F16 ? HYD_REF_GROUP_F16 : HYD_REF_GROUP_F32;
 }
 
-// Lanes per ray of the reference-schedule frame, per brick format (a wave
-// then covers an 8 x 8/LANES tile; LANES > 1 marches with
-// march_reference_coop, ref_group / LANES samples per lane and group).  A
-// frame whose time is the chain of its longest rays gains: the paged u8 frame
-// takes 0.52 ms with 1 lane (groups of 8 on one lane, the last rays handed to
-// 4 lanes each), 0.405 with 2, 0.354 with 4 and 0.42 with 8.  A frame bound by
-// instruction issue loses, since every lane of a ray repeats the positions
-// and the compositing: the plain FP32 frame takes 0.55 ms with 1 lane, 0.59
-// with 2 and 0.69 with 4.
-#ifndef HYD_REF_LANES_U8
-#define HYD_REF_LANES_U8 4
-#endif
-#ifndef HYD_REF_LANES_F16
-#define HYD_REF_LANES_F16 1
-#endif
-#ifndef HYD_REF_LANES_F32
-#define HYD_REF_LANES_F32 1
-#endif
-template <int FMT> constexpr int ref_lanes() {
-  return FMT == HYD_FMT_U8 ? HYD_REF_LANES_U8 : FMT == HYD_FMT_F16 ? HYD_REF_LANES_F16 : HYD_REF_LANES_F32;
-}
+// Lanes per ray of a frame.  A ray is one dependent chain of groups; a SIMD
+// with one wave on it issues that chain no faster than one with four.  Several
+// lanes shorten it (each resolves a share of a group's samples; all composite
+// them in order), at the price of repeating the positions and the compositing
+// on every lane.  So: 16 lanes while the launch stays around six waves per SIMD
+// (a group's colours then come by DPP row broadcasts), 4 while the chains of
+// the longest rays and not the sum of the work set the time, then one.  The
+// work is counted in rays of the longest chord (full_rays), and the line moves
+// with the pool's size: chains wait longer for taps the caches do not hold.
+// Frames in us, 1 / 4 / 16 lanes (reference schedule unless noted; full_rays
+// about 0.42 of the pixels of these square views, all of the 356 x 882 ones):
+//                             48 x 40       160^2         200^2        512^2     640^2       800^2
+//   256^3 FP32 brick       440/205/142   431/201/171   -/200/210   412/398   476/575     599/842
+//   400^3 FP32 fBm bricks  495/213/163   523/280/265   -/320/337   991/852   1206/1103   1399/1434
+//   500^3 FP16 bricks      628/343/238   733/356/280   -/373/318   943/716   1118/902    1187/1230
+//   400^3 u8 fBm bricks    425/212/162   431/250/237   -/263/317   654/641   745/907     940/1309
+//   500^3 FP16, lattice    689/281/177   697/299/221   -/310/318   915/726   1180/957    1360/1358
+//   356 x 882: 35^3 FP16 79/128, 64^3 FP16 128/182, 120^3 FP32 226/327; 60^3 u8 at 500^2 101/132
+constexpr int kLanes = 4, kManyLanes = 16;
+template <int L> constexpr int coop_group() { return L == kManyLanes ? 16 : 8; }   // samples a group
+// A wave's tile of rays.
+template <int L> constexpr int tile_w() { return L == kManyLanes ? 4 : kTile; }
+template <int L> constexpr int tile_h() { return 64 / L / tile_w<L>(); }
+constexpr long long kManyLaneRays = 24576;
+inline float lane_rays(double pool_bytes) { return 75e3f + 36e3f * (float)std::log2(1.0 + pool_bytes / 24e6); }
 
 // Render modes of volume_kernel: emit into an RGBA image only, emit into a film
 // (and optionally RGBA), or resume a film.
@@ -798,7 +840,6 @@ template <int FMT, bool COUNT, int MODE, bool BIG, int LANES>
 __global__ __launch_bounds__(64) void volume_kernel(VolumeArgs a) {
   constexpr bool RESUME = MODE == kResume;
   constexpr bool THETA = MODE != kEmitRgba;
-  static_assert(LANES == 1 || (kTile % LANES == 0 && ref_group<FMT>() % LANES == 0), "lanes per ray");
   __shared__ float4 s_tf[kTfLds];
   __shared__ unsigned long long s_count;
   stage_tf(s_tf, a.tf, a.tf_n);
@@ -808,8 +849,8 @@ __global__ __launch_bounds__(64) void volume_kernel(VolumeArgs a) {
   using OFF = std::conditional_t<BIG, uint64_t, uint32_t>;
   const int ray = (int)threadIdx.x / LANES, h = (int)threadIdx.x % LANES;
   const int tx = rotated_tile_x();
-  const int x = tx * kTile + (ray % kTile);
-  const int y = blockIdx.y * (kTile / LANES) + (ray / kTile);
+  const int x = tx * tile_w<LANES>() + (ray % tile_w<LANES>());
+  const int y = blockIdx.y * tile_h<LANES>() + (ray / tile_w<LANES>());
   unsigned count = 0;
   bool handed = false;   // this lane's ray went to the cooperative march
   MarchState st;
@@ -825,7 +866,7 @@ __global__ __launch_bounds__(64) void volume_kernel(VolumeArgs a) {
     }
     if (live) {
       if constexpr (LANES > 1)
-        march_reference_coop<FMT, COUNT, THETA, OFF, LANES, ref_group<FMT>() / LANES>(a, s_tf, st, h, count);
+        march_reference_coop<FMT, COUNT, THETA, OFF, LANES, coop_group<LANES>() / LANES>(a, s_tf, st, h, count);
       else
         march_reference_grouped<FMT, ref_group<FMT>(), COUNT, THETA, OFF>(a, s_tf, st, count, handed);
     }
@@ -861,29 +902,34 @@ __global__ __launch_bounds__(64) void volume_kernel(VolumeArgs a) {
   }
 }
 
-// Lattice-schedule frame, one lane per ray (a kernel of its own: in
+// Lattice-schedule frame, LANES lanes per ray (a kernel of its own: in
 // volume_kernel it cost the reference march 11 registers).
-template <int FMT, bool COUNT, int MODE, bool BIG>
+template <int FMT, bool COUNT, int MODE, bool BIG, int LANES>
 __global__ __launch_bounds__(64) void lattice_kernel(VolumeArgs a) {
   __shared__ float4 s_tf[kTfLds];
   __shared__ unsigned long long s_count;
   stage_tf(s_tf, a.tf, a.tf_n);
   if (COUNT && threadIdx.x == 0) s_count = 0;
   __syncthreads();
-  const int x = rotated_tile_x() * kTile + (threadIdx.x % kTile);
-  const int y = blockIdx.y * kTile + (threadIdx.x / kTile);
+  const int ray = (int)threadIdx.x / LANES, h = (int)threadIdx.x % LANES;
+  const int x = rotated_tile_x() * tile_w<LANES>() + (ray % tile_w<LANES>());
+  const int y = blockIdx.y * tile_h<LANES>() + (ray / tile_w<LANES>());
   unsigned count = 0;
   if (x < a.W && y < a.H) {
     const size_t idx = (size_t)y * a.W + x;
     MarchState st;
-    bool live = true;
-    if (MODE == kResume) load_pixel(a, idx, st);
-    else live = emit(a, x, y, st);
-    if (MODE == kResume) live = st.nsteps > 0;
+    bool live;
+    if (MODE == kResume) {
+      load_pixel(a, idx, st);
+      live = st.nsteps > 0;
+    } else {
+      live = emit(a, x, y, st);
+    }
+    constexpr int U = LANES > 1 ? coop_group<LANES>() / LANES : ref_group<FMT>();
     if (live)
-      march_lattice<FMT, ref_group<FMT>(), COUNT, MODE != kEmitRgba, std::conditional_t<BIG, uint64_t, uint32_t>>(
-          a, s_tf, st, count);
-    store_pixel(a, idx, st);
+      march_lattice<FMT, LANES, U, COUNT, MODE != kEmitRgba, std::conditional_t<BIG, uint64_t, uint32_t>>(a, s_tf, st,
+                                                                                                         h, count);
+    if (h == 0) store_pixel(a, idx, st);
   }
   if (COUNT) {
     if (count) atomicAdd(&s_count, (unsigned long long)count);
@@ -1123,19 +1169,25 @@ __global__ __launch_bounds__(256) void segment_fold_kernel(const float4 *slots, 
 template <int FMT>
 hipError_t launch_segments_fmt(const VolumeArgs &a, hipStream_t s);
 
-template <int FMT, int MODE, bool BIG>
-void launch_mode(const VolumeArgs &a, hipStream_t s) {
-  constexpr int L = ref_lanes<FMT>();
-  const bool lattice = a.schedule == HYD_SCHED_LATTICE;
-  const int rows = lattice ? kTile : kTile / L;
-  const dim3 block(kTile * kTile), grid((a.W + kTile - 1) / kTile, (a.H + rows - 1) / rows);
-  if (lattice) {
-    if (a.samples) hipLaunchKernelGGL((lattice_kernel<FMT, true, MODE, BIG>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((lattice_kernel<FMT, false, MODE, BIG>), grid, block, 0, s, a);
+template <int FMT, int MODE, bool BIG, int L>
+void launch_lanes(const VolumeArgs &a, hipStream_t s) {
+  constexpr int w = tile_w<L>(), h = tile_h<L>();
+  const dim3 block(64), grid((a.W + w - 1) / w, (a.H + h - 1) / h);
+  if (a.schedule == HYD_SCHED_LATTICE) {
+    if (a.samples) hipLaunchKernelGGL((lattice_kernel<FMT, true, MODE, BIG, L>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((lattice_kernel<FMT, false, MODE, BIG, L>), grid, block, 0, s, a);
   } else {
     if (a.samples) hipLaunchKernelGGL((volume_kernel<FMT, true, MODE, BIG, L>), grid, block, 0, s, a);
     else hipLaunchKernelGGL((volume_kernel<FMT, false, MODE, BIG, L>), grid, block, 0, s, a);
   }
+}
+
+template <int FMT, int MODE, bool BIG>
+void launch_mode(const VolumeArgs &a, hipStream_t s) {
+  const long long rays = (long long)a.W * a.H;
+  if (rays <= kManyLaneRays) launch_lanes<FMT, MODE, BIG, kManyLanes>(a, s);
+  else if (a.full_rays <= lane_rays((double)a.pool_elems * sizeof(typename RawVox<FMT>::T))) launch_lanes<FMT, MODE, BIG, kLanes>(a, s);
+  else launch_lanes<FMT, MODE, BIG, 1>(a, s);
 }
 
 template <int FMT, bool BIG>

@@ -12,7 +12,7 @@ from tests.helpers import film_fields, oracle_film_fields, oracle_view, oracle_v
 pytestmark = pytest.mark.gpu
 
 
-def _scene(n, fmt, bs, arm, density=1e-2, tf=None, poke=None):
+def _scene(n, fmt, bs, arm, density=1e-2, tf=None, poke=None, W_=37, H_=29):
     vol = D.gen_blobs(n, 6, 31, sig=(4.0, 10.0), sigma_scale=n / 32.0, amp=(0.4, 1.0))
     if fmt == L.FMT_F32:
         vol = vol.astype(np.float32) / np.float32(255)
@@ -25,7 +25,7 @@ def _scene(n, fmt, bs, arm, density=1e-2, tf=None, poke=None):
         v[at] = np.resize(np.array(poke, v.dtype), at.size)
     b = D.make_bricked(vol, bs or n, 1 if bs else 0, fmt, None, resident=1.0, seed=5)
     geom = D.geometry((n, n, n), bs or n, 0.5)
-    return W.Scene("sampler", b, D.README_TF.copy() if tf is None else tf, 37, 29, arm, 60.0, geom, density=density)
+    return W.Scene("sampler", b, D.README_TF.copy() if tf is None else tf, W_, H_, arm, 60.0, geom, density=density)
 
 
 def _same(a, b):
@@ -80,3 +80,31 @@ def test_u8_normalisation_of_every_count(gpu_ctx):
     tf = np.stack([np.linspace(0, 1, 256)] * 3 + [np.linspace(0, 0.5, 256)], 1).astype(np.float32)
     sc = W.Scene("u8", b, tf, 33, 31, AXIS[2], 60.0, D.geometry((30, 30, 30), 30, 0.5), density=0.1)
     _check(gpu_ctx, sc)
+
+
+@pytest.mark.parametrize("fmt", [L.FMT_F32, L.FMT_F16, L.FMT_U8])
+@pytest.mark.parametrize("W_,H_", [(1, 1), (5, 3), (3, 8191), (163, 157), (641, 621)])
+def test_lanes_per_ray(gpu_ctx, fmt, W_, H_):
+    """Frames of few, some and many rays (16, 4 and 1 lanes per ray), with partial tiles, at a
+    density where steps escalate inside groups."""
+    sc = _scene(24, fmt, 8, AXIS[2], density=0.5, W_=W_, H_=H_)
+    if (W_, H_) != (3, 8191):
+        return _check(gpu_ctx, sc)
+    ctx = gpu_ctx          # a sliver: the oracle's image alone
+    ctx.load(sc.bricked, sc.tf)
+    img = ctx.render_volume(sc.volume_params(), sc.view(), sc.W, sc.H, film=False)["rgba"].cpu().numpy()
+    assert _same(img, oracle_volume(sc).render(oracle_view(sc), 32, film=False)["rgba"])
+
+
+@pytest.mark.parametrize("fmt", [L.FMT_F32, L.FMT_U8])
+@pytest.mark.parametrize("W_,H_", [(37, 29), (163, 157), (641, 621)])
+def test_lattice_lanes_per_ray(gpu_ctx, fmt, W_, H_):
+    """The lattice march at each number of lanes per ray: samples and counts of the oracle's (1e-4
+    for its rounding, as the lattice tests)."""
+    sc = _scene(24, fmt, 8, AXIS[2], density=0.2, W_=W_, H_=H_)
+    sc.schedule, sc.ert = L.SCHED_LATTICE, 0.9
+    gpu_ctx.load(sc.bricked, sc.tf)
+    out = gpu_ctx.render_volume(sc.volume_params(), sc.view(), sc.W, sc.H, film=True, count=True)
+    r = oracle_volume(sc).render(oracle_view(sc), 32, film=False)
+    assert int(out["samples"].item()) == r["samples"] > 0
+    assert np.max(np.abs(out["rgba"].cpu().numpy() - r["rgba"])) <= 1e-4
