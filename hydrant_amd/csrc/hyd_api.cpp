@@ -627,7 +627,7 @@ struct hyd_segment_set {
   const void *pool[hyd::kMaxSegBatches] = {};
   int32_t *codes = nullptr;   // [n][cells]
   float4 *pages = nullptr;    // [n][max_pages]
-  float k_min = 0.f, k_max = 0.f, lo = 0.f, hi = 0.f;   // page_range over every batch
+  int32_t inner = kInnerTest;   // kInner* that every batch's pages allow
 };
 
 extern "C" {
@@ -682,6 +682,10 @@ int32_t hyd_segment_set_create(hyd_ctx *c, int32_t n_batches, const hyd_segment_
     for (int k = 0; k < b[i].n_pages; ++k)
       pages[(size_t)i * set->max_pages + k] =
           make_float4(b[i].page_k[k], b[i].page_b[3 * k], b[i].page_b[3 * k + 1], b[i].page_b[3 * k + 2]);
+    float k_min, k_max, lo, hi;
+    page_range(pages.data() + (size_t)i * set->max_pages, b[i].n_pages, k_min, k_max, lo, hi);
+    const int32_t inner = inner_mapping(k_min, lo, hi, set->pad);
+    set->inner = i == 0 ? inner : std::min(set->inner, inner);
   }
   HYD_CHECK_HIP(hipMalloc((void **)&set->codes, codes.size() * sizeof(int32_t)));
   HYD_CHECK_HIP(hipMalloc((void **)&set->pages, pages.size() * sizeof(float4)));
@@ -713,6 +717,7 @@ int32_t hyd_segments_pass_set(hyd_ctx *c, const hyd_segment_set *set, const hyd_
   a.page = set->pages;
   a.pool_elems = set->max_pool_elems;
   a.pad = set->pad;
+  a.inner = c->tf_finite ? set->inner : (int32_t)kInnerNever;
   fill_view(view, a.trans, a.ctg, a.ray_o);
   a.W = width;
   a.H = height;

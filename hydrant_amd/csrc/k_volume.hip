@@ -1023,30 +1023,24 @@ __device__ __forceinline__ bool seg_walk_cell(const VolumeArgs &a, f3 o0, f3 d, 
 // Samples [kk, min(kk + U, kc)) of a run in cell ip of page pgid, their tap
 // loads in flight together, composited in order into seg.
 template <int FMT, bool COUNT, int U, typename OFF>
-__device__ __forceinline__ void seg_sample_group(const VolumeArgs &a, const float4 *s_tf, f3 o0,
-                                                 f3 d, float lf, f3 ip, float4 pgd, OFF page_base, int pgid, int kk,
-                                                 int kc, MarchState &seg, unsigned &count) {
-  RefTap<OFF> tp[U];
-  RawTaps<FMT> raw[U];
+__device__ __forceinline__ void seg_sample_group(const VolumeArgs &a, const float4 *s_tf, f3 o0, f3 d, float lf, f3 ip,
+                                                 float4 pgd, OFF page_base, int pgid, int kk, int kc, MarchState &seg,
+                                                 unsigned &count) {
+  f3 x[U];
   bool ok[U];
-  float wj[U];
+  float w[U];
 #pragma unroll
   for (int j = 0; j < U; ++j) {
+    x[j] = sub(lattice_pos(o0, d, lf, a.step, kk + j, w[j]), ip);
     ok[j] = kk + j < kc;
-    const f3 pj = lattice_pos(o0, d, lf, a.step, ok[j] ? kk + j : kk, wj[j]);
-    tp[j] = ref_tap<OFF>(sub(pj, ip), pgd, a.pad, page_base);
-    if (ok[j]) ref_fetch<FMT, OFF>(a.pool, tp[j], a.pad, raw[j]);
   }
-#pragma unroll
-  for (int j = 0; j < U; ++j) {
-    if (ok[j]) {
-      float cur[8];
-      ref_values<FMT, OFF>(raw[j], tp[j], a.pad, cur);
-      const float s = ref_interp(cur, tp[j]);
-      shade_composite_impl<true, false>(a, s_tf, s, pgid, seg, wj[j]);
-      if (COUNT) ++count;
-    }
-  }
+  bool inner = a.inner == kInnerAlways;
+  if (a.inner == kInnerTest) inner = __all(ok[U - 1] & inner_span(x[0], x[U - 1], pgd, a.pad));
+  float4 ub[U];
+  group_colours<FMT, OFF, U, true>(a, s_tf, inner, x, ok, pgd, page_base, pgid, ub, w);
+  int n = 0;
+  composite_group<0, U, false>([&](auto j) { return ub[decltype(j)::value]; }, ok, INFINITY, seg, n);
+  if (COUNT) count += (unsigned)n;
 }
 
 template <int FMT, bool COUNT, bool BIG, bool MULTI>
