@@ -608,6 +608,7 @@ int32_t hyd_segments_pass(hyd_ctx *c, const hyd_volume_params *p, const hyd_view
   fill_view(view, a.trans, a.ctg, a.ray_o);
   a.W = width;
   a.H = height;
+  a.full_rays = full_rays(a);
   a.macro.cls = nullptr;
   a.slots = reinterpret_cast<float4 *>(slots_dev);
   a.nslots = nslots_dev;
@@ -627,6 +628,14 @@ struct hyd_segment_set {
   const void *pool[hyd::kMaxSegBatches] = {};
   int32_t *codes = nullptr;   // [n][cells]
   float4 *pages = nullptr;    // [n][max_pages]
+  // every batch together, when no two hold the same brick: cell codes over the
+  // pages of all, page descriptors [sum of pages], first voxels from `base`
+  bool together = false;
+  int32_t *all_codes = nullptr;
+  float4 *all_pages = nullptr;
+  uint64_t *all_bases = nullptr;
+  const void *base = nullptr;
+  uint64_t span = 0;          // bytes from base to the end of the highest pool
   int32_t inner = kInnerTest;   // kInner* that every batch's pages allow
 };
 
@@ -635,8 +644,9 @@ extern "C" {
 int32_t hyd_segment_set_destroy(hyd_segment_set *set) {
   if (!set) return HYD_OK;
   if (hipSetDevice(set->device) == hipSuccess) {
-    if (set->codes) (void)hipFree(set->codes);
-    if (set->pages) (void)hipFree(set->pages);
+    for (void *p : {(void *)set->codes, (void *)set->pages, (void *)set->all_codes, (void *)set->all_pages,
+                    (void *)set->all_bases})
+      if (p) (void)hipFree(p);
   }
   delete set;
   return HYD_OK;
@@ -651,7 +661,7 @@ int32_t hyd_segment_set_create(hyd_ctx *c, int32_t n_batches, const hyd_segment_
               n_batches, kMaxSegBatches);
   HYD_REQUIRE(!c->host_cheb.empty(), HYD_ERR_STATE, "no empty-space grid: call hyd_set_empty_grid first");
   const size_t cells = c->host_cheb.size();
-  std::unique_ptr<hyd_segment_set> set(new hyd_segment_set);
+  std::unique_ptr<hyd_segment_set, int32_t (*)(hyd_segment_set *)> set(new hyd_segment_set, hyd_segment_set_destroy);
   set->device = c->device;
   set->n = n_batches;
   set->fmt = b[0].fmt;
@@ -687,6 +697,48 @@ int32_t hyd_segment_set_create(hyd_ctx *c, int32_t n_batches, const hyd_segment_
     const int32_t inner = inner_mapping(k_min, lo, hi, set->pad);
     set->inner = i == 0 ? inner : std::min(set->inner, inner);
   }
+  // the batches as one pool
+  std::vector<int32_t> all(cells, -1);
+  std::vector<float4> all_pages;
+  std::vector<uint64_t> bases;
+  const size_t elem = fmt_bytes(set->fmt), page_elems = (size_t)set->pad * set->pad * set->pad;
+  uintptr_t lo = UINTPTR_MAX, hi = 0;
+  for (int i = 0; i < n_batches; ++i) {
+    lo = std::min(lo, (uintptr_t)b[i].pool_dev);
+    hi = std::max(hi, (uintptr_t)b[i].pool_dev + b[i].n_pages * page_elems * elem);
+  }
+  set->together = true;
+  for (int i = 0; i < n_batches; ++i) {
+    const uintptr_t off = (uintptr_t)b[i].pool_dev - lo;
+    const int32_t first = (int32_t)all_pages.size();
+    set->together = set->together && off % elem == 0 && all_pages.size() + (size_t)b[i].n_pages <= 0x7fffffffu;
+    for (size_t j = 0; j < cells && set->together; ++j) {
+      const int32_t c = codes[(size_t)i * cells + j];
+      if (c <= -2) all[j] = c;
+      if (c >= 0) {
+        set->together = all[j] == -1;   // else two batches hold this brick: one pass each
+        all[j] = first + c;
+      }
+    }
+    if (!set->together) break;
+    for (int k = 0; k < b[i].n_pages; ++k) {
+      all_pages.push_back(pages[(size_t)i * set->max_pages + k]);
+      bases.push_back(off / elem + (uint64_t)k * page_elems);
+    }
+  }
+  set->base = reinterpret_cast<const void *>(lo);
+  set->span = hi - lo;
+  if (set->together) {
+    HYD_CHECK_HIP(hipMalloc((void **)&set->all_codes, cells * sizeof(int32_t)));
+    HYD_CHECK_HIP(hipMalloc((void **)&set->all_pages, all_pages.size() * sizeof(float4)));
+    HYD_CHECK_HIP(hipMalloc((void **)&set->all_bases, bases.size() * sizeof(uint64_t)));
+    HYD_CHECK_HIP(hipMemcpy(set->all_codes, all.data(), cells * sizeof(int32_t), hipMemcpyHostToDevice));
+    HYD_CHECK_HIP(
+        hipMemcpy(set->all_pages, all_pages.data(), all_pages.size() * sizeof(float4), hipMemcpyHostToDevice));
+    HYD_CHECK_HIP(hipMemcpy(set->all_bases, bases.data(), bases.size() * sizeof(uint64_t), hipMemcpyHostToDevice));
+    *out = set.release();
+    return HYD_OK;
+  }
   HYD_CHECK_HIP(hipMalloc((void **)&set->codes, codes.size() * sizeof(int32_t)));
   HYD_CHECK_HIP(hipMalloc((void **)&set->pages, pages.size() * sizeof(float4)));
   HYD_CHECK_HIP(hipMemcpy(set->codes, codes.data(), codes.size() * sizeof(int32_t), hipMemcpyHostToDevice));
@@ -712,29 +764,33 @@ int32_t hyd_segments_pass_set(hyd_ctx *c, const hyd_segment_set *set, const hyd_
   if ((st = fill_volume_args(c, p, a))) return st;
   HYD_REQUIRE(a.schedule == HYD_SCHED_LATTICE, HYD_ERR_ARG, "segments need the lattice schedule");
   std::memcpy(a.vdim, set->vdim, sizeof(a.vdim));
-  a.pool = set->pool[0];
-  a.codes = set->codes;
-  a.page = set->pages;
-  a.pool_elems = set->max_pool_elems;
   a.pad = set->pad;
   a.inner = c->tf_finite ? set->inner : (int32_t)kInnerNever;
   fill_view(view, a.trans, a.ctg, a.ray_o);
   a.W = width;
   a.H = height;
+  a.full_rays = full_rays(a);
   a.macro.cls = nullptr;
   a.slots = reinterpret_cast<float4 *>(slots_dev);
   a.nslots = nslots_dev;
   a.max_slots = max_slots;
   a.samples = samples_dev;
-  SegBatchTable tb{};
-  tb.n = set->n;
-  const size_t cells = (size_t)set->vdim[0] * set->vdim[1] * set->vdim[2];
-  for (int i = 0; i < set->n; ++i) {
-    tb.pool[i] = set->pool[i];
-    tb.codes[i] = set->codes + (size_t)i * cells;
-    tb.page[i] = set->pages + (size_t)i * set->max_pages;
+  if (set->together) {
+    a.pool = set->base;
+    a.codes = set->all_codes;
+    a.page = set->all_pages;
+    a.page_base = set->all_bases;
+    HYD_CHECK_HIP(launch_segments_set(a, set->span, set->fmt, c->stream));
+    return HYD_OK;
   }
-  HYD_CHECK_HIP(launch_segments_batches(a, tb, set->fmt, c->stream));
+  const size_t cells = (size_t)set->vdim[0] * set->vdim[1] * set->vdim[2];
+  a.pool_elems = set->max_pool_elems;
+  for (int i = 0; i < set->n; ++i) {
+    a.pool = set->pool[i];
+    a.codes = set->codes + (size_t)i * cells;
+    a.page = set->pages + (size_t)i * set->max_pages;
+    HYD_CHECK_HIP(launch_segments_pass(a, set->fmt, c->stream));
+  }
   return HYD_OK;
 }
 

@@ -986,7 +986,7 @@ __device__ __forceinline__ bool same_cell(f3 p, f3 ip) {
 // and the slot index and return false.  A resident cell returns true with
 // its run [k, kc), its cell ip and its page id, k and ord unchanged.
 __device__ __forceinline__ bool seg_walk_cell(const VolumeArgs &a, f3 o0, f3 d, f3 invr, float lf, int kend,
-                                              float cdu, size_t P, size_t ray, int &k, int &ord, f3 &ip, int &kc,
+                                              float cdu, size_t P, size_t ray, bool writes, int &k, int &ord, f3 &ip, int &kc,
                                               int &pgid) {
   float w;
   const f3 o = lattice_pos(o0, d, lf, a.step, k, w);
@@ -1000,7 +1000,7 @@ __device__ __forceinline__ bool seg_walk_cell(const VolumeArgs &a, f3 o0, f3 d, 
     const float t_exit = t + tfar + float(cd - 1) * cdu;
     const int kn = (int)ceilf(t_exit / a.step - 0.5f);
     k = kn > k + 1 ? kn : k + 1;
-    a.slots[(size_t)ord * P + ray] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (writes) a.slots[(size_t)ord * P + ray] = make_float4(0.f, 0.f, 0.f, 0.f);
     ++ord;
     return false;
   }
@@ -1020,45 +1020,60 @@ __device__ __forceinline__ bool seg_walk_cell(const VolumeArgs &a, f3 o0, f3 d, 
   return true;
 }
 
-// Samples [kk, min(kk + U, kc)) of a run in cell ip of page pgid, their tap
-// loads in flight together, composited in order into seg.
-template <int FMT, bool COUNT, int U, typename OFF>
+// Samples [kk, min(kk + G U, kc)) of a run in cell ip of page pgid, their tap
+// loads in flight together, composited in order into seg.  The G lanes of a
+// ray resolve samples kk + h + G u each and composite all of them.
+template <int FMT, bool COUNT, int G, int U, typename OFF>
 __device__ __forceinline__ void seg_sample_group(const VolumeArgs &a, const float4 *s_tf, f3 o0, f3 d, float lf, f3 ip,
-                                                 float4 pgd, OFF page_base, int pgid, int kk, int kc, MarchState &seg,
-                                                 unsigned &count) {
+                                                 float4 pgd, OFF page_base, int pgid, int kk, int kc, int h,
+                                                 MarchState &seg, unsigned &count) {
   f3 x[U];
-  bool ok[U];
+  bool ok[U], okn[G * U];
   float w[U];
 #pragma unroll
-  for (int j = 0; j < U; ++j) {
-    x[j] = sub(lattice_pos(o0, d, lf, a.step, kk + j, w[j]), ip);
-    ok[j] = kk + j < kc;
+  for (int u = 0; u < U; ++u) {
+    // a lane past the run repeats its first sample
+    const int k = kk + h + G * u;
+    x[u] = sub(lattice_pos(o0, d, lf, a.step, k < kc ? k : kk, w[u]), ip);
+    ok[u] = k < kc || (G > 1 && u == 0);
   }
+#pragma unroll
+  for (int j = 0; j < G * U; ++j) okn[j] = kk + j < kc;
   bool inner = a.inner == kInnerAlways;
-  if (a.inner == kInnerTest) inner = __all(ok[U - 1] & inner_span(x[0], x[U - 1], pgd, a.pad));
+  if (a.inner == kInnerTest) inner = __all(inner_span(x[0], x[U - 1], pgd, a.pad));
   float4 ub[U];
   group_colours<FMT, OFF, U, true>(a, s_tf, inner, x, ok, pgd, page_base, pgid, ub, w);
   int n = 0;
-  composite_group<0, U, false>([&](auto j) { return ub[decltype(j)::value]; }, ok, INFINITY, seg, n);
-  if (COUNT) count += (unsigned)n;
+  composite_group<0, G * U, false>(
+      [&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        const float4 &uk = ub[j / G];
+        if constexpr (G > 1)
+          return make_float4(group_bcast<G, j % G>(uk.x), group_bcast<G, j % G>(uk.y), group_bcast<G, j % G>(uk.z),
+                             group_bcast<G, j % G>(uk.w));
+        else
+          return uk;
+      },
+      okn, INFINITY, seg, n);
+  if (COUNT && h == 0) count += (unsigned)n;
 }
 
-template <int FMT, bool COUNT, bool BIG, bool MULTI>
-__global__ __launch_bounds__(64) void segment_kernel(VolumeArgs a, SegBatchTable tb) {
+// MULTI: a segment set, whose cells name the pages of every batch: the ray is
+// walked once for all batches.  (With one layer of workgroups per batch, each
+// walked every ray's cells and found a third of them resident: 4.10 against
+// 2.81 ms for three batches of a 1024^3 u8 volume at 512^2.)
+template <int FMT, bool COUNT, bool BIG, bool MULTI, int LANES>
+__global__ __launch_bounds__(64) void segment_kernel(VolumeArgs a) {
   using OFF = std::conditional_t<BIG, uint64_t, uint32_t>;
-  if (MULTI) {   // this workgroup's residency batch
-    a.pool = tb.pool[blockIdx.z];
-    a.codes = tb.codes[blockIdx.z];
-    a.page = tb.page[blockIdx.z];
-  }
-  constexpr int U = HYD_SEG_GROUP;
+  constexpr int U = LANES > 1 ? coop_group<LANES>() / LANES : HYD_SEG_GROUP;
   __shared__ float4 s_tf[kTfLds];
   __shared__ unsigned long long s_count;
   stage_tf(s_tf, a.tf, a.tf_n);
   if (COUNT && threadIdx.x == 0) s_count = 0;
   __syncthreads();
-  const int x = rotated_tile_x() * kTile + (threadIdx.x % kTile);
-  const int y = blockIdx.y * kTile + (threadIdx.x / kTile);
+  const int r = (int)threadIdx.x / LANES, h = (int)threadIdx.x % LANES;
+  const int x = rotated_tile_x() * tile_w<LANES>() + (r % tile_w<LANES>());
+  const int y = blockIdx.y * tile_h<LANES>() + (r / tile_w<LANES>());
   unsigned count = 0;
   if (x < a.W && y < a.H) {
     const size_t P = (size_t)a.W * a.H, ray = (size_t)y * a.W + x;
@@ -1074,30 +1089,31 @@ __global__ __launch_bounds__(64) void segment_kernel(VolumeArgs a, SegBatchTable
       int k = 0, kc = 0, pgid = -1;
       f3 ip{0.f, 0.f, 0.f};
       MarchState seg;
-      if constexpr (MULTI) {
-        // the batches' waves fill the chip: the wave walks its rays' cells in
-        // lock-step (the lanes in resident cells composite their runs while
-        // the others wait), which issues the fewest instructions
+      if constexpr (MULTI || LANES > 1) {
+        // the wave walks its rays' cells in lock-step (the lanes in resident
+        // cells composite their runs while the others wait): its rays stay in
+        // the same bricks, whose lines they share, and it issues the fewest
+        // instructions
         while (k < kend && ord < a.max_slots) {
-          if (!seg_walk_cell(a, o0, d, invr, lf, kend, cdu, P, ray, k, ord, ip, kc, pgid)) continue;
+          if (!seg_walk_cell(a, o0, d, invr, lf, kend, cdu, P, ray, h == 0, k, ord, ip, kc, pgid)) continue;
           const float4 pgd = a.page[pgid];
-          const OFF page_base = (OFF)pgid * pad3;
+          const OFF page_base = MULTI ? (OFF)a.page_base[pgid] : (OFF)pgid * pad3;
           seg.v = make_float4(0.f, 0.f, 0.f, 0.f);
-          for (int kk = k; kk < kc; kk += U)
-            seg_sample_group<FMT, COUNT, U, OFF>(a, s_tf, o0, d, lf, ip, pgd, page_base, pgid, kk, kc, seg,
-                                                 count);
-          a.slots[(size_t)ord * P + ray] = seg.v;
+          for (int kk = k; kk < kc; kk += LANES * U)
+            seg_sample_group<FMT, COUNT, LANES, U, OFF>(a, s_tf, o0, d, lf, ip, pgd, page_base, pgid, kk, kc, h, seg,
+                                                        count);
+          if (h == 0) a.slots[(size_t)ord * P + ray] = seg.v;
           ++ord;
           k = kc;
         }
       } else {
-        // one batch: the waves do not fill the chip and lanes idle in
-        // lock-step cost time, so each lane composites U samples of its own
-        // run per iteration; lanes whose run ended wait until a quarter of
-        // the wave's busy lanes (or all of them) need to walk, then walk
-        // together to their next resident run (7.47 -> 6.84 ms for three
-        // one-batch passes of the 1024^3 frame; 5.16 against 4.58 ms in the
-        // set launch, which is instruction-issue bound)
+        // one batch of a large frame: lanes idle in lock-step cost time where
+        // most cells are not resident, so each lane composites U samples of
+        // its own run per iteration; lanes whose run ended wait until a
+        // quarter of the wave's busy lanes (or all of them) need to walk, then
+        // walk together to their next resident run (7.47 -> 6.84 ms for three
+        // one-batch passes of the 1024^3 frame; 4.21 -> 6.53 ms in a set,
+        // whose rays then leave each other's bricks)
         bool in_run = false;
         int kk = 0;
         float4 pgd = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1109,7 +1125,7 @@ __global__ __launch_bounds__(64) void segment_kernel(VolumeArgs a, SegBatchTable
           const bool walk_now = m_run == 0 || 4 * __popcll(m_want) >= __popcll(m_want | m_run);
           if (want && walk_now) {
             while (k < kend && ord < a.max_slots) {
-              if (!seg_walk_cell(a, o0, d, invr, lf, kend, cdu, P, ray, k, ord, ip, kc, pgid)) continue;
+              if (!seg_walk_cell(a, o0, d, invr, lf, kend, cdu, P, ray, true, k, ord, ip, kc, pgid)) continue;
               pgd = a.page[pgid];
               page_base = (OFF)pgid * pad3;
               seg.v = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1119,8 +1135,8 @@ __global__ __launch_bounds__(64) void segment_kernel(VolumeArgs a, SegBatchTable
             }
           }
           if (!in_run) continue;
-          seg_sample_group<FMT, COUNT, U, OFF>(a, s_tf, o0, d, lf, ip, pgd, page_base, pgid, kk, kc, seg,
-                                               count);
+          seg_sample_group<FMT, COUNT, 1, U, OFF>(a, s_tf, o0, d, lf, ip, pgd, page_base, pgid, kk, kc, 0, seg,
+                                                  count);
           kk += U;
           if (kk >= kc) {   // the run is complete: its slot, then the next cell
             a.slots[(size_t)ord * P + ray] = seg.v;
@@ -1131,7 +1147,7 @@ __global__ __launch_bounds__(64) void segment_kernel(VolumeArgs a, SegBatchTable
         }
       }
     }
-    a.nslots[ray] = ord;
+    if (h == 0) a.nslots[ray] = ord;
   }
   if (COUNT) {
     if (count) atomicAdd(&s_count, (unsigned long long)count);
@@ -1159,9 +1175,6 @@ __global__ __launch_bounds__(256) void segment_fold_kernel(const float4 *slots, 
   }
   rgba[i] = v;
 }
-
-template <int FMT>
-hipError_t launch_segments_fmt(const VolumeArgs &a, hipStream_t s);
 
 template <int FMT, int MODE, bool BIG, int L>
 void launch_lanes(const VolumeArgs &a, hipStream_t s) {
@@ -1201,25 +1214,29 @@ bool force_offsets64() {
   return on;
 }
 
-template <int FMT, bool MULTI>
-void launch_segments_multi(const VolumeArgs &a, const SegBatchTable &tb, hipStream_t s) {
-  dim3 grid((a.W + kTile - 1) / kTile, (a.H + kTile - 1) / kTile, MULTI ? tb.n : 1);
-  // pool_elems is the largest pool's when MULTI
-  const uint64_t bytes = a.pool_elems * (uint64_t)sizeof(typename RawVox<FMT>::T);
-  const bool big = bytes > (1ull << 32) || force_offsets64();
+template <int FMT, bool MULTI, int L>
+void launch_segments_lanes(const VolumeArgs &a, bool big, hipStream_t s) {
+  constexpr int w = tile_w<L>(), h = tile_h<L>();
+  const dim3 grid((a.W + w - 1) / w, (a.H + h - 1) / h), block(64);
   if (a.samples) {
-    if (big) hipLaunchKernelGGL((segment_kernel<FMT, true, true, MULTI>), grid, dim3(64), 0, s, a, tb);
-    else hipLaunchKernelGGL((segment_kernel<FMT, true, false, MULTI>), grid, dim3(64), 0, s, a, tb);
+    if (big) hipLaunchKernelGGL((segment_kernel<FMT, true, true, MULTI, L>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((segment_kernel<FMT, true, false, MULTI, L>), grid, block, 0, s, a);
   } else {
-    if (big) hipLaunchKernelGGL((segment_kernel<FMT, false, true, MULTI>), grid, dim3(64), 0, s, a, tb);
-    else hipLaunchKernelGGL((segment_kernel<FMT, false, false, MULTI>), grid, dim3(64), 0, s, a, tb);
+    if (big) hipLaunchKernelGGL((segment_kernel<FMT, false, true, MULTI, L>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((segment_kernel<FMT, false, false, MULTI, L>), grid, block, 0, s, a);
   }
 }
 
-template <int FMT>
-hipError_t launch_segments_fmt(const VolumeArgs &a, hipStream_t s) {
-  SegBatchTable none{};
-  launch_segments_multi<FMT, false>(a, none, s);
+// Lanes per ray as for frames, from the bytes the launch reads, but 4 lanes up
+// to twice the work: in lock-step a run of 4-lane groups wastes less of its
+// wave (512^2 frame of a 1024^3 u8 set: 4.21 ms with one lane, 2.81 with four;
+// eight drawn sets 1.17 and 2.19 times as fast as one layer of workgroups per batch).
+template <int FMT, bool MULTI>
+hipError_t launch_segments(const VolumeArgs &a, uint64_t bytes, hipStream_t s) {
+  const bool big = bytes > (1ull << 32) || force_offsets64();
+  if ((long long)a.W * a.H <= kManyLaneRays) launch_segments_lanes<FMT, MULTI, kManyLanes>(a, big, s);
+  else if (a.full_rays <= 2.f * lane_rays((double)bytes)) launch_segments_lanes<FMT, MULTI, kLanes>(a, big, s);
+  else launch_segments_lanes<FMT, MULTI, 1>(a, big, s);
   return hipGetLastError();
 }
 
@@ -1250,19 +1267,18 @@ hipError_t launch_segments_clear(float4 *slots, size_t n, hipStream_t s) {
 
 hipError_t launch_segments_pass(const VolumeArgs &a, int fmt, hipStream_t s) {
   switch (fmt) {
-    case HYD_FMT_U8: return launch_segments_fmt<HYD_FMT_U8>(a, s);
-    case HYD_FMT_F16: return launch_segments_fmt<HYD_FMT_F16>(a, s);
-    default: return launch_segments_fmt<HYD_FMT_F32>(a, s);
+    case HYD_FMT_U8: return launch_segments<HYD_FMT_U8, false>(a, a.pool_elems, s);
+    case HYD_FMT_F16: return launch_segments<HYD_FMT_F16, false>(a, a.pool_elems * 2, s);
+    default: return launch_segments<HYD_FMT_F32, false>(a, a.pool_elems * 4, s);
   }
 }
 
-hipError_t launch_segments_batches(const VolumeArgs &a, const SegBatchTable &tb, int fmt, hipStream_t s) {
+hipError_t launch_segments_set(const VolumeArgs &a, uint64_t span_bytes, int fmt, hipStream_t s) {
   switch (fmt) {
-    case HYD_FMT_U8: launch_segments_multi<HYD_FMT_U8, true>(a, tb, s); break;
-    case HYD_FMT_F16: launch_segments_multi<HYD_FMT_F16, true>(a, tb, s); break;
-    default: launch_segments_multi<HYD_FMT_F32, true>(a, tb, s); break;
+    case HYD_FMT_U8: return launch_segments<HYD_FMT_U8, true>(a, span_bytes, s);
+    case HYD_FMT_F16: return launch_segments<HYD_FMT_F16, true>(a, span_bytes, s);
+    default: return launch_segments<HYD_FMT_F32, true>(a, span_bytes, s);
   }
-  return hipGetLastError();
 }
 
 hipError_t launch_segments_composite(const float4 *slots, const int32_t *nslots, int max_slots, int P, float4 *rgba,

@@ -108,3 +108,40 @@ def test_lattice_lanes_per_ray(gpu_ctx, fmt, W_, H_):
     r = oracle_volume(sc).render(oracle_view(sc), 32, film=False)
     assert int(out["samples"].item()) == r["samples"] > 0
     assert np.max(np.abs(out["rgba"].cpu().numpy() - r["rgba"])) <= 1e-4
+
+
+@pytest.mark.parametrize("fmt", [L.FMT_U8, L.FMT_F16, L.FMT_F32])
+@pytest.mark.parametrize("W_,H_,overlap", [(37, 29, False), (163, 157, False), (163, 157, True), (1201, 621, False)])
+def test_segment_sets_at_every_lane_count(gpu_ctx, fmt, W_, H_, overlap):
+    """A segment set (one walk for all batches; one pass each when two batches hold a brick) fills
+    the slots of one pass per batch, at 16, 4 and 1 lanes per ray: image and counts bit for bit."""
+    import torch
+
+    sc = _scene(40, fmt, 8, AXIS[2], density=0.2, W_=W_, H_=H_)
+    sc.schedule = L.SCHED_LATTICE
+    b = sc.bricked
+    order = b.order
+    parts = [order[0::3], order[1::3], order[2::3]]
+    if overlap:
+        parts[1] = np.concatenate([parts[1], parts[0][:2]])
+    batches = []
+    for ids in parts:
+        pool = b.pool[b.vaddr.reshape(-1)[ids]]
+        va = np.full(b.vaddr.shape, -1, np.int32)
+        va.reshape(-1)[ids] = np.arange(len(ids), dtype=np.int32)
+        t = torch.from_numpy(pool.view(np.int16) if pool.dtype == np.uint16 else pool).cuda()
+        batches.append((fmt, b.pad, t, va, b.page_k[:1].repeat(len(ids)), np.repeat(b.page_b[:1], len(ids), axis=0)))
+    gpu_ctx.load(b, sc.tf)
+    p, view = sc.volume_params(), sc.view()
+    ref, rc = gpu_ctx.render_sort_last_resident(p, view, W_, H_, batches, b.grid, count=True)
+    gpu_ctx.load(b, sc.tf)
+    sset = gpu_ctx.segment_set(batches)
+    got, gc = gpu_ctx.render_sort_last_set(p, view, W_, H_, sset, count=True)
+    gpu_ctx.synchronize()
+    assert int(rc.item()) == int(gc.item()) > 0
+    assert torch.equal(ref, got)
+    if not overlap:
+        one = gpu_ctx.render_volume(p, view, W_, H_, film=False, count=True)
+        assert int(one["samples"].item()) == int(gc.item())
+        assert float((one["rgba"] - got).abs().max()) <= 1e-5
+    sset.close()
