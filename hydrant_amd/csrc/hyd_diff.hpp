@@ -1,6 +1,8 @@
 // Internal declarations of the differentiable renderer.
 #pragma once
 
+#include <algorithm>
+
 #include "hyd_internal.hpp"
 
 namespace hyd {
@@ -35,7 +37,8 @@ struct DiffArgs {
   float *dsmax;                // [view][y][x] max |dL/ds| of the ray (0: nothing to scatter)
   float4 *rays;                // [view][y][x][2] setup of active rays: (dx, dy, dz, tnear), (dt, 0, 0, 0)
   float *blocks;               // [view group][brick][10^3] voxel-gradient blocks (brick + one-voxel halo)
-  int32_t view_groups;         // scatter workgroups per brick (views split into contiguous groups)
+  int32_t view_groups;         // scatter workgroups per brick: contiguous groups of views, or (a multiple of
+                               // n_views) equal shares of each view's rays
   float *bound;                // [kDiffBoundParts] partial bounds of one sample's TF-gradient term
   unsigned long long *gtf_acc; // [4][256] fixed-point TF-gradient sums of the launch
   int32_t *tile_counter;       // [1] work queue of the ray-order pass
@@ -50,15 +53,20 @@ inline size_t diff_bricks(int32_t nx, int32_t ny, int32_t nz) {
   return (size_t)((nx + 7) / 8) * (size_t)((ny + 7) / 8) * (size_t)((nz + 7) / 8);
 }
 
-// view groups of the scatter: about kDiffScatterWgs workgroups in all (128 per CU
+// View groups of the scatter: about kDiffScatterWgs workgroups in all (128 per CU
 // of MI355X, so that the slow bricks' workgroups are spread over a long launch),
-// at most one group per view
-constexpr size_t kDiffScatterWgs = 32768;
+// at most one group per view; when that leaves fewer than kDiffScatterMin, each
+// view's rays are split over up to kDiffRaySplits groups (a workgroup's rounds
+// are one dependent chain: six views at 64^2 of a 48^3 volume, 1,296 workgroups,
+// took 607 us; the whole step 1350 us, 1005 with eight shares).
+constexpr size_t kDiffScatterWgs = 32768, kDiffScatterMin = 8192, kDiffRaySplits = 8;
 
 inline int32_t diff_view_groups(int32_t nx, int32_t ny, int32_t nz, int32_t n_views) {
-  const size_t nb = diff_bricks(nx, ny, nz);
-  const size_t g = (kDiffScatterWgs + nb - 1) / nb;
-  return (int32_t)(g < 1 ? 1 : (g > (size_t)n_views ? (size_t)n_views : g));
+  const size_t nb = diff_bricks(nx, ny, nz), v = (size_t)n_views;
+  const size_t g = std::max<size_t>(1, (kDiffScatterWgs + nb - 1) / nb);
+  if (g < v) return (int32_t)g;
+  const size_t splits = std::min(kDiffRaySplits, std::max<size_t>(1, kDiffScatterMin / (nb * v)));
+  return (int32_t)(v * splits);
 }
 
 // floats of the dL/ds buffer ([view][y][x][k])

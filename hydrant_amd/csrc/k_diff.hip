@@ -679,8 +679,10 @@ __global__ __launch_bounds__(64) void diff_scatter_kernel(DiffArgs a) {
   const int bx = (bl % nbx + 5 * bz) % nbx, by = ((bl / nbx) % nby + 3 * bz) % nby;
   const int bi = (bz * nby + by) * nbx + bx;
   // views of this workgroup: a contiguous share of the launch's views
-  const int v_begin = (int)((long long)a.n_views * grp / a.view_groups);
-  const int v_end = (int)((long long)a.n_views * (grp + 1) / a.view_groups);
+  // (or one view, of whose rays it takes a share)
+  const int splits = max(1, a.view_groups / a.n_views), part = grp % splits;
+  const int v_begin = (int)((long long)a.n_views * (grp / splits) / (a.view_groups / splits));
+  const int v_end = (int)((long long)a.n_views * (grp / splits + 1) / (a.view_groups / splits));
   BrickBox bb;
   bb.X0 = bx * kBrick; bb.Y0 = by * kBrick; bb.Z0 = bz * kBrick;
   bb.cx0 = bb.X0 == 0 ? -1 : bb.X0; bb.cy0 = bb.Y0 == 0 ? -1 : bb.Y0; bb.cz0 = bb.Z0 == 0 ? -1 : bb.Z0;
@@ -729,6 +731,7 @@ __global__ __launch_bounds__(64) void diff_scatter_kernel(DiffArgs a) {
     const int bw = px1 - px0 + 1, bh = py1 - py0 + 1;
     if (bw <= 0 || bh <= 0) continue;
     const int nR = bw * bh;
+    const int r0 = (int)((long long)nR * part / splits), r1 = (int)((long long)nR * (part + 1) / splits);
     // the view's scale: the largest |dL/ds| of the box's rays times 2^e below
     // 2^30, less 3 bits for the register sums, less the bits for every listed
     // sample adding to one slot beyond 2^33 terms
@@ -741,11 +744,11 @@ __global__ __launch_bounds__(64) void diff_scatter_kernel(DiffArgs a) {
     const int e = fixed_exponent(B, hv + kScatterBits);
     const float scale = ldexpf(1.f, e);
     int n = 0, total = 0;   // rays and segments in the list (wave-uniform)
-    for (int base = 0; base < nR; base += 64) {
+    for (int base = r0; base < r1; base += 64) {
       const int rr = base + lane;
       int cnt = 0, k0 = 0, k1 = -1, ray = 0;
       RaySetup rs{};
-      if (rr < nR) {
+      if (rr < r1) {
         const int y = py0 + rr / bw, x = px0 + rr % bw;
         ray = (view * a.H + y) * a.W + x;
         if (a.dsmax[ray] > 0.f) {   // an active ray: its setup was stored by the ray-order pass
