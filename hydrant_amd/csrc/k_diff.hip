@@ -162,53 +162,77 @@ __device__ __forceinline__ void position(const RaySetup &r, int k, float &px, fl
   pz = r.oz + r.dz * t;
 }
 
-template <bool COUNT>
+// Lane J of each group of G lanes (a quad, or a row of 16), to all of the group.
+template <int G, int J> __device__ __forceinline__ float lane_bcast(float v) {
+  if constexpr (G == 1) return v;
+  else return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), G == 4 ? J * 0x55 : 0x150 + J, 0xF, 0xF, false));
+}
+
+// Composites samples J .. N-1 of a group (sample j held by lane j / U, slot j % U)
+// while below n.
+template <int G, int U, int J>
+__device__ __forceinline__ void forward_over(const Shade (&sh)[U], int n, float (&C)[3], float &T, float &amax) {
+  const float alpha = lane_bcast<G, J / U>(sh[J % U].alpha), c0 = lane_bcast<G, J / U>(sh[J % U].c[0]),
+              c1 = lane_bcast<G, J / U>(sh[J % U].c[1]), c2 = lane_bcast<G, J / U>(sh[J % U].c[2]);
+  if (J < n) {
+    const float ta = T * alpha;
+    C[0] = fmaf(ta, c0, C[0]);
+    C[1] = fmaf(ta, c1, C[1]);
+    C[2] = fmaf(ta, c2, C[2]);
+    T = T * (1.f - alpha);
+    amax = fmaxf(amax, alpha);
+  }
+  if constexpr (J + 1 < G * U) forward_over<G, U, J + 1>(sh, n, C, T, amax);
+}
+
+// G lanes hold one ray: each resolves and shades U consecutive samples of a
+// group of G U, all composite them in order (the same sums as one lane's).
+template <bool COUNT, int G>
 __global__ __launch_bounds__(64) void diff_forward_kernel(DiffArgs a) {
+  constexpr int U = G == 4 ? 2 : 1, N = G * U, TW = G == 16 ? 4 : kTile, TH = 64 / G / TW;
   __shared__ float4 s_tf[kMaxTf];
   __shared__ unsigned long long s_count;
   for (int i = threadIdx.x; i < a.tf_n; i += 64) s_tf[i] = reinterpret_cast<const float4 *>(a.tf)[i];
   if (COUNT && threadIdx.x == 0) s_count = 0;
   __syncthreads();
-  const int view = blockIdx.z;
-  const int x = rotated_tile_x() * kTile + (threadIdx.x % kTile);
-  const int y = blockIdx.y * kTile + (threadIdx.x / kTile);
+  const int view = blockIdx.z, r = (int)threadIdx.x / G, h = (int)threadIdx.x % G;
+  const int x = rotated_tile_x() * TW + (r % TW);
+  const int y = blockIdx.y * TH + (r / TW);
   unsigned count = 0;
   if (x < a.W && y < a.H) {
     const size_t ray = ((size_t)view * a.H + y) * a.W + x;
     float *ck = a.ckpts + ray * a.nck;
-    RaySetup r;
+    RaySetup rs;
     const VolumeRef vr = volume_ref(a);
-    float C0 = 0.f, C1 = 0.f, C2 = 0.f, T = 1.f;
+    float C[3] = {0.f, 0.f, 0.f}, T = 1.f;
     const int nseg = a.nck - 1;
-    if (setup(a, a.views[view], x, y, r)) {
-      const float nl = opacity_const(a.sigma, r.dt);
+    if (setup(a, a.views[view], x, y, rs)) {
+      const float nl = opacity_const(a.sigma, rs.dt);
       TapCache tcf;   // consecutive samples in one cell share their taps
       for (int seg = 0; seg < nseg; ++seg) {
         const float Tstart = T;
         float amax = 0.f;
         const int k0 = seg * a.ckpt, k1 = min(a.K, k0 + a.ckpt);
-        for (int k = k0; k < k1; ++k) {
-          float px, py, pz;
-          position(r, k, px, py, pz);
-          Smp sm;
-          sample_reuse(a, vr, px, py, pz, sm, tcf);
-          Shade sh;
-          shade(s_tf, a.tf_n, nl, sm.s, sh);
-          const float ta = T * sh.alpha;
-          C0 = fmaf(ta, sh.c[0], C0);
-          C1 = fmaf(ta, sh.c[1], C1);
-          C2 = fmaf(ta, sh.c[2], C2);
-          T = T * (1.f - sh.alpha);
-          amax = fmaxf(amax, sh.alpha);
+        for (int k = k0; k < k1; k += N) {
+          Shade sh[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            float px, py, pz;
+            position(rs, min(k + h * U + u, k1 - 1), px, py, pz);
+            Smp sm;
+            sample_reuse(a, vr, px, py, pz, sm, tcf);
+            shade(s_tf, a.tf_n, nl, sm.s, sh[u]);
+          }
+          forward_over<G, U, 0>(sh, k1 - k, C, T, amax);
         }
-        if (COUNT) count += (unsigned)(k1 - k0);
-        ck[seg] = amax > 0.5f ? -Tstart : Tstart;   // sign bit: recompute this segment exactly
+        if (COUNT && h == 0) count += (unsigned)(k1 - k0);
+        if (h == 0) ck[seg] = amax > 0.5f ? -Tstart : Tstart;   // sign bit: recompute this segment exactly
       }
-      ck[nseg] = T;
-    } else {
+      if (h == 0) ck[nseg] = T;
+    } else if (h == 0) {
       for (int i = 0; i < a.nck; ++i) ck[i] = 1.f;
     }
-    a.rgba[ray] = make_float4(C0, C1, C2, 1.f - T);
+    if (h == 0) a.rgba[ray] = make_float4(C[0], C[1], C[2], 1.f - T);
   }
   if (COUNT) {
     if (count) atomicAdd(&s_count, (unsigned long long)count);
@@ -875,10 +899,24 @@ __global__ __launch_bounds__(256) void diff_combine_kernel(DiffArgs a) {
 
 }  // namespace
 
+namespace {
+template <int G> void launch_forward_lanes(const DiffArgs &a, hipStream_t s) {
+  constexpr int tw = G == 16 ? 4 : kTile, th = 64 / G / tw;
+  const dim3 grid((a.W + tw - 1) / tw, (a.H + th - 1) / th, a.n_views);
+  if (a.samples) hipLaunchKernelGGL((diff_forward_kernel<true, G>), grid, dim3(64), 0, s, a);
+  else hipLaunchKernelGGL((diff_forward_kernel<false, G>), grid, dim3(64), 0, s, a);
+}
+}  // namespace
+
+// Lanes per ray: 16 while the launch stays around six waves per SIMD, 4 while
+// one lane per ray would not give every SIMD two waves, then one (as the frame
+// marches: a ray's samples are one chain).  Whole step of six 64^2 views, one
+// lane and sixteen: 1005 and 961 us.
 hipError_t launch_diff_forward(const DiffArgs &a, hipStream_t s) {
-  dim3 grid((a.W + kTile - 1) / kTile, (a.H + kTile - 1) / kTile, a.n_views);
-  if (a.samples) hipLaunchKernelGGL(diff_forward_kernel<true>, grid, dim3(64), 0, s, a);
-  else hipLaunchKernelGGL(diff_forward_kernel<false>, grid, dim3(64), 0, s, a);
+  const long long rays = (long long)a.n_views * a.W * a.H;
+  if (rays <= 24576) launch_forward_lanes<16>(a, s);
+  else if (rays <= 131072) launch_forward_lanes<4>(a, s);
+  else launch_forward_lanes<1>(a, s);
   return hipGetLastError();
 }
 
