@@ -155,18 +155,18 @@ void fill_view(const hyd_view *v, float trans[16], float &ctg, f3 &ray_o) {
   ray_o = f3{v->ray_o[0], v->ray_o[1], v->ray_o[2]};
 }
 
-// The work of a frame as a number of rays of its longest chord: an 8 x 8 grid
-// of its pixels' chords through the box.
-float full_rays(const VolumeArgs &a) {
-  const float px = float(a.W) * float(a.H);
+}  // namespace
+
+// An 8 x 8 grid of the frame's pixels' chords through the box stands for all.
+float full_rays(const float *trans, float ctg, f3 ray_o, int W, int H, f3 bmin, f3 bmax) {
+  const float px = float(W) * float(H);
   if (px <= 24576.f || px > 4194304.f) return px;   // decided by the pixels alone
   double sum = 0.0, longest = 0.0;
   for (int j = 0; j < 8; ++j)
     for (int i = 0; i < 8; ++i) {
-      const int x = (int)((2ll * i + 1) * a.W / 16), y = (int)((2ll * j + 1) * a.H / 16);
+      const int x = (int)((2ll * i + 1) * W / 16), y = (int)((2ll * j + 1) * H / 16);
       float tn, tf;
-      if (!intersect_box(a.ray_o, pixel_ray_dir(a.trans, a.ctg, a.ray_o, x, y, a.W, a.H), a.bmin, a.bmax, tn, tf))
-        continue;
+      if (!intersect_box(ray_o, pixel_ray_dir(trans, ctg, ray_o, x, y, W, H), bmin, bmax, tn, tf)) continue;
       const double c = std::max(0.0, (double)tf) - std::max(0.0, (double)tn);
       if (!(c > 0.0)) continue;
       sum += c;
@@ -174,8 +174,6 @@ float full_rays(const VolumeArgs &a) {
     }
   return longest > 0.0 ? (float)(px * sum / (64.0 * longest)) : px;
 }
-
-}  // namespace
 
 namespace {
 // Device staging of the z order for hyd_composite_noalloc: a file-scope device
@@ -455,7 +453,7 @@ int32_t hyd_render_volume(hyd_ctx *c, const hyd_volume_params *p, const hyd_view
   a.film = film_dev;
   a.rgba = reinterpret_cast<float4 *>(rgba_dev);
   a.samples = samples_dev;
-  a.full_rays = full_rays(a);
+  a.full_rays = full_rays(a.trans, a.ctg, a.ray_o, a.W, a.H, a.bmin, a.bmax);
   HYD_CHECK_HIP(launch_volume(a, c->pool.fmt, false, c->stream));
   return HYD_OK;
 }
@@ -608,7 +606,7 @@ int32_t hyd_segments_pass(hyd_ctx *c, const hyd_volume_params *p, const hyd_view
   fill_view(view, a.trans, a.ctg, a.ray_o);
   a.W = width;
   a.H = height;
-  a.full_rays = full_rays(a);
+  a.full_rays = full_rays(a.trans, a.ctg, a.ray_o, a.W, a.H, a.bmin, a.bmax);
   a.macro.cls = nullptr;
   a.slots = reinterpret_cast<float4 *>(slots_dev);
   a.nslots = nslots_dev;
@@ -769,7 +767,7 @@ int32_t hyd_segments_pass_set(hyd_ctx *c, const hyd_segment_set *set, const hyd_
   fill_view(view, a.trans, a.ctg, a.ray_o);
   a.W = width;
   a.H = height;
-  a.full_rays = full_rays(a);
+  a.full_rays = full_rays(a.trans, a.ctg, a.ray_o, a.W, a.H, a.bmin, a.bmax);
   a.macro.cls = nullptr;
   a.slots = reinterpret_cast<float4 *>(slots_dev);
   a.nslots = nslots_dev;

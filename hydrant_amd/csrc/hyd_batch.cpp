@@ -1,6 +1,7 @@
 // C ABI of the batched renderer: multi-volume set, batch plans, HIP-graph
 // capture/replay and the launch-shape autotuner.
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
@@ -8,6 +9,7 @@
 #include <vector>
 
 #include "hyd_batch.hpp"
+#include "hyd_macro.hpp"
 
 namespace hyd {
 namespace {
@@ -45,6 +47,7 @@ struct hyd_batch {
   std::vector<int32_t> chunks[kPlans];
   unsigned *d_counters = nullptr;
   int64_t total_px = 0;
+  double full_rays = 0.0;   // over the views (full_rays)
   int32_t max_volume = 0;   // largest volume index the views name
   // captured graph
   hipGraph_t graph = nullptr;
@@ -209,6 +212,8 @@ int32_t fill_args(Ctx *c, hyd_batch *b, const hyd_batch_config *cfg, float densi
   int32_t st = ensure_tiles(b, cfg->tile_w, group, c->stream);
   if (st) return st;
   if ((st = ensure_oriented(c))) return st;
+  const uint8_t *cls = nullptr;
+  if ((st = macro_batch(c, &cls))) return st;
   const int slot = plan_slot(cfg->tile_w, group);
   std::memset(&a, 0, sizeof(a));
   a.tiles = b->d_tiles[slot];
@@ -227,6 +232,19 @@ int32_t fill_args(Ctx *c, hyd_batch *b, const hyd_batch_config *cfg, float densi
     a.pools[1] = a.oriented ? c->own_oriented : c->pool.data;
     a.pools[2] = a.oriented ? static_cast<const char *>(c->own_oriented) + layout_bytes(c) : c->pool.data;
   }
+  // opacities in [0, 1], as the classes take them
+  if (cls && density >= 0.f && c->tf_alpha_max * density <= 1.f) {
+    a.cls = cls;
+    a.nm = macro_edge(c->pool.pad);
+    a.cells_per_page = (uint32_t)a.nm * a.nm * a.nm;
+  }
+  // Four lanes a ray (8 x 8 tiles, unroll 4) while the views' rays leave a wave
+  // a few tiles at most, so that the longest rays' chains bound the launch: ten
+  // batches of 4 to 12 views took 0.47 of their time before on average, 0.58
+  // with one lane; from 175k full rays on, one lane was the faster (no samples past the brick's end, taps reused).  The line is
+  // the one of the frames (lane_rays).
+  const bool quads = cfg->tile_w == 8 && group == 1 && cfg->unroll == 4;
+  a.lanes = quads && b->full_rays <= lane_rays((double)layout_bytes(c)) ? 4 : 1;
   a.pad = c->pool.pad;
   a.page_elems = (uint32_t)c->pool.pad * c->pool.pad * c->pool.pad;
   a.tf = c->tf;
@@ -250,6 +268,7 @@ int32_t hyd_set_volumes(hyd_ctx *c, int32_t n, const hyd_volume_desc *vols) {
   HYD_REQUIRE(n >= 1 && vols, HYD_ERR_ARG, "empty volume set");
   std::vector<BatchVolDev> dv(n);
   std::vector<int32_t> cells;
+  std::vector<float> scale;   // of each page a volume names (NaN: two volumes' scales differ)
   int pad = -1, max_page = -1;
   for (int v = 0; v < n; ++v) {
     const hyd_volume_desc &d = vols[v];
@@ -276,6 +295,10 @@ int32_t hyd_set_volumes(hyd_ctx *c, int32_t n, const hyd_volume_desc *vols) {
       if (cd == 0 && c->pool.data)
         HYD_REQUIRE(pg < c->pool.n_pages, HYD_ERR_RANGE, "volume %d cell %zu: page %d beyond the pool", v, i, pg);
       if (cd == 0) max_page = std::max(max_page, pg);
+      if (cd == 0 && pg >= 0) {
+        if ((size_t)pg >= scale.size()) scale.resize((size_t)pg + 1, 0.f);
+        scale[pg] = scale[pg] == 0.f || scale[pg] == d.value_scale ? d.value_scale : NAN;
+      }
       cells.push_back(cd > 0 ? -1 - cd : pg);
     }
   }
@@ -294,6 +317,9 @@ int32_t hyd_set_volumes(hyd_ctx *c, int32_t n, const hyd_volume_desc *vols) {
   c->n_vols = n;
   c->vol_pad = pad;
   c->vol_max_page = max_page;
+  c->page_scale = std::move(scale);
+  c->vol_bmax.resize(n);
+  for (int v = 0; v < n; ++v) std::copy(vols[v].bbox_max, vols[v].bbox_max + 3, c->vol_bmax[v].begin());
   return HYD_OK;
 }
 
@@ -321,11 +347,16 @@ int32_t hyd_batch_create(hyd_ctx *c, const hyd_batch_view *views, int32_t n_view
     dv[i].out_offset = v.out_offset;
     b->total_px = std::max<int64_t>(b->total_px, v.out_offset + (int64_t)v.width * v.height);
     b->max_volume = std::max(b->max_volume, v.volume);
+    if (b->full_rays < 1e7) {
+      const std::array<float, 3> &e = c->vol_bmax[v.volume];
+      b->full_rays += full_rays(v.view.trans, v.view.ctg_fovy_2, f3{v.view.ray_o[0], v.view.ray_o[1], v.view.ray_o[2]},
+                                v.width, v.height, f3{0.f, 0.f, 0.f}, f3{e[0], e[1], e[2]});
+    }
   }
   void *p = nullptr;
   if ((st = dev_upload(&p, dv.data(), dv.size() * sizeof(BatchViewDev), c->stream))) { delete b; return st; }
   b->d_views = static_cast<BatchViewDev *>(p);
-  if (hipMalloc((void **)&b->d_counters, kXcds * sizeof(unsigned)) != hipSuccess) {
+  if (hipMalloc((void **)&b->d_counters, kXcds * kCounterStride * sizeof(unsigned)) != hipSuccess) {
     (void)hipFree(b->d_views);
     delete b;
     set_error("hipMalloc of the work counters failed");

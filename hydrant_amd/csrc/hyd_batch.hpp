@@ -6,6 +6,10 @@
 namespace hyd {
 
 constexpr int kXcds = 8;   // MI355X: 8 XCDs, workgroups dispatched round-robin over them
+// Words between the XCDs' work counters: each has a line of its own.  In one
+// line, the claims of all waves, eight of them empty-handed at a wave's end,
+// queued on it: the smallest drawn batch took 527 us, and 152 us now.
+constexpr int kCounterStride = 64;
 
 struct BatchViewDev {
   float trans[16];
@@ -29,13 +33,19 @@ struct BatchVolDev {
 struct BatchArgs {
   const uint32_t *tiles;       // view << 16 | ty << 8 | tx
   int32_t chunk_start[kXcds + 1];
-  unsigned *counters;          // kXcds work counters, zeroed by reset_counters
+  unsigned *counters;          // kXcds work counters, kCounterStride apart, zeroed by reset_counters
   const BatchViewDev *views;
   const BatchVolDev *vols;
   const int32_t *cells;        // concatenated cell codes of every volume
   const void *pools[3];         // the pool in its three layouts (x, y, z fastest)
   int32_t oriented;             // 0: only the x-fastest layout is held (every tile reads layout 0)
   int32_t pairs;                // 1: pools[] are the row-pair layouts (2 voxels per element); 2: the quad layouts (4)
+  // macrocell classes of every page (null: none), macrocells per page edge and
+  // per page (hyd_macro.hpp)
+  const uint8_t *cls;
+  int32_t nm;
+  uint32_t cells_per_page;
+  int32_t lanes;               // lanes per ray, 1 or 4 (4: 8 x 8 tiles, unroll 4, single waves)
   int32_t pad;
   uint32_t page_elems;         // pad^3
   const float *tf;

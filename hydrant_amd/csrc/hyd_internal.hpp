@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <array>
+#include <cmath>
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
@@ -116,6 +118,16 @@ struct Ctx {
   uint64_t mm_gen = ~0ull;        // pool_gen the ranges were made from
   bool mcls_valid = false;        // own_mcls belongs to own_mm and the current transfer function
   double macro_empty = 0.0;       // share of the pool's macrocells that are empty
+  // classes for the batched renderer: each page under the value scale of its
+  // volume (NaN: none, or two that differ), made at the first batched launch
+  // after a change of pool, transfer function or volume set
+  std::vector<float> page_scale;
+  std::vector<std::array<float, 3>> vol_bmax;   // extent of each volume of the set
+  float *own_bscale = nullptr;
+  uint8_t *own_bflags = nullptr, *own_bcls = nullptr;
+  size_t bcls_cap = 0, bscale_cap = 0;
+  uint64_t bcls_gen = ~0ull;      // batch_state_gen of own_bcls
+  double bcls_empty = 0.0;
   // differentiable renderer: device copy of the views
   void *own_diff_views = nullptr;
   int32_t diff_view_cap = 0;
@@ -198,6 +210,13 @@ struct VolumeArgs {
   int32_t max_slots;
   const uint64_t *page_base;   // segment sets: first voxel of each page, in voxels from pool
 };
+
+// The work of a frame as a number of rays of its longest chord (hyd_api.cpp).
+float full_rays(const float *trans, float ctg, f3 ray_o, int W, int H, f3 bmin, f3 bmax);
+
+// The work (full_rays) up to which a march of a pool of that size runs four
+// lanes per ray (measurements: k_volume.hip).
+inline float lane_rays(double pool_bytes) { return 75e3f + 36e3f * (float)std::log2(1.0 + pool_bytes / 24e6); }
 
 hipError_t launch_volume(const VolumeArgs &a, int fmt, bool resume, hipStream_t s);
 hipError_t launch_segments_clear(float4 *slots, size_t n, hipStream_t s);
@@ -288,6 +307,9 @@ int32_t macro_tf_set(Ctx *c);
 void macro_free(Ctx *c);
 // Points the march at the classes when they apply to it, else leaves it without.
 void macro_fill(const Ctx *c, VolumeArgs &a);
+// The batched renderer's classes of the current pool, brought up to date
+// (complete on return); null in *cls when the march should sample throughout.
+int32_t macro_batch(Ctx *c, const uint8_t **cls);
 struct IsoArgs;
 void macro_fill_iso(const Ctx *c, IsoArgs &a);
 

@@ -1,6 +1,7 @@
 // Host side of the macrocells: when they are made and when a march may use them.
 #include <algorithm>
 #include <cmath>
+#include <vector>
 
 #include "hyd_macro.hpp"
 
@@ -32,6 +33,12 @@ bool reserve(Ctx *c, size_t cells) {
   return true;
 }
 
+int32_t batch_classes(Ctx *c, int32_t first, int32_t n) {
+  HYD_CHECK_HIP(launch_macro_classes(c->own_mm, c->pool.pad, first, n, c->tf, c->tf_n, 1.f, c->own_bscale,
+                                     c->own_bflags, c->own_bcls, c->own_mcount, c->stream));
+  return HYD_OK;
+}
+
 int32_t classes(Ctx *c, int32_t first, int32_t n) {
   const float scale = c->pool.fmt == HYD_FMT_U8 ? 1.f / 255.f : 1.f;
   HYD_CHECK_HIP(launch_macro_classes(c->own_mm, c->pool.pad, first, n, c->tf, c->tf_n, scale, nullptr,
@@ -47,6 +54,12 @@ void macro_free(Ctx *c) {
   c->own_mm = nullptr;
   c->own_mflags = c->own_mcls = nullptr;
   c->own_mcount = nullptr;
+  for (void *p : {(void *)c->own_bscale, (void *)c->own_bflags, (void *)c->own_bcls})
+    if (p) (void)hipFree(p);
+  c->own_bscale = nullptr;
+  c->own_bflags = c->own_bcls = nullptr;
+  c->bcls_cap = c->bscale_cap = 0;
+  c->bcls_gen = ~0ull;
   c->macro_cap = 0;
   c->mm_gen = ~0ull;
   c->mcls_valid = false;
@@ -85,7 +98,60 @@ int32_t macro_pages_written(Ctx *c, int32_t first, int32_t n) {
     int32_t st = classes(c, first, n);
     if (st) return st;
   }
+  if (c->bcls_gen == c->batch_state_gen) {   // in place: captured graphs read them
+    int32_t st = batch_classes(c, first, n);
+    if (st) return st;
+  }
   HYD_CHECK_HIP(hipStreamSynchronize(c->stream));
+  return HYD_OK;
+}
+
+// Classes of every page under the scale of the volumes that name it, for the
+// batched march: made once per state of pool, table and volume set.
+int32_t macro_batch(Ctx *c, const uint8_t **cls) {
+  *cls = nullptr;
+  // a zero contribution leaves the composite as it is while colours are finite
+  if (!c->tf_finite || !(c->tf_rgb_max <= 1e15f) || !(c->tf_alpha_min >= 0.f)) return HYD_OK;
+  const size_t n = (size_t)c->pool.n_pages, cells = n * page_cells(c);
+  if (c->bcls_gen != c->batch_state_gen) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    HYD_CHECK_HIP(hipStreamIsCapturing(c->stream, &cap));
+    if (cap != hipStreamCaptureStatusNone) return HYD_OK;   // made by the next launch outside it
+    c->bcls_gen = ~0ull;
+    if (cells > 0xffffffffull || !reserve(c, cells)) return HYD_OK;   // 32-bit class offsets
+    if (c->bcls_cap < cells || c->bscale_cap < n) {
+      for (void *p : {(void *)c->own_bscale, (void *)c->own_bflags, (void *)c->own_bcls})
+        if (p) (void)hipFree(p);
+      c->own_bscale = nullptr;
+      c->own_bflags = c->own_bcls = nullptr;
+      c->bcls_cap = c->bscale_cap = 0;
+      if (hipMalloc((void **)&c->own_bscale, n * sizeof(float)) != hipSuccess ||
+          hipMalloc((void **)&c->own_bflags, cells) != hipSuccess ||
+          hipMalloc((void **)&c->own_bcls, cells) != hipSuccess) {
+        (void)hipGetLastError();
+        return HYD_OK;
+      }
+      c->bcls_cap = cells;
+      c->bscale_cap = n;
+    }
+    if (c->mm_gen != c->pool_gen) {   // a bound pool's, with its oriented copies
+      HYD_CHECK_HIP(launch_macro_minmax(c->pool.fmt, c->pool.data, c->pool.pad, 0, (int)n, c->own_mm, c->stream));
+      c->mm_gen = c->pool_gen;
+      c->mcls_valid = false;
+    }
+    std::vector<float> scale(c->page_scale);
+    scale.resize(n, NAN);
+    unsigned long long count = 0;
+    HYD_CHECK_HIP(hipMemcpyAsync(c->own_bscale, scale.data(), n * sizeof(float), hipMemcpyHostToDevice, c->stream));
+    HYD_CHECK_HIP(hipMemcpyAsync(c->own_mcount, &count, sizeof(count), hipMemcpyHostToDevice, c->stream));
+    int32_t st = batch_classes(c, 0, (int32_t)n);
+    if (st) return st;
+    HYD_CHECK_HIP(hipMemcpyAsync(&count, c->own_mcount, sizeof(count), hipMemcpyDeviceToHost, c->stream));
+    HYD_CHECK_HIP(hipStreamSynchronize(c->stream));
+    c->bcls_empty = 1.0 - (double)count / (double)cells;
+    c->bcls_gen = c->batch_state_gen;
+  }
+  if (c->bcls_empty >= kMacroWorth) *cls = c->own_bcls;
   return HYD_OK;
 }
 

@@ -12,7 +12,6 @@
 // staged in LDS per workgroup.
 #include <hip/hip_fp16.h>
 
-#include <cmath>
 #include <cstdlib>
 #include <type_traits>
 #include <utility>
@@ -830,7 +829,6 @@ template <int L> constexpr int coop_group() { return L == kManyLanes ? 16 : 8; }
 template <int L> constexpr int tile_w() { return L == kManyLanes ? 4 : kTile; }
 template <int L> constexpr int tile_h() { return 64 / L / tile_w<L>(); }
 constexpr long long kManyLaneRays = 24576;
-inline float lane_rays(double pool_bytes) { return 75e3f + 36e3f * (float)std::log2(1.0 + pool_bytes / 24e6); }
 
 // Render modes of volume_kernel: emit into an RGBA image only, emit into a film
 // (and optionally RGBA), or resume a film.
