@@ -236,6 +236,27 @@ int32_t activate(Ctx *c) {
   return HYD_OK;
 }
 
+namespace {
+// The z order for a launch: in its arguments, or copied to *owned, which the caller frees
+// after the launch (stage: a device array to copy to instead).
+int32_t place_z_order(Ctx *c, int32_t n, const int32_t *z_order, int32_t *stage, ZOrder &z, int32_t **owned) {
+  z.dev = nullptr;
+  if (owned) *owned = nullptr;
+  if (n <= kArgZ) {
+    std::memcpy(z.v, z_order, n * sizeof(int32_t));
+    return HYD_OK;
+  }
+  int32_t *dev = stage;
+  if (!dev) {
+    HYD_CHECK_HIP(hipMallocAsync((void **)&dev, n * sizeof(int32_t), c->stream));
+    *owned = dev;
+  }
+  HYD_CHECK_HIP(hipMemcpyAsync(dev, z_order, n * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
+  z.dev = dev;
+  return HYD_OK;
+}
+}  // namespace
+
 }  // namespace hyd
 
 using namespace hyd;
@@ -509,12 +530,12 @@ int32_t hyd_composite(hyd_ctx *c, int32_t n, const hyd_fetch_pixel *partials_dev
                 "z_order must be a permutation of 0..%d", n - 1);
     seen[z_order[i]] = 1;
   }
+  ZOrder z{};
   int32_t *zdev = nullptr;
-  HYD_CHECK_HIP(hipMallocAsync((void **)&zdev, n * sizeof(int32_t), c->stream));
-  HYD_CHECK_HIP(hipMemcpyAsync(zdev, z_order, n * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
-  hipError_t e = launch_composite(n, partials_dev, zdev, width, height, reinterpret_cast<float4 *>(rgba_dev),
+  if ((st = place_z_order(c, n, z_order, nullptr, z, &zdev))) return st;
+  hipError_t e = launch_composite(n, partials_dev, z, width, height, reinterpret_cast<float4 *>(rgba_dev),
                                   rgb_dev, c->srgb8_t, c->stream);
-  (void)hipFreeAsync(zdev, c->stream);
+  if (zdev) (void)hipFreeAsync(zdev, c->stream);
   HYD_CHECK_HIP(e);
   HYD_CHECK_HIP(hipStreamSynchronize(c->stream));
   return HYD_OK;
@@ -538,8 +559,9 @@ int32_t hyd_composite_noalloc(hyd_ctx *c, int32_t n, const hyd_fetch_pixel *part
   }
   int32_t *zdev = scratch_ptr(c->device);
   HYD_REQUIRE(zdev, HYD_ERR_STATE, "no scratch address resolved for device %d", c->device);
-  HYD_CHECK_HIP(hipMemcpyAsync(zdev, z_order, n * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
-  HYD_CHECK_HIP(launch_composite(n, partials_dev, zdev, width, height, reinterpret_cast<float4 *>(rgba_dev), rgb_dev,
+  ZOrder z{};
+  if ((st = place_z_order(c, n, z_order, zdev, z, nullptr))) return st;
+  HYD_CHECK_HIP(launch_composite(n, partials_dev, z, width, height, reinterpret_cast<float4 *>(rgba_dev), rgb_dev,
                                  c->srgb8_t, c->stream));
   HYD_CHECK_HIP(hipStreamSynchronize(c->stream));
   return HYD_OK;
@@ -572,11 +594,11 @@ int32_t hyd_composite_iso(hyd_ctx *c, int32_t n, const hyd_iso_fetch_pixel *part
                 "z_order must be a permutation of 0..%d", n - 1);
     seen[z_order[i]] = 1;
   }
+  ZOrder z{};
   int32_t *zdev = nullptr;
-  HYD_CHECK_HIP(hipMallocAsync((void **)&zdev, n * sizeof(int32_t), c->stream));
-  HYD_CHECK_HIP(hipMemcpyAsync(zdev, z_order, n * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
-  hipError_t e = launch_iso_composite(n, partials_dev, zdev, width, height, rgb_dev, depth_dev, c->stream);
-  (void)hipFreeAsync(zdev, c->stream);
+  if ((st = place_z_order(c, n, z_order, nullptr, z, &zdev))) return st;
+  hipError_t e = launch_iso_composite(n, partials_dev, z, width, height, rgb_dev, depth_dev, c->stream);
+  if (zdev) (void)hipFreeAsync(zdev, c->stream);
   HYD_CHECK_HIP(e);
   HYD_CHECK_HIP(hipStreamSynchronize(c->stream));
   return HYD_OK;

@@ -232,10 +232,21 @@ hipError_t launch_volume_trace(const VolumeArgs &a, int fmt, int x, int y, hyd_t
                                int *n_dev, hipStream_t s);
 hipError_t launch_pixel_pass(const float4 *rgba, int W, int H, uchar3 clear, uint8_t *rgb, hipStream_t s);
 hipError_t launch_fetch_pass(const hyd_volume_pixel *film, int W, int H, hyd_fetch_pixel *out, hipStream_t s);
-hipError_t launch_composite(int n, const hyd_fetch_pixel *partials, const int32_t *z_order_dev, int W, int H,
+// The z order of a composite, held by the launch's arguments up to kArgZ images
+// and in device memory beyond (256 bytes of arguments; a node's ranks fit).
+// An allocation, a copy and a free about each composite of eight 1024^2 images made
+// it 83 us; without them, and with four images' loads in flight, it takes 77
+// (the copy's rate gives 61).
+constexpr int kArgZ = 64;
+struct ZOrder {
+  const int32_t *dev;   // null: v
+  int32_t v[kArgZ];
+  __host__ __device__ int at(int k) const { return dev ? dev[k] : v[k]; }
+};
+hipError_t launch_composite(int n, const hyd_fetch_pixel *partials, const ZOrder &z, int W, int H,
                             float4 *rgba, uint8_t *rgb, const float *srgb_t, hipStream_t s);
 hipError_t launch_iso_fetch(const hyd_iso_pixel *px, int W, int H, hyd_iso_fetch_pixel *out, hipStream_t s);
-hipError_t launch_iso_composite(int n, const hyd_iso_fetch_pixel *partials, const int32_t *z_order_dev, int W, int H,
+hipError_t launch_iso_composite(int n, const hyd_iso_fetch_pixel *partials, const ZOrder &z, int W, int H,
                                 uint8_t *rgb, float *depth, hipStream_t s);
 // t[0] = -inf, t[k] (k = 1..255) = least float whose saturated sRGB byte is >= k
 // (volume.cc:175-181,284-288 evaluated on the host).

@@ -70,7 +70,7 @@ __device__ __forceinline__ uint8_t srgb8(const float *t, float x) {
 // Front-to-back "over" of n partial images in z order, then sRGB + saturate
 // (volume.cc:267-292).  One lane per pixel; partials are image-major.
 __global__ __launch_bounds__(kBlock) void composite_kernel(int n, const hyd_fetch_pixel *partials,
-                                                           const int32_t *z_order, int P, float4 *rgba,
+                                                           ZOrder z, int P, float4 *rgba,
                                                            uint8_t *rgb, const float *srgb_t) {
   __shared__ float s_t[256];
   s_t[threadIdx.x] = srgb_t[threadIdx.x];
@@ -78,9 +78,10 @@ __global__ __launch_bounds__(kBlock) void composite_kernel(int n, const hyd_fetc
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= P) return;
   const float4 *base = reinterpret_cast<const float4 *>(partials);
-  float4 f = base[((size_t)z_order[0] * P + i) * 2 + 1];
+  float4 f = base[((size_t)z.at(0) * P + i) * 2 + 1];
+#pragma unroll 4
   for (int k = 1; k < n; ++k) {
-    const size_t j = ((size_t)z_order[k] * P + i) * 2;
+    const size_t j = ((size_t)z.at(k) * P + i) * 2;
     const float4 bt = base[j];      // theta, phi
     const float4 bv = base[j + 1];  // val
     const float vx = f.x + bv.x - f.w * bt.x;
@@ -116,13 +117,13 @@ __global__ __launch_bounds__(kBlock) void iso_fetch_kernel(const hyd_iso_pixel *
 // z_order[0] is the front; each later one in z order replaces a front pixel
 // whose depth is strictly greater.  Writes the bytes and, if asked, the depth.
 __global__ __launch_bounds__(kBlock) void iso_composite_kernel(int n, const hyd_iso_fetch_pixel *partials,
-                                                               const int32_t *z_order, int P, uint8_t *rgb,
+                                                               ZOrder z, int P, uint8_t *rgb,
                                                                float *depth) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= P) return;
-  hyd_iso_fetch_pixel front = partials[(size_t)z_order[0] * P + i];
+  hyd_iso_fetch_pixel front = partials[(size_t)z.at(0) * P + i];
   for (int k = 1; k < n; ++k) {
-    const hyd_iso_fetch_pixel back = partials[(size_t)z_order[k] * P + i];
+    const hyd_iso_fetch_pixel back = partials[(size_t)z.at(k) * P + i];
     if (back.depth < front.depth) front = back;
   }
   if (rgb) {
@@ -155,11 +156,11 @@ hipError_t launch_fetch_pass(const hyd_volume_pixel *film, int W, int H, hyd_fet
   return hipGetLastError();
 }
 
-hipError_t launch_composite(int n, const hyd_fetch_pixel *partials, const int32_t *z_order_dev, int W, int H,
+hipError_t launch_composite(int n, const hyd_fetch_pixel *partials, const ZOrder &z, int W, int H,
                             float4 *rgba, uint8_t *rgb, const float *srgb_t, hipStream_t s) {
   const int P = W * H;
   hipLaunchKernelGGL(composite_kernel, dim3((P + kBlock - 1) / kBlock), dim3(kBlock), 0, s, n, partials,
-                     z_order_dev, P, rgba, rgb, srgb_t);
+                     z, P, rgba, rgb, srgb_t);
   return hipGetLastError();
 }
 
@@ -169,11 +170,11 @@ hipError_t launch_iso_fetch(const hyd_iso_pixel *px, int W, int H, hyd_iso_fetch
   return hipGetLastError();
 }
 
-hipError_t launch_iso_composite(int n, const hyd_iso_fetch_pixel *partials, const int32_t *z_order_dev, int W, int H,
+hipError_t launch_iso_composite(int n, const hyd_iso_fetch_pixel *partials, const ZOrder &z, int W, int H,
                                 uint8_t *rgb, float *depth, hipStream_t s) {
   const int P = W * H;
   hipLaunchKernelGGL(iso_composite_kernel, dim3((P + kBlock - 1) / kBlock), dim3(kBlock), 0, s, n, partials,
-                     z_order_dev, P, rgb, depth);
+                     z, P, rgb, depth);
   return hipGetLastError();
 }
 
