@@ -1,7 +1,7 @@
 // Volume ray-march kernels for gfx950.
 //
-// One lane per pixel; a 64-lane workgroup covers an 8x8 pixel tile so a
-// wavefront marches a coherent ray packet.  Ray emit, box clip and the march
+// One, 4 or 16 lanes per pixel; a 64-lane workgroup covers the tile of its rays
+// (8x8 pixels at one lane), so a wavefront marches a coherent ray packet.  Ray emit, box clip and the march
 // loop are fused (the reference splits them over ray_emit_kernel_impl and a
 // device-function-pointer call to VolumeShaderKernel::main,
 // src/slave/core/cuda_shading.cu:14-37 and volume_shader.cu:32-81).
