@@ -1030,9 +1030,10 @@ __device__ __forceinline__ void seg_sample_group(const VolumeArgs &a, const floa
   float w[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    // a lane past the run repeats its first sample
+    // a slot past the run repeats its last sample, so that x[0] .. x[U - 1] spans
+    // every sample read
     const int k = kk + h + G * u;
-    x[u] = sub(lattice_pos(o0, d, lf, a.step, k < kc ? k : kk, w[u]), ip);
+    x[u] = sub(lattice_pos(o0, d, lf, a.step, k < kc ? k : kc - 1, w[u]), ip);
     ok[u] = k < kc || (G > 1 && u == 0);
   }
 #pragma unroll
