@@ -649,11 +649,13 @@ struct hyd_segment_set {
   int32_t *codes = nullptr;   // [n][cells]
   float4 *pages = nullptr;    // [n][max_pages]
   // every batch together, when no two hold the same brick: cell codes over the
-  // pages of all, page descriptors [sum of pages], first voxels from `base`
+  // pages of all, page descriptors [sum of pages], first voxels from `base`, page
+  // ids in the batches
   bool together = false;
   int32_t *all_codes = nullptr;
   float4 *all_pages = nullptr;
   uint64_t *all_bases = nullptr;
+  int32_t *all_ids = nullptr;
   const void *base = nullptr;
   uint64_t span = 0;          // bytes from base to the end of the highest pool
   int32_t inner = kInnerTest;   // kInner* that every batch's pages allow
@@ -665,7 +667,7 @@ int32_t hyd_segment_set_destroy(hyd_segment_set *set) {
   if (!set) return HYD_OK;
   if (hipSetDevice(set->device) == hipSuccess) {
     for (void *p : {(void *)set->codes, (void *)set->pages, (void *)set->all_codes, (void *)set->all_pages,
-                    (void *)set->all_bases})
+                    (void *)set->all_bases, (void *)set->all_ids})
       if (p) (void)hipFree(p);
   }
   delete set;
@@ -721,6 +723,7 @@ int32_t hyd_segment_set_create(hyd_ctx *c, int32_t n_batches, const hyd_segment_
   std::vector<int32_t> all(cells, -1);
   std::vector<float4> all_pages;
   std::vector<uint64_t> bases;
+  std::vector<int32_t> ids;
   const size_t elem = fmt_bytes(set->fmt), page_elems = (size_t)set->pad * set->pad * set->pad;
   uintptr_t lo = UINTPTR_MAX, hi = 0;
   for (int i = 0; i < n_batches; ++i) {
@@ -744,6 +747,7 @@ int32_t hyd_segment_set_create(hyd_ctx *c, int32_t n_batches, const hyd_segment_
     for (int k = 0; k < b[i].n_pages; ++k) {
       all_pages.push_back(pages[(size_t)i * set->max_pages + k]);
       bases.push_back(off / elem + (uint64_t)k * page_elems);
+      ids.push_back(k);
     }
   }
   set->base = reinterpret_cast<const void *>(lo);
@@ -752,10 +756,12 @@ int32_t hyd_segment_set_create(hyd_ctx *c, int32_t n_batches, const hyd_segment_
     HYD_CHECK_HIP(hipMalloc((void **)&set->all_codes, cells * sizeof(int32_t)));
     HYD_CHECK_HIP(hipMalloc((void **)&set->all_pages, all_pages.size() * sizeof(float4)));
     HYD_CHECK_HIP(hipMalloc((void **)&set->all_bases, bases.size() * sizeof(uint64_t)));
+    HYD_CHECK_HIP(hipMalloc((void **)&set->all_ids, ids.size() * sizeof(int32_t)));
     HYD_CHECK_HIP(hipMemcpy(set->all_codes, all.data(), cells * sizeof(int32_t), hipMemcpyHostToDevice));
     HYD_CHECK_HIP(
         hipMemcpy(set->all_pages, all_pages.data(), all_pages.size() * sizeof(float4), hipMemcpyHostToDevice));
     HYD_CHECK_HIP(hipMemcpy(set->all_bases, bases.data(), bases.size() * sizeof(uint64_t), hipMemcpyHostToDevice));
+    HYD_CHECK_HIP(hipMemcpy(set->all_ids, ids.data(), ids.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     *out = set.release();
     return HYD_OK;
   }
@@ -800,6 +806,7 @@ int32_t hyd_segments_pass_set(hyd_ctx *c, const hyd_segment_set *set, const hyd_
     a.codes = set->all_codes;
     a.page = set->all_pages;
     a.page_base = set->all_bases;
+    a.page_local = set->all_ids;
     HYD_CHECK_HIP(launch_segments_set(a, set->span, set->fmt, c->stream));
     return HYD_OK;
   }

@@ -209,6 +209,7 @@ struct VolumeArgs {
   int32_t *nslots;
   int32_t max_slots;
   const uint64_t *page_base;   // segment sets: first voxel of each page, in voxels from pool
+  const int32_t *page_local;   // segment sets: each page's id in its own batch (Paging mode colours by it)
 };
 
 // The work of a frame as a number of rays of its longest chord (hyd_api.cpp).
@@ -221,8 +222,8 @@ inline float lane_rays(double pool_bytes) { return 75e3f + 36e3f * (float)std::l
 hipError_t launch_volume(const VolumeArgs &a, int fmt, bool resume, hipStream_t s);
 hipError_t launch_segments_clear(float4 *slots, size_t n, hipStream_t s);
 hipError_t launch_segments_pass(const VolumeArgs &a, int fmt, hipStream_t s);
-// A segment set's batches in one launch: codes, page descriptors and page bases
-// run over the pages of every batch, pool is the lowest of their pools and
+// A segment set's batches in one launch: codes, page descriptors, bases and local
+// ids run over the pages of every batch, pool is the lowest of their pools and
 // span_bytes the distance from it to the end of the highest.
 hipError_t launch_segments_set(const VolumeArgs &a, uint64_t span_bytes, int fmt, hipStream_t s);
 constexpr int kMaxSegBatches = 16;

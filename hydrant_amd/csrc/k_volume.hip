@@ -1097,9 +1097,10 @@ __global__ __launch_bounds__(64) void segment_kernel(VolumeArgs a) {
           if (!seg_walk_cell(a, o0, d, invr, lf, kend, cdu, P, ray, h == 0, k, ord, ip, kc, pgid)) continue;
           const float4 pgd = a.page[pgid];
           const OFF page_base = MULTI ? (OFF)a.page_base[pgid] : (OFF)pgid * pad3;
+          const int id = MULTI && a.mode == HYD_MODE_PAGING ? a.page_local[pgid] : pgid;
           seg.v = make_float4(0.f, 0.f, 0.f, 0.f);
           for (int kk = k; kk < kc; kk += LANES * U)
-            seg_sample_group<FMT, COUNT, LANES, U, OFF>(a, s_tf, o0, d, lf, ip, pgd, page_base, pgid, kk, kc, h, seg,
+            seg_sample_group<FMT, COUNT, LANES, U, OFF>(a, s_tf, o0, d, lf, ip, pgd, page_base, id, kk, kc, h, seg,
                                                         count);
           if (h == 0) a.slots[(size_t)ord * P + ray] = seg.v;
           ++ord;
