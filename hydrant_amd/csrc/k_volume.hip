@@ -368,9 +368,11 @@ __device__ __forceinline__ void group_colours(const VolumeArgs &a, const float4 
 
 // Alpha at which a sample changes the step (volume_shader.cu:71-76: v.w > 0.93
 // gives 16, else v.w > 0.85 gives 4; see march_reference for the literals).  At 16
-// only a falling alpha does, which opacities in [0, 1] rule out.
-__device__ __forceinline__ float escalation_alpha(const VolumeArgs &a, int step_size) {
-  return step_size == 4 ? 0.93f : step_size == 16 && a.monotone ? INFINITY : 0.85f;
+// with an alpha past 0.93 only a falling alpha does, which opacities in [0, 1] rule
+// out; a film may hold a step of 16 at a lower alpha (written under other
+// opacities), which the next escalation changes.
+__device__ __forceinline__ float escalation_alpha(const VolumeArgs &a, int step_size, float alpha) {
+  return step_size == 4 ? 0.93f : step_size == 16 && a.monotone && alpha >= 0.93f ? INFINITY : 0.85f;
 }
 __device__ __forceinline__ int escalated_step(float alpha, int step_size) {
   return alpha >= 0.93f ? 16 : alpha >= 0.85f ? 4 : step_size;
@@ -459,8 +461,8 @@ __device__ void march_reference_grouped(const VolumeArgs &a, const float4 *tf, M
     if (a.macro.cls) cnext = macro_class(a.macro, pgid, sub(add(q, inc), ip));
     group_colours<FMT, OFF, U>(a, tf, inner, x, ok, pgd, page_base, pgid, ub);
     int n = 0;
-    composite_group<0, U, THETA>([&](auto j) { return ub[decltype(j)::value]; }, ok, escalation_alpha(a, step_size), st,
-                                 n);
+    composite_group<0, U, THETA>([&](auto j) { return ub[decltype(j)::value]; }, ok, escalation_alpha(a, step_size, st.v.w),
+                                 st, n);
     if (COUNT) count += (unsigned)n;
     // samples 0 .. n-2 advanced by the group's step, the last by its own
     const int last_ss = escalated_step(st.v.w, step_size);
@@ -603,7 +605,7 @@ __device__ void march_reference_coop(const VolumeArgs &a, const float4 *tf, Marc
           return make_float4(group_bcast<G, j % G>(uk.x), group_bcast<G, j % G>(uk.y), group_bcast<G, j % G>(uk.z),
                              group_bcast<G, j % G>(uk.w));
         },
-        ok, escalation_alpha(a, step_size), st, n);
+        ok, escalation_alpha(a, step_size, st.v.w), st, n);
     if (COUNT && h == 0) count += (unsigned)n;
     const int last_ss = escalated_step(st.v.w, step_size);
     cls = n == N && last_ss == step_size ? cnext : -1;
