@@ -648,8 +648,8 @@ __device__ void march_lattice(const VolumeArgs &a, const float4 *tf, MarchState 
   int k = st.step_size;
   const int kend = (int)ceilf(lf);
   const float cdu = 1.f / comp_max(abs3(d));
-  // v.w > ert as v.w >= the next float
-  const float stop = a.ert > 0.f ? __uint_as_float(__float_as_uint(a.ert) + 1u) : INFINITY;
+  // v.w > ert as v.w >= the next float; NaN, which no alpha reaches, without termination
+  const float stop = a.ert > 0.f ? __uint_as_float(__float_as_uint(a.ert) + 1u) : NAN;
   const OFF pad3 = (OFF)a.pad * (OFF)a.pad * (OFF)a.pad;
   int cpg = -1;               // page of the cached descriptor
   float4 pgd = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1055,7 +1055,7 @@ __device__ __forceinline__ void seg_sample_group(const VolumeArgs &a, const floa
         else
           return uk;
       },
-      okn, INFINITY, seg, n);
+      okn, NAN, seg, n);   // no alpha stops a segment
   if (COUNT && h == 0) count += (unsigned)n;
 }
 
