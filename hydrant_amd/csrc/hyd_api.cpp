@@ -101,7 +101,10 @@ int32_t inner_mapping(float k_min, float lo, float hi, int32_t pad) {
   const bool all = k_min >= 0.f && float(pad) * lo - 0.5f >= 1e-3f && float(pad) * hi - 0.5f <= float(pad) - 1.001f;
   return all ? kInnerAlways : kInnerTest;
 }
-int32_t pages_inner(const Ctx *c) { return inner_mapping(c->page_k_min, c->page_lo, c->page_hi, c->pool.pad); }
+int32_t pages_inner(const Ctx *c) {
+  if (capturing(c)) return kInnerTest;
+  return inner_mapping(c->page_k_min, c->page_lo, c->page_hi, c->pool.pad);
+}
 
 int32_t check_volume_state(const Ctx *c) {
   HYD_REQUIRE(c->pool.data, HYD_ERR_STATE, "no brick pool: call hyd_upload_pool first");
@@ -228,6 +231,13 @@ void srgb8_thresholds(float t[256]) {
     }
     std::memcpy(&t[k], &hi, 4);
   }
+}
+
+bool capturing(const Ctx *c) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(c->stream, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();   // the null stream during a capture elsewhere
+  return true;
 }
 
 int32_t activate(Ctx *c) {

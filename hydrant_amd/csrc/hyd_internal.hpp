@@ -307,6 +307,11 @@ struct IsoArgs {
 hipError_t launch_iso(const IsoArgs &a, int fmt, hipStream_t s);
 
 int32_t activate(Ctx *c);
+// Whether the context's stream is being captured.  A replay may meet another page
+// table (hyd_set_page_table rewrites it in place), so a captured march takes
+// nothing that the host derived from the table's mappings: its samples are
+// tested per group, and no macrocells are passed over.
+bool capturing(const Ctx *c);
 // After pool pages [first, first + n) were overwritten in place: updates the
 // batched renderer's oriented copies of those pages if they are current.
 int32_t refresh_oriented_pages(Ctx *c, int32_t first, int32_t n);

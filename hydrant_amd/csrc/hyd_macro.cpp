@@ -114,9 +114,7 @@ int32_t macro_batch(Ctx *c, const uint8_t **cls) {
   if (!c->tf_finite || !(c->tf_rgb_max <= 1e15f) || !(c->tf_alpha_min >= 0.f)) return HYD_OK;
   const size_t n = (size_t)c->pool.n_pages, cells = n * page_cells(c);
   if (c->bcls_gen != c->batch_state_gen) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    HYD_CHECK_HIP(hipStreamIsCapturing(c->stream, &cap));
-    if (cap != hipStreamCaptureStatusNone) return HYD_OK;   // made by the next launch outside it
+    if (capturing(c)) return HYD_OK;   // made by the next launch outside it
     c->bcls_gen = ~0ull;
     if (cells > 0xffffffffull || !reserve(c, cells)) return HYD_OK;   // 32-bit class offsets
     if (c->bcls_cap < cells || c->bscale_cap < n) {
@@ -158,7 +156,7 @@ int32_t macro_batch(Ctx *c, const uint8_t **cls) {
 namespace {
 // The grid for marches within [bmin, bmax]; false when it does not apply.
 bool grid_of(const Ctx *c, f3 bmin, f3 bmax, MacroGrid &g) {
-  if (!c->pool.owned || c->mm_gen != c->pool_gen) return false;
+  if (!c->pool.owned || c->mm_gen != c->pool_gen || capturing(c)) return false;
   // every page has the same mapping, one b on each axis, inside the page
   const float k = c->page_k_min, lo = c->page_lo;
   if (!(k > 0.f && c->page_k_max == k && lo >= 0.f && c->page_hi == k + lo && k + lo <= 1.000001f)) return false;
