@@ -1,7 +1,6 @@
 // C ABI of the batched renderer: multi-volume set, batch plans, HIP-graph
 // capture/replay and the launch-shape autotuner.
 #include <algorithm>
-#include <cmath>
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
@@ -268,7 +267,7 @@ int32_t hyd_set_volumes(hyd_ctx *c, int32_t n, const hyd_volume_desc *vols) {
   HYD_REQUIRE(n >= 1 && vols, HYD_ERR_ARG, "empty volume set");
   std::vector<BatchVolDev> dv(n);
   std::vector<int32_t> cells;
-  std::vector<float> scale;   // of each page a volume names (NaN: two volumes' scales differ)
+  std::vector<std::pair<int32_t, float>> pages;
   int pad = -1, max_page = -1;
   for (int v = 0; v < n; ++v) {
     const hyd_volume_desc &d = vols[v];
@@ -295,10 +294,7 @@ int32_t hyd_set_volumes(hyd_ctx *c, int32_t n, const hyd_volume_desc *vols) {
       if (cd == 0 && c->pool.data)
         HYD_REQUIRE(pg < c->pool.n_pages, HYD_ERR_RANGE, "volume %d cell %zu: page %d beyond the pool", v, i, pg);
       if (cd == 0) max_page = std::max(max_page, pg);
-      if (cd == 0 && pg >= 0) {
-        if ((size_t)pg >= scale.size()) scale.resize((size_t)pg + 1, 0.f);
-        scale[pg] = scale[pg] == 0.f || scale[pg] == d.value_scale ? d.value_scale : NAN;
-      }
+      if (cd == 0 && pg >= 0) pages.emplace_back(pg, d.value_scale);
       cells.push_back(cd > 0 ? -1 - cd : pg);
     }
   }
@@ -317,7 +313,7 @@ int32_t hyd_set_volumes(hyd_ctx *c, int32_t n, const hyd_volume_desc *vols) {
   c->n_vols = n;
   c->vol_pad = pad;
   c->vol_max_page = max_page;
-  c->page_scale = std::move(scale);
+  c->vol_pages = std::move(pages);
   c->vol_bmax.resize(n);
   for (int v = 0; v < n; ++v) std::copy(vols[v].bbox_max, vols[v].bbox_max + 3, c->vol_bmax[v].begin());
   return HYD_OK;

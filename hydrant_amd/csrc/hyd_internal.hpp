@@ -9,6 +9,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/hydrant_hip.h"
@@ -121,7 +122,7 @@ struct Ctx {
   // classes for the batched renderer: each page under the value scale of its
   // volume (NaN: none, or two that differ), made at the first batched launch
   // after a change of pool, transfer function or volume set
-  std::vector<float> page_scale;
+  std::vector<std::pair<int32_t, float>> vol_pages;   // {page, value scale} of every resident cell
   std::vector<std::array<float, 3>> vol_bmax;   // extent of each volume of the set
   float *own_bscale = nullptr;
   uint8_t *own_bflags = nullptr, *own_bcls = nullptr;

@@ -137,8 +137,9 @@ int32_t macro_batch(Ctx *c, const uint8_t **cls) {
       c->mm_gen = c->pool_gen;
       c->mcls_valid = false;
     }
-    std::vector<float> scale(c->page_scale);
-    scale.resize(n, NAN);
+    std::vector<float> scale(n, 0.f);   // the set's pages lie in the pool (fill_args)
+    for (const auto &[pg, sc] : c->vol_pages) scale[pg] = scale[pg] == 0.f || scale[pg] == sc ? sc : NAN;
+    for (float &sc : scale) sc = sc == 0.f ? NAN : sc;
     unsigned long long count = 0;
     HYD_CHECK_HIP(hipMemcpyAsync(c->own_bscale, scale.data(), n * sizeof(float), hipMemcpyHostToDevice, c->stream));
     HYD_CHECK_HIP(hipMemcpyAsync(c->own_mcount, &count, sizeof(count), hipMemcpyHostToDevice, c->stream));
