@@ -1,6 +1,8 @@
 // Macrocell ranges and classes (hyd_macro.hpp).
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
+
 #include "hyd_macro.hpp"
 
 namespace hyd {
@@ -143,19 +145,24 @@ __global__ __launch_bounds__(256) void macro_class_kernel(const uint8_t *flags, 
 }  // namespace
 
 hipError_t launch_macro_minmax(int fmt, const void *pool, int pad, int first, int n, float2 *mm, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
-  const dim3 grid(n, macro_edge(pad));
-  switch (fmt) {
-    case HYD_FMT_U8:
-      hipLaunchKernelGGL(macro_minmax_kernel<HYD_FMT_U8>, grid, dim3(256), 0, s, pool, pad, first, mm);
-      break;
-    case HYD_FMT_F16:
-      hipLaunchKernelGGL(macro_minmax_kernel<HYD_FMT_F16>, grid, dim3(256), 0, s, pool, pad, first, mm);
-      break;
-    default:
-      hipLaunchKernelGGL(macro_minmax_kernel<HYD_FMT_F32>, grid, dim3(256), 0, s, pool, pad, first, mm);
+  // a launch holds fewer than 2^32 threads on an axis: 256 a page
+  constexpr int kPages = 1 << 22;
+  for (; n > 0; first += kPages, n -= kPages) {
+    const dim3 grid(std::min(n, kPages), macro_edge(pad));
+    switch (fmt) {
+      case HYD_FMT_U8:
+        hipLaunchKernelGGL(macro_minmax_kernel<HYD_FMT_U8>, grid, dim3(256), 0, s, pool, pad, first, mm);
+        break;
+      case HYD_FMT_F16:
+        hipLaunchKernelGGL(macro_minmax_kernel<HYD_FMT_F16>, grid, dim3(256), 0, s, pool, pad, first, mm);
+        break;
+      default:
+        hipLaunchKernelGGL(macro_minmax_kernel<HYD_FMT_F32>, grid, dim3(256), 0, s, pool, pad, first, mm);
+    }
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
   }
-  return hipGetLastError();
+  return hipSuccess;
 }
 
 hipError_t launch_macro_classes(const float2 *mm, int pad, int first, int n, const float *tf, int tf_n, float scale,
