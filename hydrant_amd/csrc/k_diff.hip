@@ -915,7 +915,7 @@ template <int G> void launch_forward_lanes(const DiffArgs &a, hipStream_t s) {
 hipError_t launch_diff_forward(const DiffArgs &a, hipStream_t s) {
   const long long rays = (long long)a.n_views * a.W * a.H;
   if (rays <= 24576) launch_forward_lanes<16>(a, s);
-  else if (rays <= 131072) launch_forward_lanes<4>(a, s);
+  else if (rays <= 131072 && (a.H + 1) / 2 <= 65535) launch_forward_lanes<4>(a, s);   // a launch's y axis
   else launch_forward_lanes<1>(a, s);
   return hipGetLastError();
 }

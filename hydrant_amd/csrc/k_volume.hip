@@ -831,6 +831,9 @@ template <int L> constexpr int coop_group() { return L == kManyLanes ? 16 : 8; }
 template <int L> constexpr int tile_w() { return L == kManyLanes ? 4 : kTile; }
 template <int L> constexpr int tile_h() { return 64 / L / tile_w<L>(); }
 constexpr long long kManyLaneRays = 24576;
+// A tall frame's workgroups of L lanes a ray fit a launch's y axis (16 lanes always
+// do, at kManyLaneRays).
+template <int L> bool rows_fit(int H) { return (H + tile_h<L>() - 1) / tile_h<L>() <= 65535; }
 
 // Render modes of volume_kernel: emit into an RGBA image only, emit into a film
 // (and optionally RGBA), or resume a film.
@@ -1195,7 +1198,8 @@ template <int FMT, int MODE, bool BIG>
 void launch_mode(const VolumeArgs &a, hipStream_t s) {
   const long long rays = (long long)a.W * a.H;
   if (rays <= kManyLaneRays) launch_lanes<FMT, MODE, BIG, kManyLanes>(a, s);
-  else if (a.full_rays <= lane_rays((double)a.pool_elems * sizeof(typename RawVox<FMT>::T))) launch_lanes<FMT, MODE, BIG, kLanes>(a, s);
+  else if (rows_fit<kLanes>(a.H) && a.full_rays <= lane_rays((double)a.pool_elems * sizeof(typename RawVox<FMT>::T)))
+    launch_lanes<FMT, MODE, BIG, kLanes>(a, s);
   else launch_lanes<FMT, MODE, BIG, 1>(a, s);
 }
 
@@ -1237,7 +1241,7 @@ template <int FMT, bool MULTI>
 hipError_t launch_segments(const VolumeArgs &a, uint64_t bytes, hipStream_t s) {
   const bool big = bytes > (1ull << 32) || force_offsets64();
   if ((long long)a.W * a.H <= kManyLaneRays) launch_segments_lanes<FMT, MULTI, kManyLanes>(a, big, s);
-  else if (a.full_rays <= 2.f * lane_rays((double)bytes)) launch_segments_lanes<FMT, MULTI, kLanes>(a, big, s);
+  else if (rows_fit<kLanes>(a.H) && a.full_rays <= 2.f * lane_rays((double)bytes)) launch_segments_lanes<FMT, MULTI, kLanes>(a, big, s);
   else launch_segments_lanes<FMT, MULTI, 1>(a, big, s);
   return hipGetLastError();
 }
