@@ -141,7 +141,10 @@ int32_t hyd_diff_backward(hyd_ctx *c, const hyd_diff_params *p, const hyd_view *
   const size_t ds_floats = diff_ds_floats(n_views, width, height, a.K);
   const size_t rays_off = (ds_floats * sizeof(float) + 255) & ~(size_t)255;
   a.view_groups = diff_view_groups(a.nx, a.ny, a.nz, n_views);
-  const size_t blocks_floats = (size_t)a.view_groups * diff_bricks(a.nx, a.ny, a.nz) * kDiffBlock;
+  const size_t nb = diff_bricks(a.nx, a.ny, a.nz);
+  const bool split = diff_ray_splits(a.view_groups, n_views) > 1;   // int64 blocks, and their exponents
+  const size_t block_entries = (size_t)a.view_groups * nb * kDiffBlock;
+  const size_t blocks_floats = split ? 2 * block_entries + (size_t)n_views * nb : block_entries;
   const size_t gtf_off = (rays_off + sizeof(float) * (8 * (size_t)n_rays + blocks_floats + (size_t)n_rays +
                                                      kDiffBoundParts) + 255) & ~(size_t)255;
   const size_t need = gtf_off + sizeof(unsigned long long) * 4 * 256 + 64;
@@ -156,6 +159,7 @@ int32_t hyd_diff_backward(hyd_ctx *c, const hyd_diff_params *p, const hyd_view *
   a.ds = reinterpret_cast<float *>(base);
   a.rays = reinterpret_cast<float4 *>(base + rays_off);
   a.blocks = reinterpret_cast<float *>(a.rays + 2 * n_rays);
+  a.block_exp = split ? reinterpret_cast<int32_t *>(a.blocks + 2 * block_entries) : nullptr;
   a.dsmax = a.blocks + blocks_floats;
   a.bound = a.dsmax + n_rays;
   a.gtf_acc = reinterpret_cast<unsigned long long *>(base + gtf_off);

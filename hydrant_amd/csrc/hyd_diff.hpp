@@ -36,7 +36,9 @@ struct DiffArgs {
   float *ds;                   // [view][y][x][K] dL/ds per sample
   float *dsmax;                // [view][y][x] max |dL/ds| of the ray (0: nothing to scatter)
   float4 *rays;                // [view][y][x][2] setup of active rays: (dx, dy, dz, tnear), (dt, 0, 0, 0)
-  float *blocks;               // [view group][brick][10^3] voxel-gradient blocks (brick + one-voxel halo)
+  float *blocks;               // [view group][brick][10^3] voxel-gradient blocks (brick + one-voxel halo); int64
+                               // sums before their rounding when a view's rays are split (diff_ray_splits > 1)
+  int32_t *block_exp;          // [view][brick] then: the power of two of the sums
   int32_t view_groups;         // scatter workgroups per brick: contiguous groups of views, or (a multiple of
                                // n_views) equal shares of each view's rays
   float *bound;                // [kDiffBoundParts] partial bounds of one sample's TF-gradient term
@@ -58,7 +60,9 @@ inline size_t diff_bricks(int32_t nx, int32_t ny, int32_t nz) {
 // at most one group per view; when that leaves fewer than kDiffScatterMin, each
 // view's rays are split over up to kDiffRaySplits groups (a workgroup's rounds
 // are one dependent chain: six views at 64^2 of a 48^3 volume, 1,296 workgroups,
-// took 607 us; the whole step 1350 us, 1005 with eight shares).
+// took 607 us; the whole step 1350 us, 1005 with eight shares).  A view's shares
+// have one scale and are added as the integers they are, so a gradient does not
+// depend on the split.
 constexpr size_t kDiffScatterWgs = 32768, kDiffScatterMin = 8192, kDiffRaySplits = 8;
 
 inline int32_t diff_view_groups(int32_t nx, int32_t ny, int32_t nz, int32_t n_views) {
@@ -67,6 +71,11 @@ inline int32_t diff_view_groups(int32_t nx, int32_t ny, int32_t nz, int32_t n_vi
   if (g < v) return (int32_t)g;
   const size_t splits = std::min(kDiffRaySplits, std::max<size_t>(1, kDiffScatterMin / (nb * v)));
   return (int32_t)(v * splits);
+}
+
+// Shares of a view's rays among view_groups groups (1: whole views).
+__host__ __device__ inline int32_t diff_ray_splits(int32_t view_groups, int32_t n_views) {
+  return view_groups > n_views ? view_groups / n_views : 1;
 }
 
 // floats of the dL/ds buffer ([view][y][x][k])

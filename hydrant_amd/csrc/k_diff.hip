@@ -704,7 +704,7 @@ __global__ __launch_bounds__(64) void diff_scatter_kernel(DiffArgs a) {
   const int bi = (bz * nby + by) * nbx + bx;
   // views of this workgroup: a contiguous share of the launch's views
   // (or one view, of whose rays it takes a share)
-  const int splits = max(1, a.view_groups / a.n_views), part = grp % splits;
+  const int splits = diff_ray_splits(a.view_groups, a.n_views), part = grp % splits;
   const int v_begin = (int)((long long)a.n_views * (grp / splits) / (a.view_groups / splits));
   const int v_end = (int)((long long)a.n_views * (grp / splits + 1) / (a.view_groups / splits));
   BrickBox bb;
@@ -712,7 +712,7 @@ __global__ __launch_bounds__(64) void diff_scatter_kernel(DiffArgs a) {
   bb.cx0 = bb.X0 == 0 ? -1 : bb.X0; bb.cy0 = bb.Y0 == 0 ? -1 : bb.Y0; bb.cz0 = bb.Z0 == 0 ? -1 : bb.Z0;
   bb.cx1 = min(bb.X0 + kBrick - 1, a.nx - 1); bb.cy1 = min(bb.Y0 + kBrick - 1, a.ny - 1);
   bb.cz1 = min(bb.Z0 + kBrick - 1, a.nz - 1);
-  float *blk = a.blocks + ((size_t)grp * nbx * nby * nbz + bi) * kBlk3;
+  const size_t blk = ((size_t)grp * nbx * nby * nbz + bi) * kBlk3;   // this workgroup's block
   for (int i = lane; i < kBlk3; i += 64) s_acc[i] = 0ull;
   float acc[kBlkPerLane];   // the block's FP32 sums over this group's views; entry lane + 64 i
 #pragma unroll
@@ -826,6 +826,10 @@ __global__ __launch_bounds__(64) void diff_scatter_kernel(DiffArgs a) {
       scatter_list(a, v, L, n, total, scale, s_acc, lane, bb);
     }
     wave_sync();
+    if (splits > 1) {   // the one view's share stays an integer: the combine adds the shares
+      if (part == 0 && lane == 0) a.block_exp[(size_t)view * nbx * nby * nbz + bi] = e;
+      break;
+    }
     const float unscale = ldexpf(1.f, -e);
 #pragma unroll
     for (int i = 0; i < kBlkPerLane; ++i) {
@@ -840,10 +844,15 @@ __global__ __launch_bounds__(64) void diff_scatter_kernel(DiffArgs a) {
     }
     wave_sync();
   }
+  if (splits > 1) {
+    unsigned long long *sums = reinterpret_cast<unsigned long long *>(a.blocks) + blk;
+    for (int i = lane; i < kBlk3; i += 64) sums[i] = s_acc[i];
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < kBlkPerLane; ++i) {
     const int idx = lane + 64 * i;
-    if (idx < kBlk3) blk[idx] = acc[i];
+    if (idx < kBlk3) a.blocks[blk + idx] = acc[i];
   }
 }
 
@@ -878,6 +887,7 @@ __global__ __launch_bounds__(256) void diff_combine_kernel(DiffArgs a) {
   const size_t nvox = (size_t)a.nx * a.ny * a.nz;
   const int nbx = (a.nx + kBrick - 1) / kBrick, nby = (a.ny + kBrick - 1) / kBrick;
   const size_t nb = (size_t)nbx * nby * ((a.nz + kBrick - 1) / kBrick);
+  const int splits = diff_ray_splits(a.view_groups, a.n_views);
   for (size_t vi = (size_t)blockIdx.x * 256 + threadIdx.x; vi < nvox; vi += (size_t)gridDim.x * 256) {
     const int X = (int)(vi % a.nx), Y = (int)((vi / a.nx) % a.ny), Z = (int)(vi / ((size_t)a.nx * a.ny));
     const int bx = X / kBrick, by = Y / kBrick, bz = Z / kBrick;
@@ -885,12 +895,21 @@ __global__ __launch_bounds__(256) void diff_combine_kernel(DiffArgs a) {
     const int cx = axis_sources(X, a.nx, dbx, sx), cy = axis_sources(Y, a.ny, dby, sy),
               cz = axis_sources(Z, a.nz, dbz, sz);
     float g = 0.f;
-    for (int grp = 0; grp < a.view_groups; ++grp) {
+    for (int grp = 0; grp < a.view_groups; grp += splits) {
       for (int k = 0; k < cz; ++k)
         for (int j = 0; j < cy; ++j)
           for (int i = 0; i < cx; ++i) {
-            const size_t b = grp * nb + ((size_t)(bz + dbz[k]) * nby + (by + dby[j])) * nbx + (bx + dbx[i]);
-            g += a.blocks[b * kBlk3 + (sz[k] * kBlk + sy[j]) * kBlk + sx[i]];
+            const size_t bi = ((size_t)(bz + dbz[k]) * nby + (by + dby[j])) * nbx + (bx + dbx[i]);
+            const int slot = (sz[k] * kBlk + sy[j]) * kBlk + sx[i];
+            if (splits == 1) {
+              g += a.blocks[(grp * nb + bi) * kBlk3 + slot];
+              continue;
+            }
+            // the shares of one view: integers of one scale, rounded once
+            long long sum = 0;
+            for (int q = 0; q < splits; ++q)
+              sum += reinterpret_cast<const long long *>(a.blocks)[((grp + q) * nb + bi) * kBlk3 + slot];
+            if (sum != 0) g += (float)sum * ldexpf(1.f, -a.block_exp[(grp / splits) * nb + bi]);
           }
     }
     a.grad_vol[vi] = g;
