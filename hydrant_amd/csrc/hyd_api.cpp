@@ -353,12 +353,15 @@ int32_t hyd_upload_pool(hyd_ctx *c, int32_t fmt, int32_t pad_edge, int32_t n_pag
   HYD_REQUIRE(pad_edge >= 2 && pad_edge <= 1024, HYD_ERR_ARG, "pad_edge %d out of range [2, 1024]", pad_edge);
   HYD_REQUIRE(n_pages > 0 && host, HYD_ERR_ARG, "empty pool");
   const size_t bytes = (size_t)n_pages * pad_edge * pad_edge * pad_edge * fmt_bytes(fmt);
-  st = upload(c->own_pool, host, bytes, c->stream);
-  if (st) return st;
+  free_dev(c->own_pool);
+  HYD_CHECK_HIP(hipMalloc((void **)&c->own_pool, bytes));
+  HYD_CHECK_HIP(hipMemcpyAsync(c->own_pool, host, bytes, hipMemcpyHostToDevice, c->stream));
   c->pool = Pool{c->own_pool, fmt, pad_edge, n_pages, true};
   ++c->pool_gen;
   ++c->batch_state_gen;
-  return macro_pool_uploaded(c);
+  if ((st = macro_pool_uploaded(c))) return st;
+  HYD_CHECK_HIP(hipStreamSynchronize(c->stream));
+  return HYD_OK;
 }
 
 int32_t hyd_bind_pool_device(hyd_ctx *c, int32_t fmt, int32_t pad_edge, int32_t n_pages, const void *pool_dev) {

@@ -72,9 +72,7 @@ int32_t macro_pool_uploaded(Ctx *c) {
   HYD_CHECK_HIP(launch_macro_minmax(c->pool.fmt, c->pool.data, c->pool.pad, 0, c->pool.n_pages, c->own_mm,
                                     c->stream));
   c->mm_gen = c->pool_gen;
-  if (c->tf) return macro_tf_set(c);
-  HYD_CHECK_HIP(hipStreamSynchronize(c->stream));
-  return HYD_OK;
+  return c->tf ? macro_tf_set(c) : HYD_OK;   // the caller waits for the stream
 }
 
 int32_t macro_tf_set(Ctx *c) {

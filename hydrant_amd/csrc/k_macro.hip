@@ -25,47 +25,63 @@ template <> struct MVox<HYD_FMT_F32> {
   static __device__ __forceinline__ float get(T v) { return v; }
 };
 
-// One workgroup per (page, z row of macrocells): each thread takes the range of
-// one x column over a macrocell row's 9 x 9 (y, z) voxels, so reads run along
-// x; the columns are then reduced by 9 in LDS.  Bound by the voxel reads (1.27
-// of the pool, the overlaps from the L2); runs once per pool upload.
-template <int FMT>
-__global__ __launch_bounds__(256) void macro_minmax_kernel(const void *pool, int pad, int first, float2 *mm) {
-  using V = MVox<FMT>;
+// One workgroup per (page, z row of macrocells, `rows` of their y rows): each
+// thread takes the ranges of V neighbouring x columns over a macrocell row's 9 x 9
+// (y, z) voxels, nine loads of V voxels in flight; the columns are then reduced by
+// 9 in LDS.  Bound by the voxel reads (1.27 of the pool, the overlaps from the
+// L2); runs once per pool upload, behind the copy.  With single-voxel loads and
+// every y row in one workgroup (32 of them for one 256^3 page) an upload of that
+// page in FP32 took 3.77 ms and one of 4096 u8 pages of 66^3 44.3 ms; 2.38 and
+// 39.5 ms so, and 2.58 and 41.5 before there were ranges.
+template <int FMT, int V>
+__global__ __launch_bounds__(256) void macro_minmax_kernel(const void *pool, int pad, int first, int rows, float2 *mm) {
+  using X = MVox<FMT>;
   __shared__ float2 s_col[kColumns];
-  const int nm = (pad + kMacro - 1) / kMacro;
+  const int nm = (pad + kMacro - 1) / kMacro, nx = (pad + V - 1) / V;
   const size_t page = (size_t)first + blockIdx.x;
-  const typename V::T *pg = static_cast<const typename V::T *>(pool) + page * pad * pad * pad;
+  const typename X::T *pg = static_cast<const typename X::T *>(pool) + page * pad * pad * pad;
   float2 *out = mm + page * nm * nm * nm;
   const int mz = blockIdx.y, z0 = mz * kMacro, z1 = min(z0 + kMacro, pad - 1);
-  const int rows = kColumns / pad;
-  for (int my0 = 0; my0 < nm; my0 += rows) {
-    const int nr = min(rows, nm - my0);
-    for (int i = threadIdx.x; i < nr * pad; i += 256) {
-      const int y0 = (my0 + i / pad) * kMacro, y1 = min(y0 + kMacro, pad - 1), x = i % pad;
-      float lo = INFINITY, hi = -INFINITY;
-      bool bad = false;
-      for (int z = z0; z <= z1; ++z)
-        for (int y = y0; y <= y1; ++y) {
-          const float v = V::get(pg[((size_t)z * pad + y) * pad + x]);
-          bad = bad || !(fabsf(v) <= 1e30f);
-          lo = fminf(lo, v);
-          hi = fmaxf(hi, v);
+  const int my0 = blockIdx.z * rows, nr = min(rows, nm - my0);
+  for (int i = threadIdx.x; i < nr * nx; i += 256) {
+    const int r = i / nx, x = min((i % nx) * V, pad - V), y0 = (my0 + r) * kMacro;
+    float lo[V], hi[V];
+    bool bad[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      lo[v] = INFINITY;
+      hi[v] = -INFINITY;
+      bad[v] = false;
+    }
+    for (int z = z0; z <= z1; ++z) {
+      typename X::T t[kMacro + 1][V];
+#pragma unroll
+      for (int y = 0; y <= kMacro; ++y)   // the last rows of a page repeat
+        __builtin_memcpy(t[y], pg + ((size_t)z * pad + min(y0 + y, pad - 1)) * pad + x, sizeof(t[y]));
+#pragma unroll
+      for (int y = 0; y <= kMacro; ++y)
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          const float f = X::get(t[y][v]);
+          bad[v] = bad[v] || !(fabsf(f) <= 1e30f);
+          lo[v] = fminf(lo[v], f);
+          hi[v] = fmaxf(hi[v], f);
         }
-      s_col[i] = bad ? make_float2(-INFINITY, INFINITY) : make_float2(lo, hi);
     }
-    __syncthreads();
-    for (int i = threadIdx.x; i < nr * nm; i += 256) {
-      const int r = i / nm, mx = i % nm, x0 = mx * kMacro, x1 = min(x0 + kMacro, pad - 1);
-      float lo = INFINITY, hi = -INFINITY;
-      for (int x = x0; x <= x1; ++x) {
-        lo = fminf(lo, s_col[r * pad + x].x);
-        hi = fmaxf(hi, s_col[r * pad + x].y);
-      }
-      const bool bad = lo == -INFINITY || hi == INFINITY;
-      out[((size_t)mz * nm + my0 + r) * nm + mx] = bad ? make_float2(NAN, NAN) : make_float2(lo, hi);
+#pragma unroll
+    for (int v = 0; v < V; ++v)
+      s_col[r * pad + x + v] = bad[v] ? make_float2(-INFINITY, INFINITY) : make_float2(lo[v], hi[v]);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < nr * nm; i += 256) {
+    const int r = i / nm, mx = i % nm, x0 = mx * kMacro, x1 = min(x0 + kMacro, pad - 1);
+    float lo = INFINITY, hi = -INFINITY;
+    for (int x = x0; x <= x1; ++x) {
+      lo = fminf(lo, s_col[r * pad + x].x);
+      hi = fmaxf(hi, s_col[r * pad + x].y);
     }
-    __syncthreads();
+    const bool bad = lo == -INFINITY || hi == INFINITY;
+    out[((size_t)mz * nm + my0 + r) * nm + mx] = bad ? make_float2(NAN, NAN) : make_float2(lo, hi);
   }
 }
 
@@ -144,22 +160,28 @@ __global__ __launch_bounds__(256) void macro_class_kernel(const uint8_t *flags, 
 
 }  // namespace
 
+namespace {
+template <int FMT>
+hipError_t minmax_pages(const void *pool, int pad, int first, int n, int rows, float2 *mm, hipStream_t s) {
+  const int nm = macro_edge(pad);
+  const dim3 grid(n, nm, (nm + rows - 1) / rows), block(256);
+  if (pad >= 4) hipLaunchKernelGGL((macro_minmax_kernel<FMT, 4>), grid, block, 0, s, pool, pad, first, rows, mm);
+  else hipLaunchKernelGGL((macro_minmax_kernel<FMT, 1>), grid, block, 0, s, pool, pad, first, rows, mm);
+  return hipGetLastError();
+}
+}  // namespace
+
 hipError_t launch_macro_minmax(int fmt, const void *pool, int pad, int first, int n, float2 *mm, hipStream_t s) {
   // a launch holds fewer than 2^32 threads on an axis: 256 a page
   constexpr int kPages = 1 << 22;
+  // as many y rows a workgroup as its LDS holds, or fewer while that leaves the chip idle
+  const int nm = macro_edge(pad), most = std::min(nm, kColumns / pad);
+  const int rows = (int64_t)n * nm >= 4096 ? most : std::min(most, std::max(1, 256 / pad));
   for (; n > 0; first += kPages, n -= kPages) {
-    const dim3 grid(std::min(n, kPages), macro_edge(pad));
-    switch (fmt) {
-      case HYD_FMT_U8:
-        hipLaunchKernelGGL(macro_minmax_kernel<HYD_FMT_U8>, grid, dim3(256), 0, s, pool, pad, first, mm);
-        break;
-      case HYD_FMT_F16:
-        hipLaunchKernelGGL(macro_minmax_kernel<HYD_FMT_F16>, grid, dim3(256), 0, s, pool, pad, first, mm);
-        break;
-      default:
-        hipLaunchKernelGGL(macro_minmax_kernel<HYD_FMT_F32>, grid, dim3(256), 0, s, pool, pad, first, mm);
-    }
-    const hipError_t e = hipGetLastError();
+    const int k = std::min(n, kPages);
+    const hipError_t e = fmt == HYD_FMT_U8    ? minmax_pages<HYD_FMT_U8>(pool, pad, first, k, rows, mm, s)
+                         : fmt == HYD_FMT_F16 ? minmax_pages<HYD_FMT_F16>(pool, pad, first, k, rows, mm, s)
+                                              : minmax_pages<HYD_FMT_F32>(pool, pad, first, k, rows, mm, s);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

@@ -41,3 +41,35 @@ def test_pool_of_16_million_pages():
     ctx.close()
     assert images[0][1] == images[1][1] > 0
     assert torch.equal(images[0][0], images[1][0]) and bool((images[0][0] > 0).any())
+
+
+@pytest.mark.parametrize("fmt", [L.FMT_U8, L.FMT_F16, L.FMT_F32])
+@pytest.mark.parametrize("n", [2, 3, 4, 5, 9, 17, 67, 131, 257])
+def test_ranges_at_odd_page_edges(gpu_ctx, fmt, n):
+    """One page of every kind of edge (below and above the four-voxel loads and the macrocell's
+    eight), with single contributing voxels that a lost column or row would drop."""
+    import torch
+
+    rng = np.random.default_rng(n)
+    vol = np.zeros((n, n, n), np.uint8)
+    for _ in range(12):   # faces and corners among them
+        vol[tuple(int(rng.choice([0, n - 1, int(rng.integers(0, n))])) for _ in range(3))] = 255
+    if fmt != L.FMT_U8:
+        vol = vol.astype(np.float32) / np.float32(255)
+        vol = vol.astype(np.float16).view(np.uint16) if fmt == L.FMT_F16 else vol
+    b = D.single_brick(vol, fmt)
+    tf = np.array([[0, 0, 0, 0]] * 2 + [[1, 0.5, 0.2, 0.4]] * 6, np.float32)
+    geom = D.geometry((n,) * 3, n, 0.5)
+    p = hip.volume_params((0.0, 0.0, 0.0), geom.f_dim, geom.step, geom.du, density=0.5)
+    t = torch.from_numpy(b.pool.view(np.int16) if b.pool.dtype == np.uint16 else b.pool).cuda()
+    for arm, size in (((33.0, 21.0, 2.2), (61, 43)), ((200.0, -50.0, 1.2), (163, 157)), ((0.0, 0.0, 2.0), (641, 621))):
+        view = hip.make_view(hip.orbit_camera(arm), geom.center, geom.f_dim)
+        images = []
+        for owned in (True, False):
+            gpu_ctx.load(b, tf)
+            if not owned:
+                gpu_ctx.bind_pool_device(b.fmt, b.pad, b.n_pages, t.data_ptr())
+            out = gpu_ctx.render_volume(p, view, *size, film=False, count=True)
+            images.append((out["rgba"].clone(), int(out["samples"].item())))
+        assert images[0][1] == images[1][1] > 0
+        assert torch.equal(images[0][0], images[1][0])
