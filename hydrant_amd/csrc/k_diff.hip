@@ -688,6 +688,9 @@ __device__ __forceinline__ void wave_sync() {
 // the largest |dL/ds| of the rays reaching the brick's box, the view's terms
 // in the int64 block, then the block folded into FP32 sums held in registers
 // (fixed order over the views: deterministic) and cleared.
+// SPLIT: a view's rays are shared among workgroups (diff_ray_splits), whose sums stay
+// integers for the combine to add (a branch at run time cost unsplit launches 2%).
+template <bool SPLIT>
 __global__ __launch_bounds__(64) void diff_scatter_kernel(DiffArgs a) {
   __shared__ unsigned long long s_acc[kBlk3];
   __shared__ ScatterList L;
@@ -704,7 +707,7 @@ __global__ __launch_bounds__(64) void diff_scatter_kernel(DiffArgs a) {
   const int bi = (bz * nby + by) * nbx + bx;
   // views of this workgroup: a contiguous share of the launch's views
   // (or one view, of whose rays it takes a share)
-  const int splits = diff_ray_splits(a.view_groups, a.n_views), part = grp % splits;
+  const int splits = SPLIT ? diff_ray_splits(a.view_groups, a.n_views) : 1, part = SPLIT ? grp % splits : 0;
   const int v_begin = (int)((long long)a.n_views * (grp / splits) / (a.view_groups / splits));
   const int v_end = (int)((long long)a.n_views * (grp / splits + 1) / (a.view_groups / splits));
   BrickBox bb;
@@ -826,7 +829,7 @@ __global__ __launch_bounds__(64) void diff_scatter_kernel(DiffArgs a) {
       scatter_list(a, v, L, n, total, scale, s_acc, lane, bb);
     }
     wave_sync();
-    if (splits > 1) {   // the one view's share stays an integer: the combine adds the shares
+    if constexpr (SPLIT) {   // the workgroup's only view
       if (part == 0 && lane == 0) a.block_exp[(size_t)view * nbx * nby * nbz + bi] = e;
       break;
     }
@@ -844,7 +847,7 @@ __global__ __launch_bounds__(64) void diff_scatter_kernel(DiffArgs a) {
     }
     wave_sync();
   }
-  if (splits > 1) {
+  if constexpr (SPLIT) {
     unsigned long long *sums = reinterpret_cast<unsigned long long *>(a.blocks) + blk;
     for (int i = lane; i < kBlk3; i += 64) sums[i] = s_acc[i];
     return;
@@ -875,6 +878,7 @@ __device__ __forceinline__ int axis_sources(int v, int n, int *db, int *slot) {
 // (axis_sources on each axis), summed in a fixed order.  Workgroup 0 also
 // writes grad_tf from the int64 sums: one rounding (int64 -> float) and an
 // exact power-of-two scale.
+template <bool SPLIT>
 __global__ __launch_bounds__(256) void diff_combine_kernel(DiffArgs a) {
   if (blockIdx.x == 0) {
     const int e = tf_exponent(a, threadIdx.x & 63);
@@ -887,7 +891,7 @@ __global__ __launch_bounds__(256) void diff_combine_kernel(DiffArgs a) {
   const size_t nvox = (size_t)a.nx * a.ny * a.nz;
   const int nbx = (a.nx + kBrick - 1) / kBrick, nby = (a.ny + kBrick - 1) / kBrick;
   const size_t nb = (size_t)nbx * nby * ((a.nz + kBrick - 1) / kBrick);
-  const int splits = diff_ray_splits(a.view_groups, a.n_views);
+  const int splits = SPLIT ? diff_ray_splits(a.view_groups, a.n_views) : 1;
   for (size_t vi = (size_t)blockIdx.x * 256 + threadIdx.x; vi < nvox; vi += (size_t)gridDim.x * 256) {
     const int X = (int)(vi % a.nx), Y = (int)((vi / a.nx) % a.ny), Z = (int)(vi / ((size_t)a.nx * a.ny));
     const int bx = X / kBrick, by = Y / kBrick, bz = Z / kBrick;
@@ -901,15 +905,22 @@ __global__ __launch_bounds__(256) void diff_combine_kernel(DiffArgs a) {
           for (int i = 0; i < cx; ++i) {
             const size_t bi = ((size_t)(bz + dbz[k]) * nby + (by + dby[j])) * nbx + (bx + dbx[i]);
             const int slot = (sz[k] * kBlk + sy[j]) * kBlk + sx[i];
-            if (splits == 1) {
+            if constexpr (!SPLIT) {
               g += a.blocks[(grp * nb + bi) * kBlk3 + slot];
               continue;
             }
-            // the shares of one view: integers of one scale, rounded once
+            // the shares of one view: integers of one scale, rounded once (every
+            // load in flight together: one after another they took the shares' gain
+            // back where a view's rays are split most)
+            const long long *sh = reinterpret_cast<const long long *>(a.blocks) + (grp * nb + bi) * kBlk3 + slot;
+            const int e = a.block_exp[(grp / splits) * nb + bi];
+            long long part[kDiffRaySplits];
+#pragma unroll
+            for (int q = 0; q < (int)kDiffRaySplits; ++q) part[q] = q < splits ? sh[q * nb * kBlk3] : 0;
             long long sum = 0;
-            for (int q = 0; q < splits; ++q)
-              sum += reinterpret_cast<const long long *>(a.blocks)[((grp + q) * nb + bi) * kBlk3 + slot];
-            if (sum != 0) g += (float)sum * ldexpf(1.f, -a.block_exp[(grp / splits) * nb + bi]);
+#pragma unroll
+            for (int q = 0; q < (int)kDiffRaySplits; ++q) sum += part[q];
+            if (sum != 0) g += (float)sum * ldexpf(1.f, -e);
           }
     }
     a.grad_vol[vi] = g;
@@ -946,11 +957,14 @@ hipError_t launch_diff_backward(const DiffArgs &a, hipStream_t s) {
   hipLaunchKernelGGL(diff_adjoint_kernel, dim3(a.n_workers), dim3(256), 0, s, a);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   const int nb = ((a.nx + kBrick - 1) / kBrick) * ((a.ny + kBrick - 1) / kBrick) * ((a.nz + kBrick - 1) / kBrick);
-  hipLaunchKernelGGL(diff_scatter_kernel, dim3(nb * a.view_groups), dim3(64), 0, s, a);
+  const bool split = diff_ray_splits(a.view_groups, a.n_views) > 1;
+  if (split) hipLaunchKernelGGL(diff_scatter_kernel<true>, dim3(nb * a.view_groups), dim3(64), 0, s, a);
+  else hipLaunchKernelGGL(diff_scatter_kernel<false>, dim3(nb * a.view_groups), dim3(64), 0, s, a);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   const size_t nvox = (size_t)a.nx * a.ny * a.nz;
   const int cg = (int)std::min<size_t>((nvox + 255) / 256, 4096);
-  hipLaunchKernelGGL(diff_combine_kernel, dim3(cg), dim3(256), 0, s, a);
+  if (split) hipLaunchKernelGGL(diff_combine_kernel<true>, dim3(cg), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL(diff_combine_kernel<false>, dim3(cg), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
