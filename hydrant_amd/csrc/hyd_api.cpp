@@ -101,8 +101,8 @@ int32_t inner_mapping(float k_min, float lo, float hi, int32_t pad) {
   const bool all = k_min >= 0.f && float(pad) * lo - 0.5f >= 1e-3f && float(pad) * hi - 0.5f <= float(pad) - 1.001f;
   return all ? kInnerAlways : kInnerTest;
 }
-int32_t pages_inner(const Ctx *c) {
-  if (capturing(c)) return kInnerTest;
+int32_t pages_inner(const Ctx *c, bool captured) {
+  if (captured) return kInnerTest;
   return inner_mapping(c->page_k_min, c->page_lo, c->page_hi, c->pool.pad);
 }
 
@@ -116,7 +116,7 @@ int32_t check_volume_state(const Ctx *c) {
   return HYD_OK;
 }
 
-int32_t fill_volume_args(const Ctx *c, const hyd_volume_params *p, VolumeArgs &a) {
+int32_t fill_volume_args(const Ctx *c, const hyd_volume_params *p, bool captured, VolumeArgs &a) {
   HYD_REQUIRE(p, HYD_ERR_ARG, "null params");
   HYD_REQUIRE(p->step > 0.f, HYD_ERR_ARG, "step must be > 0");
   HYD_REQUIRE(p->schedule == HYD_SCHED_REFERENCE || p->schedule == HYD_SCHED_LATTICE, HYD_ERR_ARG,
@@ -146,9 +146,8 @@ int32_t fill_volume_args(const Ctx *c, const hyd_volume_params *p, VolumeArgs &a
   a.pad = c->pool.pad;
   // the inner marches' table lookup reads the next entry at weight 0, which
   // must be finite
-  a.inner = c->tf_finite ? pages_inner(c) : (int32_t)kInnerNever;
+  a.inner = c->tf_finite ? pages_inner(c, captured) : (int32_t)kInnerNever;
   a.monotone = c->tf_finite && c->tf_alpha_min >= 0.f && p->density >= 0.f && c->tf_alpha_max * p->density <= 1.f;
-  macro_fill(c, a);
   return HYD_OK;
 }
 
@@ -386,11 +385,12 @@ int32_t hyd_write_pool_pages(hyd_ctx *c, int32_t first_page, int32_t n_pages, co
   const size_t page = (size_t)c->pool.pad * c->pool.pad * c->pool.pad * fmt_bytes(c->pool.fmt);
   char *dst = static_cast<char *>(const_cast<void *>(c->pool.data)) + (size_t)first_page * page;
   HYD_CHECK_HIP(hipMemcpyAsync(dst, host, (size_t)n_pages * page, hipMemcpyHostToDevice, c->stream));
-  HYD_CHECK_HIP(hipStreamSynchronize(c->stream));
   // the batched renderer's oriented copies of these pages follow (in place, so
   // captured graphs stay valid), and so do their macrocells
   if ((st = macro_pages_written(c, first_page, n_pages))) return st;
-  return refresh_oriented_pages(c, first_page, n_pages);
+  if ((st = refresh_oriented_pages(c, first_page, n_pages))) return st;
+  HYD_CHECK_HIP(hipStreamSynchronize(c->stream));
+  return HYD_OK;
 }
 
 int32_t hyd_set_page_table(hyd_ctx *c, const int32_t dims[3], const int32_t *vaddr, int32_t n_pages,
@@ -469,7 +469,8 @@ int32_t hyd_set_tf(hyd_ctx *c, int32_t n, const float *rgba) {
     }
   }
   ++c->batch_state_gen;
-  return macro_tf_set(c);
+  c->mcls_valid = false;
+  return HYD_OK;
 }
 
 int32_t hyd_render_volume(hyd_ctx *c, const hyd_volume_params *p, const hyd_view *view, int32_t width,
@@ -480,7 +481,8 @@ int32_t hyd_render_volume(hyd_ctx *c, const hyd_volume_params *p, const hyd_view
   if ((st = check_volume_state(c))) return st;
   HYD_REQUIRE(view && width > 0 && height > 0, HYD_ERR_ARG, "invalid view or image size");
   VolumeArgs a;
-  if ((st = fill_volume_args(c, p, a))) return st;
+  const bool captured = capturing(c);
+  if ((st = fill_volume_args(c, p, captured, a))) return st;
   fill_view(view, a.trans, a.ctg, a.ray_o);
   a.W = width;
   a.H = height;
@@ -488,6 +490,7 @@ int32_t hyd_render_volume(hyd_ctx *c, const hyd_volume_params *p, const hyd_view
   a.rgba = reinterpret_cast<float4 *>(rgba_dev);
   a.samples = samples_dev;
   a.full_rays = full_rays(a.trans, a.ctg, a.ray_o, a.W, a.H, a.bmin, a.bmax);
+  if (!captured && (st = macro_fill(c, a))) return st;
   HYD_CHECK_HIP(launch_volume(a, c->pool.fmt, false, c->stream));
   return HYD_OK;
 }
@@ -499,13 +502,15 @@ int32_t hyd_resume_volume(hyd_ctx *c, const hyd_volume_params *p, int32_t width,
   if ((st = check_volume_state(c))) return st;
   HYD_REQUIRE(film_dev && width > 0 && height > 0, HYD_ERR_ARG, "resume needs a film");
   VolumeArgs a;
-  if ((st = fill_volume_args(c, p, a))) return st;
+  const bool captured = capturing(c);
+  if ((st = fill_volume_args(c, p, captured, a))) return st;
   a.W = width;
   a.H = height;
   a.film = film_dev;
   a.rgba = reinterpret_cast<float4 *>(rgba_dev);
   a.samples = samples_dev;
   a.full_rays = 0.42f * float(width) * float(height);   // of a square view of a cube: the film holds no view
+  if (!captured && (st = macro_fill(c, a))) return st;
   HYD_CHECK_HIP(launch_volume(a, c->pool.fmt, true, c->stream));
   return HYD_OK;
 }
@@ -636,13 +641,12 @@ int32_t hyd_segments_pass(hyd_ctx *c, const hyd_volume_params *p, const hyd_view
   const int32_t need = c->paging.vdim[0] + c->paging.vdim[1] + c->paging.vdim[2];
   HYD_REQUIRE(max_slots >= need, HYD_ERR_RANGE, "max_slots %d < %d (sum of the brick grid dims)", max_slots, need);
   VolumeArgs a;
-  if ((st = fill_volume_args(c, p, a))) return st;
+  if ((st = fill_volume_args(c, p, capturing(c), a))) return st;
   HYD_REQUIRE(a.schedule == HYD_SCHED_LATTICE, HYD_ERR_ARG, "segments need the lattice schedule");
   fill_view(view, a.trans, a.ctg, a.ray_o);
   a.W = width;
   a.H = height;
   a.full_rays = full_rays(a.trans, a.ctg, a.ray_o, a.W, a.H, a.bmin, a.bmax);
-  a.macro.cls = nullptr;
   a.slots = reinterpret_cast<float4 *>(slots_dev);
   a.nslots = nslots_dev;
   a.max_slots = max_slots;
@@ -800,7 +804,7 @@ int32_t hyd_segments_pass_set(hyd_ctx *c, const hyd_segment_set *set, const hyd_
   const int32_t need = set->vdim[0] + set->vdim[1] + set->vdim[2];
   HYD_REQUIRE(max_slots >= need, HYD_ERR_RANGE, "max_slots %d < %d (sum of the brick grid dims)", max_slots, need);
   VolumeArgs a;
-  if ((st = fill_volume_args(c, p, a))) return st;
+  if ((st = fill_volume_args(c, p, capturing(c), a))) return st;
   HYD_REQUIRE(a.schedule == HYD_SCHED_LATTICE, HYD_ERR_ARG, "segments need the lattice schedule");
   std::memcpy(a.vdim, set->vdim, sizeof(a.vdim));
   a.pad = set->pad;
@@ -809,7 +813,6 @@ int32_t hyd_segments_pass_set(hyd_ctx *c, const hyd_segment_set *set, const hyd_
   a.W = width;
   a.H = height;
   a.full_rays = full_rays(a.trans, a.ctg, a.ray_o, a.W, a.H, a.bmin, a.bmax);
-  a.macro.cls = nullptr;
   a.slots = reinterpret_cast<float4 *>(slots_dev);
   a.nslots = nslots_dev;
   a.max_slots = max_slots;
@@ -854,7 +857,7 @@ int32_t hyd_trace_volume(hyd_ctx *c, const hyd_volume_params *p, const hyd_view 
   HYD_REQUIRE(view && out && n_out && max_recs > 0, HYD_ERR_ARG, "invalid trace arguments");
   HYD_REQUIRE(x >= 0 && x < width && y >= 0 && y < height, HYD_ERR_ARG, "pixel outside the image");
   VolumeArgs a;
-  if ((st = fill_volume_args(c, p, a))) return st;
+  if ((st = fill_volume_args(c, p, capturing(c), a))) return st;
   HYD_REQUIRE(a.schedule == HYD_SCHED_REFERENCE, HYD_ERR_ARG, "trace supports the reference schedule only");
   fill_view(view, a.trans, a.ctg, a.ray_o);
   a.W = width;
@@ -956,8 +959,9 @@ int32_t hyd_render_iso(hyd_ctx *c, const hyd_iso_params *p, const hyd_view *view
   a.pool = c->pool.data;
   a.pool_elems = (uint64_t)c->pool.n_pages * c->pool.pad * c->pool.pad * c->pool.pad;
   a.pad = c->pool.pad;
-  a.inner = pages_inner(c);
-  macro_fill_iso(c, a);
+  const bool captured = capturing(c);
+  a.inner = pages_inner(c, captured);
+  if (!captured && (st = macro_fill_iso(c, a))) return st;
   a.out = out_dev;
   a.samples = samples_dev;
   HYD_CHECK_HIP(launch_iso(a, c->pool.fmt, c->stream));

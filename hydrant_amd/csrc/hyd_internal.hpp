@@ -111,21 +111,28 @@ struct Ctx {
   int32_t n_cus = 0;
   // macrocells of the pool (hyd_macro.hpp): value ranges, and their classes under
   // the transfer function for the frame marches (owned pools only: a bound
-  // pool's contents may change without notice)
+  // pool's contents may change without notice).  The classes are made by the first
+  // frame that can use them, and pages written since (dirty) join them at the
+  // next frame or isosurface.
   float2 *own_mm = nullptr;
-  uint8_t *own_mflags = nullptr, *own_mcls = nullptr;
-  unsigned long long *own_mcount = nullptr;   // macrocells that may contribute (one word)
+  uint8_t *own_mcls = nullptr;
+  // {macrocells of class 0, of class >= 3} (launch_macro_classes): of the frame classes, in
+  // one of two slots (the other is zero, for the next), then of the batch's
+  unsigned long long *own_mcount = nullptr;
+  int32_t mcount_slot = 0;
+  hipEvent_t macro_ev = nullptr;  // behind the last update of the ranges and frame classes
+  bool macro_pending = false;     // ... which may still run
   size_t macro_cap = 0;           // macrocells the arrays hold
   uint64_t mm_gen = ~0ull;        // pool_gen the ranges were made from
+  std::vector<std::pair<int32_t, int32_t>> mm_dirty;   // runs {first, number} of pages whose ranges are behind
   bool mcls_valid = false;        // own_mcls belongs to own_mm and the current transfer function
-  double macro_empty = 0.0;       // share of the pool's macrocells that are empty
   // classes for the batched renderer: each page under the value scale of its
   // volume (NaN: none, or two that differ), made at the first batched launch
   // after a change of pool, transfer function or volume set
   std::vector<std::pair<int32_t, float>> vol_pages;   // {page, value scale} of every resident cell
   std::vector<std::array<float, 3>> vol_bmax;   // extent of each volume of the set
   float *own_bscale = nullptr;
-  uint8_t *own_bflags = nullptr, *own_bcls = nullptr;
+  uint8_t *own_bcls = nullptr;
   size_t bcls_cap = 0, bscale_cap = 0;
   uint64_t bcls_gen = ~0ull;      // batch_state_gen of own_bcls
   double bcls_empty = 0.0;
@@ -160,6 +167,10 @@ struct MacroGrid {
   int32_t nm, cells;    // macrocells per page edge and per page
   float K, B;           // voxels per brick unit, tap coordinate of x = 0
   float run_max;        // longest run to skip at once
+  // the classes are looked up while *flagged, the macrocells that may contribute,
+  // stays at or below this
+  const unsigned long long *flagged;
+  unsigned long long flagged_max;
 };
 
 // Samplers of a march (hyd_sampler.hpp): the clamping one for every sample;
@@ -316,20 +327,20 @@ bool capturing(const Ctx *c);
 // After pool pages [first, first + n) were overwritten in place: updates the
 // batched renderer's oriented copies of those pages if they are current.
 int32_t refresh_oriented_pages(Ctx *c, int32_t first, int32_t n);
-// Macrocells of an owned pool (hyd_macro.cpp), each complete on return: the
-// whole pool's ranges and classes after an upload, those of pages [first, first
-// + n) after a write, the classes after a new transfer function.
+// Macrocells of a pool (hyd_macro.cpp).  After an upload: its ranges (on the
+// stream; the caller waits).  After a write of pages [first, first + n): noted for
+// the next march, or, where the batched renderer's classes are current, brought
+// up to date in place (on the stream; the caller waits).
 int32_t macro_pool_uploaded(Ctx *c);
 int32_t macro_pages_written(Ctx *c, int32_t first, int32_t n);
-int32_t macro_tf_set(Ctx *c);
 void macro_free(Ctx *c);
-// Points the march at the classes when they apply to it, else leaves it without.
-void macro_fill(const Ctx *c, VolumeArgs &a);
+// Points the march at the classes when they apply to it, else leaves it without;
+// brings them up to date first, ahead of the march on its stream (not under capture).
+int32_t macro_fill(Ctx *c, VolumeArgs &a);
 // The batched renderer's classes of the current pool, brought up to date
 // (complete on return); null in *cls when the march should sample throughout.
 int32_t macro_batch(Ctx *c, const uint8_t **cls);
-struct IsoArgs;
-void macro_fill_iso(const Ctx *c, IsoArgs &a);
+int32_t macro_fill_iso(Ctx *c, IsoArgs &a);
 
 }  // namespace hyd
 

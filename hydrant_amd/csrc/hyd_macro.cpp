@@ -13,95 +13,172 @@ namespace {
 // us a paged frame without and with them), and 44% empty saves 27% of it.
 constexpr double kMacroWorth = 0.1;
 
+// Macrocells (of 512 voxels) from which an upload takes the ranges behind its copy, where
+// they are lost in it (40 of 2400 us for one 256^3 FP32 page); a kernel behind the copy of
+// a 32^3 u8 page made its upload 45 us of 28.
+constexpr size_t kRangesWithUpload = 8192;
+
 size_t page_cells(const Ctx *c) {
   const size_t nm = (size_t)macro_edge(c->pool.pad);
   return nm * nm * nm;
 }
 
+constexpr size_t kCounts = 6;   // two slots of the frame classes, and the batch's
+constexpr int kBatchCounts = 4;
+
 bool reserve(Ctx *c, size_t cells) {
   if (c->macro_cap >= cells) return true;
   macro_free(c);
+  const size_t counts = kCounts * sizeof(*c->own_mcount);
   if (hipMalloc((void **)&c->own_mm, cells * sizeof(float2)) != hipSuccess ||
-      hipMalloc((void **)&c->own_mflags, cells) != hipSuccess ||
       hipMalloc((void **)&c->own_mcls, cells) != hipSuccess ||
-      hipMalloc((void **)&c->own_mcount, sizeof(*c->own_mcount)) != hipSuccess) {
+      hipMalloc((void **)&c->own_mcount, counts) != hipSuccess ||
+      hipMemsetAsync(c->own_mcount, 0, counts, c->stream) != hipSuccess ||
+      hipEventCreateWithFlags(&c->macro_ev, hipEventDisableTiming) != hipSuccess) {
     (void)hipGetLastError();   // no memory for them: the marches sample everything
     macro_free(c);
     return false;
   }
+  c->mcount_slot = 0;
   c->macro_cap = cells;
   return true;
 }
 
-int32_t batch_classes(Ctx *c, int32_t first, int32_t n) {
-  HYD_CHECK_HIP(launch_macro_classes(c->own_mm, c->pool.pad, first, n, c->tf, c->tf_n, 1.f, c->own_bscale,
-                                     c->own_bflags, c->own_bcls, c->own_mcount, c->stream));
+MacroRuns run_of(int32_t first, int32_t n) {
+  MacroRuns r{};
+  r.n = 1;
+  r.total = n;
+  r.first[0] = first;
+  return r;
+}
+
+int32_t ranges(Ctx *c, const MacroRuns &r) {
+  HYD_CHECK_HIP(launch_macro_minmax(c->pool.fmt, c->pool.data, c->pool.pad, r, c->own_mm, c->stream));
   return HYD_OK;
 }
 
-int32_t classes(Ctx *c, int32_t first, int32_t n) {
+int32_t classes(Ctx *c, const MacroRuns &r, bool replace) {
   const float scale = c->pool.fmt == HYD_FMT_U8 ? 1.f / 255.f : 1.f;
-  HYD_CHECK_HIP(launch_macro_classes(c->own_mm, c->pool.pad, first, n, c->tf, c->tf_n, scale, nullptr,
-                                     c->own_mflags, c->own_mcls, c->own_mcount, c->stream));
+  if (!replace) c->mcount_slot ^= 1;   // zero: the last full pass or reserve() made it so
+  HYD_CHECK_HIP(launch_macro_classes(c->own_mm, c->pool.pad, r, c->tf, c->tf_n, scale, nullptr, c->own_mcls, replace,
+                                     c->own_mcount + 2 * c->mcount_slot,
+                                     replace ? nullptr : c->own_mcount + 2 * (c->mcount_slot ^ 1), c->stream));
+  return HYD_OK;
+}
+
+// Complete on return, with the share of the batch's classes.
+int32_t batch_classes(Ctx *c, const MacroRuns &r, bool replace) {
+  unsigned long long *counts = c->own_mcount + kBatchCounts, n = 0;
+  if (!replace) HYD_CHECK_HIP(hipMemcpyAsync(counts, &n, sizeof(n), hipMemcpyHostToDevice, c->stream));
+  HYD_CHECK_HIP(launch_macro_classes(c->own_mm, c->pool.pad, r, c->tf, c->tf_n, 1.f, c->own_bscale, c->own_bcls,
+                                     replace, counts, nullptr, c->stream));
+  HYD_CHECK_HIP(hipMemcpyAsync(&n, counts, sizeof(n), hipMemcpyDeviceToHost, c->stream));
+  HYD_CHECK_HIP(hipStreamSynchronize(c->stream));
+  c->bcls_empty = 1.0 - (double)n / ((double)c->pool.n_pages * (double)page_cells(c));
+  return HYD_OK;
+}
+
+// Puts the context's stream behind the last update of the ranges and frame classes,
+// which may have been queued on another.
+int32_t await(Ctx *c) {
+  if (!c->macro_pending) return HYD_OK;
+  const hipError_t e = hipEventQuery(c->macro_ev);
+  if (e == hipErrorNotReady) {
+    (void)hipGetLastError();
+    HYD_CHECK_HIP(hipStreamWaitEvent(c->stream, c->macro_ev, 0));
+    return HYD_OK;
+  }
+  HYD_CHECK_HIP(e);
+  c->macro_pending = false;
+  return HYD_OK;
+}
+
+// Brings the ranges, and with_classes the frame classes, up to date on the
+// context's stream.
+int32_t refresh(Ctx *c, bool with_classes) {
+  int32_t st = await(c);
+  if (st) return st;
+  std::vector<std::pair<int32_t, int32_t>> &d = c->mm_dirty;
+  const bool dirty = !d.empty(), make = with_classes && !c->mcls_valid;
+  if (!dirty && !make) return HYD_OK;
+  const bool update = dirty && c->mcls_valid;
+  c->mcls_valid = false;   // until all of it is queued
+  if (dirty) {
+    std::sort(d.begin(), d.end());
+    MacroRuns r{};
+    for (const auto &[first, n] : d) {   // each page once: the counts follow its old and new classes
+      const int32_t end = first + n, last = r.n > 0 ? r.first[r.n - 1] + (r.total - r.start[r.n - 1]) : -1;
+      if (end <= last) continue;
+      const int32_t from = std::max(first, last);
+      r.first[r.n] = from;
+      r.start[r.n++] = r.total;
+      r.total += end - from;
+    }
+    if ((st = ranges(c, r)) || (update && (st = classes(c, r, true)))) return st;
+  }
+  if (make && (st = classes(c, run_of(0, c->pool.n_pages), false))) return st;
+  HYD_CHECK_HIP(hipEventRecord(c->macro_ev, c->stream));
+  c->macro_pending = true;
+  d.clear();
+  c->mcls_valid = update || make;
   return HYD_OK;
 }
 
 }  // namespace
 
 void macro_free(Ctx *c) {
-  for (void *p : {(void *)c->own_mm, (void *)c->own_mflags, (void *)c->own_mcls, (void *)c->own_mcount})
+  for (void *p : {(void *)c->own_mm, (void *)c->own_mcls, (void *)c->own_mcount, (void *)c->own_bscale,
+                  (void *)c->own_bcls})
     if (p) (void)hipFree(p);
+  if (c->macro_ev) (void)hipEventDestroy(c->macro_ev);
+  c->macro_ev = nullptr;
+  c->macro_pending = false;
   c->own_mm = nullptr;
-  c->own_mflags = c->own_mcls = nullptr;
+  c->own_mcls = nullptr;
   c->own_mcount = nullptr;
-  for (void *p : {(void *)c->own_bscale, (void *)c->own_bflags, (void *)c->own_bcls})
-    if (p) (void)hipFree(p);
   c->own_bscale = nullptr;
-  c->own_bflags = c->own_bcls = nullptr;
+  c->own_bcls = nullptr;
   c->bcls_cap = c->bscale_cap = 0;
   c->bcls_gen = ~0ull;
   c->macro_cap = 0;
   c->mm_gen = ~0ull;
+  c->mm_dirty.clear();
   c->mcls_valid = false;
 }
 
 int32_t macro_pool_uploaded(Ctx *c) {
   c->mcls_valid = false;
   c->mm_gen = ~0ull;
+  c->mm_dirty.clear();
   if (!reserve(c, (size_t)c->pool.n_pages * page_cells(c))) return HYD_OK;
-  HYD_CHECK_HIP(launch_macro_minmax(c->pool.fmt, c->pool.data, c->pool.pad, 0, c->pool.n_pages, c->own_mm,
-                                    c->stream));
   c->mm_gen = c->pool_gen;
-  return c->tf ? macro_tf_set(c) : HYD_OK;   // the caller waits for the stream
-}
-
-int32_t macro_tf_set(Ctx *c) {
-  c->mcls_valid = false;
-  if (c->mm_gen != c->pool_gen) return HYD_OK;
-  unsigned long long n = 0;
-  HYD_CHECK_HIP(hipMemcpyAsync(c->own_mcount, &n, sizeof(n), hipMemcpyHostToDevice, c->stream));
-  int32_t st = classes(c, 0, c->pool.n_pages);
-  if (st) return st;
-  HYD_CHECK_HIP(hipMemcpyAsync(&n, c->own_mcount, sizeof(n), hipMemcpyDeviceToHost, c->stream));
-  HYD_CHECK_HIP(hipStreamSynchronize(c->stream));   // complete before a march on another stream reads them
-  c->macro_empty = 1.0 - (double)n / ((double)c->pool.n_pages * (double)page_cells(c));
-  c->mcls_valid = true;
-  return HYD_OK;
+  if ((size_t)c->pool.n_pages * page_cells(c) < kRangesWithUpload) {
+    c->mm_dirty.emplace_back(0, c->pool.n_pages);   // taken with the classes
+    return HYD_OK;
+  }
+  int32_t st = ranges(c, run_of(0, c->pool.n_pages));
+  if (st) c->mm_gen = ~0ull;
+  return st;
 }
 
 int32_t macro_pages_written(Ctx *c, int32_t first, int32_t n) {
   if (c->mm_gen != c->pool_gen || n <= 0) return HYD_OK;
-  HYD_CHECK_HIP(launch_macro_minmax(c->pool.fmt, c->pool.data, c->pool.pad, first, n, c->own_mm, c->stream));
-  if (c->mcls_valid) {
-    int32_t st = classes(c, first, n);
-    if (st) return st;
-  }
   if (c->bcls_gen == c->batch_state_gen) {   // in place: captured graphs read them
-    int32_t st = batch_classes(c, first, n);
-    if (st) return st;
+    const MacroRuns r = run_of(first, n);
+    int32_t st = await(c);
+    if (st || (st = ranges(c, r)) || (st = batch_classes(c, r, true))) return st;
+    if (!c->mcls_valid) return HYD_OK;   // the frame classes will be made from these ranges
   }
-  HYD_CHECK_HIP(hipStreamSynchronize(c->stream));
-  return HYD_OK;
+  std::vector<std::pair<int32_t, int32_t>> &d = c->mm_dirty;
+  for (auto &[f, k] : d) {
+    if (first >= f && first + n <= f + k) return HYD_OK;
+    if (first == f + k) {   // pages in their order extend a run
+      k += n;
+      return HYD_OK;
+    }
+  }
+  d.emplace_back(first, n);
+  return d.size() < (size_t)kMacroRuns ? (int32_t)HYD_OK : refresh(c, false);
 }
 
 // Classes of every page under the scale of the volumes that name it, for the
@@ -116,13 +193,12 @@ int32_t macro_batch(Ctx *c, const uint8_t **cls) {
     c->bcls_gen = ~0ull;
     if (cells > 0xffffffffull || !reserve(c, cells)) return HYD_OK;   // 32-bit class offsets
     if (c->bcls_cap < cells || c->bscale_cap < n) {
-      for (void *p : {(void *)c->own_bscale, (void *)c->own_bflags, (void *)c->own_bcls})
+      for (void *p : {(void *)c->own_bscale, (void *)c->own_bcls})
         if (p) (void)hipFree(p);
       c->own_bscale = nullptr;
-      c->own_bflags = c->own_bcls = nullptr;
+      c->own_bcls = nullptr;
       c->bcls_cap = c->bscale_cap = 0;
       if (hipMalloc((void **)&c->own_bscale, n * sizeof(float)) != hipSuccess ||
-          hipMalloc((void **)&c->own_bflags, cells) != hipSuccess ||
           hipMalloc((void **)&c->own_bcls, cells) != hipSuccess) {
         (void)hipGetLastError();
         return HYD_OK;
@@ -130,22 +206,19 @@ int32_t macro_batch(Ctx *c, const uint8_t **cls) {
       c->bcls_cap = cells;
       c->bscale_cap = n;
     }
+    int32_t st = HYD_OK;
     if (c->mm_gen != c->pool_gen) {   // a bound pool's, with its oriented copies
-      HYD_CHECK_HIP(launch_macro_minmax(c->pool.fmt, c->pool.data, c->pool.pad, 0, (int)n, c->own_mm, c->stream));
+      if ((st = ranges(c, run_of(0, (int32_t)n)))) return st;
       c->mm_gen = c->pool_gen;
+      c->mm_dirty.clear();
       c->mcls_valid = false;
     }
+    if ((st = refresh(c, false))) return st;
     std::vector<float> scale(n, 0.f);   // the set's pages lie in the pool (fill_args)
     for (const auto &[pg, sc] : c->vol_pages) scale[pg] = scale[pg] == 0.f || scale[pg] == sc ? sc : NAN;
     for (float &sc : scale) sc = sc == 0.f ? NAN : sc;
-    unsigned long long count = 0;
     HYD_CHECK_HIP(hipMemcpyAsync(c->own_bscale, scale.data(), n * sizeof(float), hipMemcpyHostToDevice, c->stream));
-    HYD_CHECK_HIP(hipMemcpyAsync(c->own_mcount, &count, sizeof(count), hipMemcpyHostToDevice, c->stream));
-    int32_t st = batch_classes(c, 0, (int32_t)n);
-    if (st) return st;
-    HYD_CHECK_HIP(hipMemcpyAsync(&count, c->own_mcount, sizeof(count), hipMemcpyDeviceToHost, c->stream));
-    HYD_CHECK_HIP(hipStreamSynchronize(c->stream));
-    c->bcls_empty = 1.0 - (double)count / (double)cells;
+    if ((st = batch_classes(c, run_of(0, (int32_t)n), false))) return st;
     c->bcls_gen = c->batch_state_gen;
   }
   if (c->bcls_empty >= kMacroWorth) *cls = c->own_bcls;
@@ -155,7 +228,7 @@ int32_t macro_batch(Ctx *c, const uint8_t **cls) {
 namespace {
 // The grid for marches within [bmin, bmax]; false when it does not apply.
 bool grid_of(const Ctx *c, f3 bmin, f3 bmax, MacroGrid &g) {
-  if (!c->pool.owned || c->mm_gen != c->pool_gen || capturing(c)) return false;
+  if (!c->pool.owned || c->mm_gen != c->pool_gen) return false;
   // every page has the same mapping, one b on each axis, inside the page
   const float k = c->page_k_min, lo = c->page_lo;
   if (!(k > 0.f && c->page_k_max == k && lo >= 0.f && c->page_hi == k + lo && k + lo <= 1.000001f)) return false;
@@ -177,19 +250,27 @@ bool grid_of(const Ctx *c, f3 bmin, f3 bmax, MacroGrid &g) {
 }
 }  // namespace
 
-void macro_fill(const Ctx *c, VolumeArgs &a) {
-  if (!c->mcls_valid || c->macro_empty < kMacroWorth || !grid_of(c, a.bmin, a.bmax, a.macro)) return;
+int32_t macro_fill(Ctx *c, VolumeArgs &a) {
   // opacities in [0, 1] and colours whose length is finite keep the composite
   // finite, so that a zero contribution leaves it as it is
-  if (!a.monotone || !(c->tf_rgb_max <= 1e15f)) return;
-  if (a.mode == HYD_MODE_PARTITION && !(std::fabs(a.rank) <= 1e15f)) return;
+  if (!a.monotone || !(c->tf_rgb_max <= 1e15f)) return HYD_OK;
+  if (a.mode == HYD_MODE_PARTITION && !(std::fabs(a.rank) <= 1e15f)) return HYD_OK;
+  if (!grid_of(c, a.bmin, a.bmax, a.macro)) return HYD_OK;
+  int32_t st = refresh(c, true);
+  if (st) return st;
   a.macro.cls = c->own_mcls;
+  a.macro.flagged = c->own_mcount + 2 * c->mcount_slot;
+  a.macro.flagged_max = (unsigned long long)((1.0 - kMacroWorth) * (double)c->pool.n_pages * (double)page_cells(c));
+  return HYD_OK;
 }
 
-void macro_fill_iso(const Ctx *c, IsoArgs &a) {
-  if (!grid_of(c, a.bmin, a.bmax, a.macro)) return;
+int32_t macro_fill_iso(Ctx *c, IsoArgs &a) {
+  if (!grid_of(c, a.bmin, a.bmax, a.macro)) return HYD_OK;
+  int32_t st = refresh(c, false);
+  if (st) return st;
   a.mm = c->own_mm;
   a.mm_scale = c->pool.fmt == HYD_FMT_U8 ? 1.f / 255.f : 1.f;
+  return HYD_OK;
 }
 
 }  // namespace hyd

@@ -33,6 +33,10 @@ inline int macro_edge(int pad) { return (pad + kMacro - 1) / kMacro; }
 constexpr float kMacroSlack = 1.f / 64.f;
 constexpr float kMacroGuard = 1.f / 1024.f;
 
+// Whether enough macrocells are empty for the lookups to pay: read by the march, since
+// the host would have to wait for the count.
+__device__ __forceinline__ bool macro_pays(const MacroGrid &g) { return g.cls && *g.flagged <= g.flagged_max; }
+
 // Macrocell coordinate (clamped to the page) of a tap coordinate / 8.
 __device__ __forceinline__ float macro_floor(float f8, float hi) {
   return __builtin_amdgcn_fmed3f(floorf(f8), 0.f, hi);
@@ -77,15 +81,22 @@ __device__ __forceinline__ int macro_run(const MacroGrid &g, int c, f3 x, f3 inv
   return (int)fminf(n + 1.f, g.run_max);
 }
 
-// Launches over pages [first, first + n) of a pool.  mm: {min, max} of every
-// macrocell's voxels as stored (u8 as counts), {NaN, NaN} when a voxel is not finite or
-// beyond 1e30.
-hipError_t launch_macro_minmax(int fmt, const void *pool, int pad, int first, int n, float2 *mm, hipStream_t s);
-// flags then classes under a transfer function (value = stored * scale; page_scale,
-// if not null, holds each page's own scale, NaN: never empty); the number of
-// macrocells that may contribute is added to *n_flagged.
-hipError_t launch_macro_classes(const float2 *mm, int pad, int first, int n, const float *tf, int tf_n, float scale,
-                                const float *page_scale, uint8_t *flags, uint8_t *cls, unsigned long long *n_flagged,
-                                hipStream_t s);
+// Runs of pages that a launch works on, one after another.
+constexpr int kMacroRuns = 64;
+struct MacroRuns {
+  int32_t n, total;                             // runs, pages in all
+  int32_t first[kMacroRuns], start[kMacroRuns];   // each run's first page and the pages before it
+};
+
+// mm: {min, max} of every macrocell's voxels as stored (u8 as counts), {NaN, NaN}
+// when a voxel is not finite or beyond 1e30.
+hipError_t launch_macro_minmax(int fmt, const void *pool, int pad, const MacroRuns &runs, float2 *mm, hipStream_t s);
+// Classes under a transfer function (value = stored * scale; page_scale, if not
+// null, holds each page's own scale, NaN: never empty).  counts[0] and counts[1]
+// gain the macrocells of class 0 and of class 3 or more; replace: and lose those of
+// the classes that stood there.  Two counts at zero (if not null) are set to 0.
+hipError_t launch_macro_classes(const float2 *mm, int pad, const MacroRuns &runs, const float *tf, int tf_n, float scale,
+                                const float *page_scale, uint8_t *cls, bool replace, unsigned long long *counts,
+                                unsigned long long *zero, hipStream_t s);
 
 }  // namespace hyd

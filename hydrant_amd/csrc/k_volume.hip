@@ -848,6 +848,7 @@ __global__ __launch_bounds__(64) void volume_kernel(VolumeArgs a) {
   stage_tf(s_tf, a.tf, a.tf_n);
   if (COUNT && threadIdx.x == 0) s_count = 0;
   __syncthreads();
+  if (!macro_pays(a.macro)) a.macro.cls = nullptr;
 
   using OFF = std::conditional_t<BIG, uint64_t, uint32_t>;
   const int ray = (int)threadIdx.x / LANES, h = (int)threadIdx.x % LANES;
@@ -914,6 +915,7 @@ __global__ __launch_bounds__(64) void lattice_kernel(VolumeArgs a) {
   stage_tf(s_tf, a.tf, a.tf_n);
   if (COUNT && threadIdx.x == 0) s_count = 0;
   __syncthreads();
+  if (!macro_pays(a.macro)) a.macro.cls = nullptr;
   const int ray = (int)threadIdx.x / LANES, h = (int)threadIdx.x % LANES;
   const int x = rotated_tile_x() * tile_w<LANES>() + (ray % tile_w<LANES>());
   const int y = blockIdx.y * tile_h<LANES>() + (ray / tile_w<LANES>());
