@@ -490,6 +490,7 @@ int32_t hyd_render_volume(hyd_ctx *c, const hyd_volume_params *p, const hyd_view
   a.rgba = reinterpret_cast<float4 *>(rgba_dev);
   a.samples = samples_dev;
   a.full_rays = full_rays(a.trans, a.ctg, a.ray_o, a.W, a.H, a.bmin, a.bmax);
+  a.lanes = frame_lanes(width, height, a.full_rays, (double)a.pool_elems * fmt_bytes(c->pool.fmt));
   if (!captured && (st = macro_fill(c, a))) return st;
   HYD_CHECK_HIP(launch_volume(a, c->pool.fmt, false, c->stream));
   return HYD_OK;
@@ -510,6 +511,7 @@ int32_t hyd_resume_volume(hyd_ctx *c, const hyd_volume_params *p, int32_t width,
   a.rgba = reinterpret_cast<float4 *>(rgba_dev);
   a.samples = samples_dev;
   a.full_rays = 0.42f * float(width) * float(height);   // of a square view of a cube: the film holds no view
+  a.lanes = frame_lanes(width, height, a.full_rays, (double)a.pool_elems * fmt_bytes(c->pool.fmt));
   if (!captured && (st = macro_fill(c, a))) return st;
   HYD_CHECK_HIP(launch_volume(a, c->pool.fmt, true, c->stream));
   return HYD_OK;

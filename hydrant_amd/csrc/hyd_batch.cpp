@@ -211,8 +211,6 @@ int32_t fill_args(Ctx *c, hyd_batch *b, const hyd_batch_config *cfg, float densi
   int32_t st = ensure_tiles(b, cfg->tile_w, group, c->stream);
   if (st) return st;
   if ((st = ensure_oriented(c))) return st;
-  const uint8_t *cls = nullptr;
-  if ((st = macro_batch(c, &cls))) return st;
   const int slot = plan_slot(cfg->tile_w, group);
   std::memset(&a, 0, sizeof(a));
   a.tiles = b->d_tiles[slot];
@@ -231,12 +229,6 @@ int32_t fill_args(Ctx *c, hyd_batch *b, const hyd_batch_config *cfg, float densi
     a.pools[1] = a.oriented ? c->own_oriented : c->pool.data;
     a.pools[2] = a.oriented ? static_cast<const char *>(c->own_oriented) + layout_bytes(c) : c->pool.data;
   }
-  // opacities in [0, 1], as the classes take them
-  if (cls && density >= 0.f && c->tf_alpha_max * density <= 1.f) {
-    a.cls = cls;
-    a.nm = macro_edge(c->pool.pad);
-    a.cells_per_page = (uint32_t)a.nm * a.nm * a.nm;
-  }
   // Four lanes a ray (8 x 8 tiles, unroll 4) while the views' rays leave a wave
   // a few tiles at most, so that the longest rays' chains bound the launch: ten
   // batches of 4 to 12 views took 0.47 of their time before on average, 0.58
@@ -244,6 +236,14 @@ int32_t fill_args(Ctx *c, hyd_batch *b, const hyd_batch_config *cfg, float densi
   // the one of the frames (lane_rays).
   const bool quads = cfg->tile_w == 8 && group == 1 && cfg->unroll == 4;
   a.lanes = quads && b->full_rays <= lane_rays((double)layout_bytes(c)) ? 4 : 1;
+  const uint8_t *cls = nullptr;
+  if ((st = macro_batch(c, a.lanes, &cls))) return st;
+  // opacities in [0, 1], as the classes take them
+  if (cls && density >= 0.f && c->tf_alpha_max * density <= 1.f) {
+    a.cls = cls;
+    a.nm = macro_edge(c->pool.pad);
+    a.cells_per_page = (uint32_t)a.nm * a.nm * a.nm;
+  }
   a.pad = c->pool.pad;
   a.page_elems = (uint32_t)c->pool.pad * c->pool.pad * c->pool.pad;
   a.tf = c->tf;

@@ -135,7 +135,7 @@ struct Ctx {
   uint8_t *own_bcls = nullptr;
   size_t bcls_cap = 0, bscale_cap = 0;
   uint64_t bcls_gen = ~0ull;      // batch_state_gen of own_bcls
-  double bcls_empty = 0.0;
+  double bcls_empty = 0.0, bcls_deep = 0.0;   // shares of class > 0 and of class >= 3
   // differentiable renderer: device copy of the views
   void *own_diff_views = nullptr;
   int32_t diff_view_cap = 0;
@@ -167,10 +167,10 @@ struct MacroGrid {
   int32_t nm, cells;    // macrocells per page edge and per page
   float K, B;           // voxels per brick unit, tap coordinate of x = 0
   float run_max;        // longest run to skip at once
-  // the classes are looked up while *flagged, the macrocells that may contribute,
-  // stays at or below this
-  const unsigned long long *flagged;
-  unsigned long long flagged_max;
+  // the classes are looked up while *count, of the macrocells that may contribute (one
+  // lane a ray) or of those deep in empty space (several), lies in this range
+  const unsigned long long *count;
+  unsigned long long count_min, count_max;
 };
 
 // Samplers of a march (hyd_sampler.hpp): the clamping one for every sample;
@@ -209,7 +209,8 @@ struct VolumeArgs {
   uint64_t pool_elems;    // voxels in the pool (n_pages * pad^3)
   int32_t pad;
   int32_t inner;          // kInner*: which samples take the sampler without wraps and clamps
-  float full_rays;        // the frame's work in rays of its longest chord (host: lanes per ray)
+  float full_rays;        // the launch's work in rays of its longest chord (host: lanes per ray)
+  int32_t lanes;          // frames: lanes per ray (frame_lanes)
   int32_t monotone;       // opacities in [0, 1]: a ray's alpha never falls
   MacroGrid macro;        // hyd_macro.hpp
   // outputs
@@ -230,6 +231,9 @@ float full_rays(const float *trans, float ctg, f3 ray_o, int W, int H, f3 bmin, 
 // The work (full_rays) up to which a march of a pool of that size runs four
 // lanes per ray (measurements: k_volume.hip).
 inline float lane_rays(double pool_bytes) { return 75e3f + 36e3f * (float)std::log2(1.0 + pool_bytes / 24e6); }
+
+// Lanes per ray of a frame over a pool of that size: 16, 4 or 1 (k_volume.hip).
+int32_t frame_lanes(int W, int H, float full_rays, double pool_bytes);
 
 hipError_t launch_volume(const VolumeArgs &a, int fmt, bool resume, hipStream_t s);
 hipError_t launch_segments_clear(float4 *slots, size_t n, hipStream_t s);
@@ -338,8 +342,9 @@ void macro_free(Ctx *c);
 // brings them up to date first, ahead of the march on its stream (not under capture).
 int32_t macro_fill(Ctx *c, VolumeArgs &a);
 // The batched renderer's classes of the current pool, brought up to date
-// (complete on return); null in *cls when the march should sample throughout.
-int32_t macro_batch(Ctx *c, const uint8_t **cls);
+// (complete on return); null in *cls when the march, of that many lanes a ray,
+// should sample throughout.
+int32_t macro_batch(Ctx *c, int32_t lanes, const uint8_t **cls);
 int32_t macro_fill_iso(Ctx *c, IsoArgs &a);
 
 }  // namespace hyd

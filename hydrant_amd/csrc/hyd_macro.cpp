@@ -8,10 +8,30 @@
 namespace hyd {
 namespace {
 
-// Share of empty macrocells from which a frame looks them up: the lookups cost
-// about 5% of a march (the 1024^3 fBm volume, 16% empty, breaks even: 186 and 187
-// us a paged frame without and with them), and 44% empty saves 27% of it.
-constexpr double kMacroWorth = 0.1;
+// When the lookups pay.  One lane a ray: from a share of empty macrocells (class > 0)
+// of 0.1 on; frames of volumes 11 to 90% empty run 1.01 to 6 times as fast, batches
+// from 12% on.  Several lanes a ray take a whole macrocell in one group, so a
+// skip saves little but deep in empty space, and what tells is the share of macrocells
+// of class 3 or more (none may contribute within two): frames with lookups, 512^2
+// and 150^2 pixels, against without, by that share (of three kinds of data at 11
+// to 90% empty):
+//   256^3 u8    4 lanes  .06 0.91  .10 0.99  .16 1.04  .25 1.08    16 lanes  .12 0.94  .32 0.93  .42 1.01  .51 1.21
+//   256^3 FP32  4 lanes  .06 0.91  .10 0.98  .16 1.05  .25 1.11    16 lanes  .12 1.03  .32 0.97  .42 1.10  .51 1.28
+//   448^3 u8    4 lanes  .02 0.96  .05 1.05  .10 1.09  .26 1.23    16 lanes  .12 0.94  .17 0.99  .25 1.03  .52 1.22
+//   448^3 FP32  4 lanes  .02 0.97  .05 1.05  .10 1.16  .26 1.55    16 lanes  .05 1.01  .17 1.13  .25 1.18  .52 1.37
+// So the lines fall with the pool's size, as samples cost more where the caches do not
+// hold them.  Pages of fewer than 6 macrocells an edge (32^3 bricks) count as deep more
+// than they save, since a page sees only itself: twice the share, and nothing for 16
+// lanes, whose group crosses half of such a page.  Batches, with four lanes (128^3 in
+// 64^3 bricks): 20% empty 0.98, 40% 1.00, 60% 1.13.  At 0.1 of empties for all of
+// them a 160^2 frame of the 256^3 FP32 volume, 30% empty, took 235 us for 191 without.
+constexpr double kWorthEmpty = 0.1, kWorthBatch = 0.12, kWorthBatchDeep = 0.1;
+constexpr int kSmallPage = 6;
+double worth_deep(int32_t lanes, int nm, double pool_bytes) {
+  const double l = std::log2(1.0 + pool_bytes / 24e6);
+  const double share = lanes == 4 ? std::max(0.02, 0.17 - 0.033 * l) : std::max(0.05, 0.39 - 0.055 * l);
+  return nm < kSmallPage ? 2.0 * share : share;
+}
 
 // Macrocells (of 512 voxels) from which an upload takes the ranges behind its copy, where
 // they are lost in it (40 of 2400 us for one 256^3 FP32 page); a kernel behind the copy of
@@ -66,15 +86,17 @@ int32_t classes(Ctx *c, const MacroRuns &r, bool replace) {
   return HYD_OK;
 }
 
-// Complete on return, with the share of the batch's classes.
+// Complete on return, with the shares of the batch's classes.
 int32_t batch_classes(Ctx *c, const MacroRuns &r, bool replace) {
-  unsigned long long *counts = c->own_mcount + kBatchCounts, n = 0;
-  if (!replace) HYD_CHECK_HIP(hipMemcpyAsync(counts, &n, sizeof(n), hipMemcpyHostToDevice, c->stream));
+  unsigned long long *counts = c->own_mcount + kBatchCounts, n[2] = {0, 0};
+  if (!replace) HYD_CHECK_HIP(hipMemcpyAsync(counts, n, sizeof(n), hipMemcpyHostToDevice, c->stream));
   HYD_CHECK_HIP(launch_macro_classes(c->own_mm, c->pool.pad, r, c->tf, c->tf_n, 1.f, c->own_bscale, c->own_bcls,
                                      replace, counts, nullptr, c->stream));
-  HYD_CHECK_HIP(hipMemcpyAsync(&n, counts, sizeof(n), hipMemcpyDeviceToHost, c->stream));
+  HYD_CHECK_HIP(hipMemcpyAsync(n, counts, sizeof(n), hipMemcpyDeviceToHost, c->stream));
   HYD_CHECK_HIP(hipStreamSynchronize(c->stream));
-  c->bcls_empty = 1.0 - (double)n / ((double)c->pool.n_pages * (double)page_cells(c));
+  const double cells = (double)c->pool.n_pages * (double)page_cells(c);
+  c->bcls_empty = 1.0 - (double)n[0] / cells;
+  c->bcls_deep = (double)n[1] / cells;
   return HYD_OK;
 }
 
@@ -183,7 +205,7 @@ int32_t macro_pages_written(Ctx *c, int32_t first, int32_t n) {
 
 // Classes of every page under the scale of the volumes that name it, for the
 // batched march: made once per state of pool, table and volume set.
-int32_t macro_batch(Ctx *c, const uint8_t **cls) {
+int32_t macro_batch(Ctx *c, int32_t lanes, const uint8_t **cls) {
   *cls = nullptr;
   // a zero contribution leaves the composite as it is while colours are finite
   if (!c->tf_finite || !(c->tf_rgb_max <= 1e15f) || !(c->tf_alpha_min >= 0.f)) return HYD_OK;
@@ -221,7 +243,7 @@ int32_t macro_batch(Ctx *c, const uint8_t **cls) {
     if ((st = batch_classes(c, run_of(0, (int32_t)n), false))) return st;
     c->bcls_gen = c->batch_state_gen;
   }
-  if (c->bcls_empty >= kMacroWorth) *cls = c->own_bcls;
+  if (lanes > 1 ? c->bcls_deep >= kWorthBatchDeep : c->bcls_empty >= kWorthBatch) *cls = c->own_bcls;
   return HYD_OK;
 }
 
@@ -255,12 +277,17 @@ int32_t macro_fill(Ctx *c, VolumeArgs &a) {
   // finite, so that a zero contribution leaves it as it is
   if (!a.monotone || !(c->tf_rgb_max <= 1e15f)) return HYD_OK;
   if (a.mode == HYD_MODE_PARTITION && !(std::fabs(a.rank) <= 1e15f)) return HYD_OK;
+  const int nm = macro_edge(c->pool.pad);
+  if (a.lanes == 16 && nm < kSmallPage) return HYD_OK;
   if (!grid_of(c, a.bmin, a.bmax, a.macro)) return HYD_OK;
   int32_t st = refresh(c, true);
   if (st) return st;
+  const double cells = (double)c->pool.n_pages * (double)page_cells(c);
+  const double bytes = (double)a.pool_elems * (c->pool.fmt == HYD_FMT_U8 ? 1 : c->pool.fmt == HYD_FMT_F16 ? 2 : 4);
   a.macro.cls = c->own_mcls;
-  a.macro.flagged = c->own_mcount + 2 * c->mcount_slot;
-  a.macro.flagged_max = (unsigned long long)((1.0 - kMacroWorth) * (double)c->pool.n_pages * (double)page_cells(c));
+  a.macro.count = c->own_mcount + 2 * c->mcount_slot + (a.lanes > 1 ? 1 : 0);
+  a.macro.count_min = a.lanes > 1 ? (unsigned long long)std::ceil(worth_deep(a.lanes, nm, bytes) * cells) : 0;
+  a.macro.count_max = a.lanes > 1 ? ~0ull : (unsigned long long)((1.0 - kWorthEmpty) * cells);
   return HYD_OK;
 }
 

@@ -35,7 +35,11 @@ constexpr float kMacroGuard = 1.f / 1024.f;
 
 // Whether enough macrocells are empty for the lookups to pay: read by the march, since
 // the host would have to wait for the count.
-__device__ __forceinline__ bool macro_pays(const MacroGrid &g) { return g.cls && *g.flagged <= g.flagged_max; }
+__device__ __forceinline__ bool macro_pays(const MacroGrid &g) {
+  if (!g.cls) return false;
+  const unsigned long long n = *g.count;
+  return n >= g.count_min && n <= g.count_max;
+}
 
 // Macrocell coordinate (clamped to the page) of a tap coordinate / 8.
 __device__ __forceinline__ float macro_floor(float f8, float hi) {

@@ -1198,10 +1198,8 @@ void launch_lanes(const VolumeArgs &a, hipStream_t s) {
 
 template <int FMT, int MODE, bool BIG>
 void launch_mode(const VolumeArgs &a, hipStream_t s) {
-  const long long rays = (long long)a.W * a.H;
-  if (rays <= kManyLaneRays) launch_lanes<FMT, MODE, BIG, kManyLanes>(a, s);
-  else if (rows_fit<kLanes>(a.H) && a.full_rays <= lane_rays((double)a.pool_elems * sizeof(typename RawVox<FMT>::T)))
-    launch_lanes<FMT, MODE, BIG, kLanes>(a, s);
+  if (a.lanes == kManyLanes) launch_lanes<FMT, MODE, BIG, kManyLanes>(a, s);
+  else if (a.lanes == kLanes) launch_lanes<FMT, MODE, BIG, kLanes>(a, s);
   else launch_lanes<FMT, MODE, BIG, 1>(a, s);
 }
 
@@ -1259,6 +1257,11 @@ hipError_t launch_fmt(const VolumeArgs &a, bool resume, hipStream_t s) {
 }
 
 }  // namespace
+
+int32_t frame_lanes(int W, int H, float full_rays, double pool_bytes) {
+  if ((long long)W * H <= kManyLaneRays) return kManyLanes;
+  return rows_fit<kLanes>(H) && full_rays <= lane_rays(pool_bytes) ? kLanes : 1;
+}
 
 hipError_t launch_volume(const VolumeArgs &a, int fmt, bool resume, hipStream_t s) {
   switch (fmt) {
