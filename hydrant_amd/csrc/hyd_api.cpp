@@ -677,6 +677,7 @@ struct hyd_segment_set {
   int32_t *all_ids = nullptr;
   const void *base = nullptr;
   uint64_t span = 0;          // bytes from base to the end of the highest pool
+  uint64_t bytes = 0;         // of the pools
   int32_t inner = kInnerTest;   // kInner* that every batch's pages allow
 };
 
@@ -746,8 +747,10 @@ int32_t hyd_segment_set_create(hyd_ctx *c, int32_t n_batches, const hyd_segment_
   const size_t elem = fmt_bytes(set->fmt), page_elems = (size_t)set->pad * set->pad * set->pad;
   uintptr_t lo = UINTPTR_MAX, hi = 0;
   for (int i = 0; i < n_batches; ++i) {
+    const size_t bytes = b[i].n_pages * page_elems * elem;
     lo = std::min(lo, (uintptr_t)b[i].pool_dev);
-    hi = std::max(hi, (uintptr_t)b[i].pool_dev + b[i].n_pages * page_elems * elem);
+    hi = std::max(hi, (uintptr_t)b[i].pool_dev + bytes);
+    set->bytes += bytes;
   }
   set->together = true;
   for (int i = 0; i < n_batches; ++i) {
@@ -825,7 +828,7 @@ int32_t hyd_segments_pass_set(hyd_ctx *c, const hyd_segment_set *set, const hyd_
     a.page = set->all_pages;
     a.page_base = set->all_bases;
     a.page_local = set->all_ids;
-    HYD_CHECK_HIP(launch_segments_set(a, set->span, set->fmt, c->stream));
+    HYD_CHECK_HIP(launch_segments_set(a, set->span, set->bytes, set->fmt, c->stream));
     return HYD_OK;
   }
   const size_t cells = (size_t)set->vdim[0] * set->vdim[1] * set->vdim[2];

@@ -239,9 +239,10 @@ hipError_t launch_volume(const VolumeArgs &a, int fmt, bool resume, hipStream_t 
 hipError_t launch_segments_clear(float4 *slots, size_t n, hipStream_t s);
 hipError_t launch_segments_pass(const VolumeArgs &a, int fmt, hipStream_t s);
 // A segment set's batches in one launch: codes, page descriptors, bases and local
-// ids run over the pages of every batch, pool is the lowest of their pools and
-// span_bytes the distance from it to the end of the highest.
-hipError_t launch_segments_set(const VolumeArgs &a, uint64_t span_bytes, int fmt, hipStream_t s);
+// ids run over the pages of every batch, pool is the lowest of their pools,
+// span_bytes the distance from it to the end of the highest (which the offsets
+// have to reach) and pool_bytes what the pools hold (which the launch reads).
+hipError_t launch_segments_set(const VolumeArgs &a, uint64_t span_bytes, uint64_t pool_bytes, int fmt, hipStream_t s);
 constexpr int kMaxSegBatches = 16;
 hipError_t launch_segments_composite(const float4 *slots, const int32_t *nslots, int max_slots, int P, float4 *rgba,
                                      hipStream_t s);

@@ -1068,8 +1068,11 @@ __device__ __forceinline__ void seg_sample_group(const VolumeArgs &a, const floa
 // walked once for all batches.  (With one layer of workgroups per batch, each
 // walked every ray's cells and found a third of them resident: 4.10 against
 // 2.81 ms for three batches of a 1024^3 u8 volume at 512^2.)
+// The 64-bit offsets of a set whose pools lie far apart are held to three waves per
+// SIMD (one register too many leaves two: 1024^2 FP16 frame of two pools 10 GB apart
+// 3.89 ms, 2.98 with three, and 3.12 with 32-bit offsets).
 template <int FMT, bool COUNT, bool BIG, bool MULTI, int LANES>
-__global__ __launch_bounds__(64) void segment_kernel(VolumeArgs a) {
+__global__ __launch_bounds__(64, BIG && MULTI && LANES == 1 ? 3 : 1) void segment_kernel(VolumeArgs a) {
   using OFF = std::conditional_t<BIG, uint64_t, uint32_t>;
   constexpr int U = LANES > 1 ? coop_group<LANES>() / LANES : HYD_SEG_GROUP;
   __shared__ float4 s_tf[kTfLds];
@@ -1238,8 +1241,8 @@ void launch_segments_lanes(const VolumeArgs &a, bool big, hipStream_t s) {
 // wave (512^2 frame of a 1024^3 u8 set: 4.21 ms with one lane, 2.81 with four;
 // eight drawn sets 1.17 and 2.19 times as fast as one layer of workgroups per batch).
 template <int FMT, bool MULTI>
-hipError_t launch_segments(const VolumeArgs &a, uint64_t bytes, hipStream_t s) {
-  const bool big = bytes > (1ull << 32) || force_offsets64();
+hipError_t launch_segments(const VolumeArgs &a, uint64_t span, uint64_t bytes, hipStream_t s) {
+  const bool big = span > (1ull << 32) || force_offsets64();
   if ((long long)a.W * a.H <= kManyLaneRays) launch_segments_lanes<FMT, MULTI, kManyLanes>(a, big, s);
   else if (rows_fit<kLanes>(a.H) && a.full_rays <= 2.f * lane_rays((double)bytes)) launch_segments_lanes<FMT, MULTI, kLanes>(a, big, s);
   else launch_segments_lanes<FMT, MULTI, 1>(a, big, s);
@@ -1278,17 +1281,17 @@ hipError_t launch_segments_clear(float4 *slots, size_t n, hipStream_t s) {
 
 hipError_t launch_segments_pass(const VolumeArgs &a, int fmt, hipStream_t s) {
   switch (fmt) {
-    case HYD_FMT_U8: return launch_segments<HYD_FMT_U8, false>(a, a.pool_elems, s);
-    case HYD_FMT_F16: return launch_segments<HYD_FMT_F16, false>(a, a.pool_elems * 2, s);
-    default: return launch_segments<HYD_FMT_F32, false>(a, a.pool_elems * 4, s);
+    case HYD_FMT_U8: return launch_segments<HYD_FMT_U8, false>(a, a.pool_elems, a.pool_elems, s);
+    case HYD_FMT_F16: return launch_segments<HYD_FMT_F16, false>(a, a.pool_elems * 2, a.pool_elems * 2, s);
+    default: return launch_segments<HYD_FMT_F32, false>(a, a.pool_elems * 4, a.pool_elems * 4, s);
   }
 }
 
-hipError_t launch_segments_set(const VolumeArgs &a, uint64_t span_bytes, int fmt, hipStream_t s) {
+hipError_t launch_segments_set(const VolumeArgs &a, uint64_t span_bytes, uint64_t pool_bytes, int fmt, hipStream_t s) {
   switch (fmt) {
-    case HYD_FMT_U8: return launch_segments<HYD_FMT_U8, true>(a, span_bytes, s);
-    case HYD_FMT_F16: return launch_segments<HYD_FMT_F16, true>(a, span_bytes, s);
-    default: return launch_segments<HYD_FMT_F32, true>(a, span_bytes, s);
+    case HYD_FMT_U8: return launch_segments<HYD_FMT_U8, true>(a, span_bytes, pool_bytes, s);
+    case HYD_FMT_F16: return launch_segments<HYD_FMT_F16, true>(a, span_bytes, pool_bytes, s);
+    default: return launch_segments<HYD_FMT_F32, true>(a, span_bytes, pool_bytes, s);
   }
 }
 
