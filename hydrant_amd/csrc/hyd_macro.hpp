@@ -41,6 +41,13 @@ __device__ __forceinline__ bool macro_pays(const MacroGrid &g) {
   return n >= g.count_min && n <= g.count_max;
 }
 
+// How far outside a macrocell's range an interpolated value may lie: the rounding of
+// three lerps, 2^-19 of the range's magnitude; below the normal floats it no longer
+// shrinks with it (half the least denormal rounds to zero).
+__device__ __forceinline__ float range_margin(float2 r) {
+  return fmaf(fmaxf(fabsf(r.x), fabsf(r.y)), 1.9073486e-6f, 1e-37f);
+}
+
 // Macrocell coordinate (clamped to the page) of a tap coordinate / 8.
 __device__ __forceinline__ float macro_floor(float f8, float hi) {
   return __builtin_amdgcn_fmed3f(floorf(f8), 0.f, hi);

@@ -164,10 +164,10 @@ __device__ __forceinline__ float iso_srgb(float linear) {
 constexpr int32_t kIsoPending = -1;
 
 // Side of the isovalue that every sample of a macrocell lies on, from its
-// value range widened by 2^-19 of its magnitude (the interpolation's rounding):
-// +1, -1, or 0 when both sides (or a voxel that is not finite) are possible.
+// value range widened by range_margin(): +1, -1, or 0 when both sides (or a voxel
+// that is not finite) are possible.
 __device__ __forceinline__ float range_side(float2 r, float scale, float iso) {
-  const float m = fmaxf(fabsf(r.x), fabsf(r.y)) * 1.9073486e-6f;
+  const float m = range_margin(r);
   return (r.x - m) * scale > iso ? 1.f : (r.y + m) * scale < iso ? -1.f : 0.f;
 }
 
