@@ -209,6 +209,8 @@ int32_t macro_batch(Ctx *c, int32_t lanes, const uint8_t **cls) {
   *cls = nullptr;
   // a zero contribution leaves the composite as it is while colours are finite
   if (!c->tf_finite || !(c->tf_rgb_max <= 1e15f) || !(c->tf_alpha_min >= 0.f)) return HYD_OK;
+  // without oriented copies the march reads a bound pool as it is at the launch
+  if (!c->pool.owned && !c->own_oriented) return HYD_OK;
   const size_t n = (size_t)c->pool.n_pages, cells = n * page_cells(c);
   if (c->bcls_gen != c->batch_state_gen) {
     if (capturing(c)) return HYD_OK;   // made by the next launch outside it
