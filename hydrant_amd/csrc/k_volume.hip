@@ -189,19 +189,9 @@ __device__ __forceinline__ void composite_ub(float4 ub, MarchState &st) {
   st.v.w = st.v.w + ub.w * t;
 }
 
-template <bool WEIGHTED = false, bool THETA = true>
-__device__ __forceinline__ void shade_composite_impl(const VolumeArgs &a, const float4 *tf, float s, int pgid,
-                                                     MarchState &st, float w) {
-  composite_ub<THETA>(shade_sample<WEIGHTED>(a, tf, s, pgid, w), st);
-}
-
 __device__ __forceinline__ void shade_composite(const VolumeArgs &a, const float4 *tf, float s, int pgid,
                                                 MarchState &st) {
-  shade_composite_impl<false>(a, tf, s, pgid, st, 1.f);
-}
-__device__ __forceinline__ void shade_composite(const VolumeArgs &a, const float4 *tf, float s, int pgid,
-                                                MarchState &st, float w) {
-  shade_composite_impl<true>(a, tf, s, pgid, st, w);
+  composite_ub(shade_sample(a, tf, s, pgid, 1.f), st);
 }
 
 // The chebyshev and page-table entries of the brick the last sample fell in:
