@@ -190,9 +190,10 @@ int32_t hyd_mat4_inverse(const float m[16], float out[16]);
 int32_t hyd_upload_pool(hyd_ctx *ctx, int32_t fmt, int32_t pad_edge, int32_t n_pages, const void *host);
 /* Same, but the pool already lives on the device; the context keeps the pointer
  * (not a copy), which must stay valid while the context renders from it.
- * The batched renderer reads the pool through oriented copies that it derives
- * at its first launch after an upload or bind: after changing a bound pool's
- * contents in place, call this again before the next batched launch.  The
+ * The batched renderer reads the pool through oriented copies and the classes
+ * of its empty blocks, which it derives at its first launch after an upload or bind:
+ * after changing a bound pool's contents in place, call this again before the next
+ * batched launch.  (Frames and isosurfaces read a bound pool as it is.)  The
  * copies take 12x the pool's bytes for FP16 and u8 pools (three quad
  * layouts), or 6x (three row-pair layouts) when the device cannot hold those,
  * else 2x (y- and z-fastest layouts); with less free memory the renderer
@@ -201,8 +202,9 @@ int32_t hyd_bind_pool_device(hyd_ctx *ctx, int32_t fmt, int32_t pad_edge, int32_
 /* Overwrite pages [first_page, first_page + n_pages) of the current pool with
  * n_pages host bricks of its format and edge: the reference's block_storage
  * upload when a decoded brick takes a slot (rt_block_paging.cc:277-280).
- * Synchronous.  The batched renderer's oriented copies of those pages are
- * updated in place, so captured batch graphs stay valid. */
+ * Synchronous.  The batched renderer's oriented copies and classes of those pages
+ * are updated in place, so captured batch graphs stay valid; what the frame marches
+ * know of them is brought up to date by the next frame. */
 int32_t hyd_write_pool_pages(hyd_ctx *ctx, int32_t first_page, int32_t n_pages, const void *host);
 /* Page table (BlockPaging, block_paging.hpp:38-44): vaddr grid of dims[0]*dims[1]*dims[2]
  * int32 (x fastest, -1 = not resident) and per-page BlockSamplerMapping {k, b[3]}
@@ -222,7 +224,10 @@ int32_t hyd_set_tf(hyd_ctx *ctx, int32_t n, const float *rgba);
  * cuda_shading.cu:14-37, volume_shader.cu:32-81).  film_dev (hyd_volume_pixel
  * per pixel) and rgba_dev (float4 per pixel) may each be NULL.  samples_dev, if
  * not NULL, is a device uint64 to which the number of composited samples is
- * added (slower counting variant). */
+ * added (slower counting variant).  Over a pool of hyd_upload_pool the first frame
+ * after a new pool, table or pages also classes the pool's empty blocks, on the
+ * context's stream.  Captured in a HIP graph, a frame samples throughout, and replays
+ * follow a page table set or pages written since. */
 int32_t hyd_render_volume(hyd_ctx *ctx, const hyd_volume_params *p, const hyd_view *view, int32_t width,
                           int32_t height, hyd_volume_pixel *film_dev, float *rgba_dev,
                           unsigned long long *samples_dev);
@@ -243,12 +248,13 @@ int32_t hyd_fetch_pass(hyd_ctx *ctx, const hyd_volume_pixel *film_dev, int32_t w
 int32_t hyd_composite(hyd_ctx *ctx, int32_t n, const hyd_fetch_pixel *partials_dev, const int32_t *z_order,
                       int32_t width, int32_t height, float *rgba_dev, uint8_t *rgb_dev);
 /* hyd_composite without any device allocation (no counterpart in the reference):
- * for callers that cannot allocate, such as code under HIP graph capture or a
- * serving loop that composites every frame.  The z order is staged in a fixed
- * device array of the library (one per device, resolved by hyd_create); n is at
- * most 4096 (HYD_ERR_RANGE beyond).  Every call on one device uses that same
- * array, so calls that overlap on a device (other streams, other contexts,
- * other threads) race.  Same results as hyd_composite.  Synchronous. */
+ * for callers that cannot allocate, such as a serving loop that composites every
+ * frame.  Up to 64 images the z order travels with the launch (as in hyd_composite);
+ * beyond, it is staged in a fixed device array of the library (one per device, resolved
+ * by hyd_create), n at most 4096 (HYD_ERR_RANGE beyond).  Calls of more than 64 images
+ * on one device use that same array, so those that overlap on a device (other
+ * streams, other contexts, other threads) race.  Same results as hyd_composite.
+ * Synchronous. */
 int32_t hyd_composite_noalloc(hyd_ctx *ctx, int32_t n, const hyd_fetch_pixel *partials_dev, const int32_t *z_order,
                               int32_t width, int32_t height, float *rgba_dev, uint8_t *rgb_dev);
 /* The bytes hyd_composite writes: t[0] = -inf and, for k = 1..255, t[k] = the
@@ -306,9 +312,9 @@ typedef struct hyd_segment_set hyd_segment_set;
 int32_t hyd_segment_set_create(hyd_ctx *ctx, int32_t n_batches, const hyd_segment_batch *batches,
                                hyd_segment_set **out);
 int32_t hyd_segment_set_destroy(hyd_segment_set *set);
-/* hyd_segments_pass for every batch of the set, in one launch (the batches'
- * bricks are disjoint, so their slots are too): the same slots as one pass per
- * batch with that batch bound. */
+/* hyd_segments_pass for every batch of the set: the same slots as one pass per
+ * batch with that batch bound.  One launch where the batches' bricks are disjoint
+ * (their slots are too); batches that share a brick take one launch each. */
 int32_t hyd_segments_pass_set(hyd_ctx *ctx, const hyd_segment_set *set, const hyd_volume_params *p,
                               const hyd_view *view, int32_t width, int32_t height, int32_t max_slots,
                               float *slots_dev, int32_t *nslots_dev, unsigned long long *samples_dev);
