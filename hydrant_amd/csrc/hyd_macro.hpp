@@ -41,11 +41,12 @@ __device__ __forceinline__ bool macro_pays(const MacroGrid &g) {
   return n >= g.count_min && n <= g.count_max;
 }
 
-// How far outside a macrocell's range an interpolated value may lie: the rounding of
+// How far outside [lo, hi] a value interpolated in it may lie: the rounding of
 // three lerps, 2^-19 of the range's magnitude; below the normal floats it no longer
-// shrinks with it (half the least denormal rounds to zero).
-__device__ __forceinline__ float range_margin(float2 r) {
-  return fmaf(fmaxf(fabsf(r.x), fabsf(r.y)), 1.9073486e-6f, 1e-37f);
+// shrinks with it (half the least denormal rounds to zero).  The ranges are kept widened
+// by it, so that a lookup compares and no more.
+__device__ __forceinline__ float range_margin(float lo, float hi) {
+  return fmaf(fmaxf(fabsf(lo), fabsf(hi)), 1.9073486e-6f, 1e-37f);
 }
 
 // Macrocell coordinate (clamped to the page) of a tap coordinate / 8.
@@ -99,8 +100,8 @@ struct MacroRuns {
   int32_t first[kMacroRuns], start[kMacroRuns];   // each run's first page and the pages before it
 };
 
-// mm: {min, max} of every macrocell's voxels as stored (u8 as counts), {NaN, NaN}
-// when a voxel is not finite or beyond 1e30.
+// mm: {min, max} of every macrocell's voxels as stored (u8 as counts), widened by
+// range_margin(); {NaN, NaN} when a voxel is not finite or beyond 1e30.
 hipError_t launch_macro_minmax(int fmt, const void *pool, int pad, const MacroRuns &runs, float2 *mm, hipStream_t s);
 // Classes under a transfer function (value = stored * scale; page_scale, if not
 // null, holds each page's own scale, NaN: never empty).  counts[0] and counts[1]

@@ -164,11 +164,10 @@ __device__ __forceinline__ float iso_srgb(float linear) {
 constexpr int32_t kIsoPending = -1;
 
 // Side of the isovalue that every sample of a macrocell lies on, from its
-// value range widened by range_margin(): +1, -1, or 0 when both sides (or a voxel
-// that is not finite) are possible.
+// (widened) value range: +1, -1, or 0 when both sides (or a voxel that is not
+// finite) are possible.
 __device__ __forceinline__ float range_side(float2 r, float scale, float iso) {
-  const float m = range_margin(r);
-  return (r.x - m) * scale > iso ? 1.f : (r.y + m) * scale < iso ? -1.f : 0.f;
+  return r.x * scale > iso ? 1.f : r.y * scale < iso ? -1.f : 0.f;
 }
 
 // The march of IsosurfaceShaderKernel::main up to the first crossing, with the

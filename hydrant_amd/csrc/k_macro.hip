@@ -89,15 +89,15 @@ __global__ __launch_bounds__(256) void macro_minmax_kernel(const void *pool, int
       hi = fmaxf(hi, s_col[r * pad + x].y);
     }
     const bool bad = lo == -INFINITY || hi == INFINITY;
-    out[((size_t)mz * nm + my0 + r) * nm + mx] = bad ? make_float2(NAN, NAN) : make_float2(lo, hi);
+    const float m = range_margin(lo, hi);
+    out[((size_t)mz * nm + my0 + r) * nm + mx] = bad ? make_float2(NAN, NAN) : make_float2(lo - m, hi + m);
   }
 }
 
 // Classes of whole pages (up to 16 macrocells an edge, as many pages as give 256
 // rows) or of tiles of 8 macrocells an edge.  A macrocell is flagged when it may
 // contribute: some transfer-function entry that a value of its range can touch
-// has a non-zero alpha; the range is widened by range_margin() and the entry
-// positions by 1e-3.  The flags of a page
+// has a non-zero alpha; the entry positions are widened by 1e-3.  The flags of a page
 // or of a tile with its neighbours up to kMacroCap - 1 away are one word of bits per
 // x row in LDS; widened by one macrocell on every axis, a thread a row, the r-th
 // time they hold what lies within r, so the class is the number of widenings
@@ -162,8 +162,7 @@ __global__ __launch_bounds__(256) void macro_class_kernel(const float2 *mm, int 
       for (int k = 0; k < kAhead; ++k) {
         const float2 r = rg[k];
         const float sc = page_scale ? page_scale[page[k]] : scale;
-        const float mag = range_margin(r);
-        const float lo = (r.x - mag) * sc, hi = (r.y + mag) * sc;
+        const float lo = r.x * sc, hi = r.y * sc;
         bool f = true;
         if (hi < 0.f || lo > 1.f) {
           f = false;   // outside the table: the border's zero
