@@ -20,11 +20,13 @@ namespace {
 //   448^3 u8    4 lanes  .02 0.96  .05 1.05  .10 1.09  .26 1.23    16 lanes  .12 0.94  .17 0.99  .25 1.03  .52 1.22
 //   448^3 FP32  4 lanes  .02 0.97  .05 1.05  .10 1.16  .26 1.55    16 lanes  .05 1.01  .17 1.13  .25 1.18  .52 1.37
 // So the lines fall with the pool's size, as samples cost more where the caches do not
-// hold them.  Pages of fewer than 6 macrocells an edge (32^3 bricks) count as deep more
+// hold them. Pages of fewer than 6 macrocells an edge (32^3 bricks) count as deep more
 // than they save, since a page sees only itself: twice the share, and nothing for 16
-// lanes, whose group crosses half of such a page.  Batches, with four lanes (128^3 in
-// 64^3 bricks): 20% empty 0.98, 40% 1.00, 60% 1.13.  At 0.1 of empties for all of
-// them a 160^2 frame of the 256^3 FP32 volume, 30% empty, took 235 us for 191 without.
+// lanes, whose group crosses half of such a page. Batches: one lane as frames (24
+// views at 256 to 384 pixels: 15% 1.02, 40% 1.21, 60% 1.52; 8 at 128 to 160 break even
+// at a third); four lanes, 0.98 to 1.21 in eight batches with .16 to .26 deep. At 0.1
+// of empties for all of them a 160^2 frame of the 256^3 FP32 volume, 30% empty, took
+// 235 us for 191 without.
 constexpr double kWorthEmpty = 0.1, kWorthBatch = 0.12, kWorthBatchDeep = 0.1;
 constexpr int kSmallPage = 6;
 double worth_deep(int32_t lanes, int nm, double pool_bytes) {
