@@ -12,7 +12,7 @@ namespace {
 // of 0.1 on; frames of volumes 11 to 90% empty run 1.01 to 6 times as fast, batches
 // from 12% on.  Several lanes a ray take a whole macrocell in one group, so a
 // skip saves little but deep in empty space, and what tells is the share of macrocells
-// of class 3 or more (none may contribute within two): frames with lookups, 512^2
+// of class 3 or more (none may contribute within two): frames with lookups, 400^2
 // and 150^2 pixels, against without, by that share (of three kinds of data at 11
 // to 90% empty):
 //   256^3 u8    4 lanes  .06 0.91  .10 0.99  .16 1.04  .25 1.08    16 lanes  .12 0.94  .32 0.93  .42 1.01  .51 1.21
@@ -31,7 +31,7 @@ constexpr double kWorthEmpty = 0.1, kWorthBatch = 0.12, kWorthBatchDeep = 0.1;
 constexpr int kSmallPage = 6;
 double worth_deep(int32_t lanes, int nm, double pool_bytes) {
   const double l = std::log2(1.0 + pool_bytes / 24e6);
-  const double share = lanes == 4 ? std::max(0.02, 0.17 - 0.033 * l) : std::max(0.05, 0.39 - 0.055 * l);
+  const double share = lanes == 4 ? std::max(0.02, 0.17 - 0.033 * l) : std::max(0.05, 0.39 - 0.06 * l);
   return nm < kSmallPage ? 2.0 * share : share;
 }
 
